@@ -364,7 +364,7 @@ ndc_status bake(ndc_handle hh, const ndc_conv_desc* d, const void* k, Baked** ou
     // the kernel on the device, at the view's element offsets
     const size_t kb = size_t(p.k_hi - p.k_lo + 1) * es;
     const void* dk = k;
-    const size_t sb = fft_kernel_spectrum_bytes(p, h.max_lds());
+    const size_t sb = fft_kernel_spectrum_bytes(p, h);
     if (host || sb == 0) {
         if (hipMalloc(&b->kcopy.ptr, kb) != hipSuccess) return set_err(hh, NDC_ERR_OUT_OF_MEMORY, "kernel copy allocation failed");
         b->kcopy.bytes = kb;

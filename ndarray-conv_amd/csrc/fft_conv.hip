@@ -1,4 +1,6 @@
-// FFT convolution on gfx950 (conv_fft/mod.rs:185-292).
+// FFT convolution on gfx950 (conv_fft/mod.rs:185-292): the multi-pass form, for
+// kernels too long for a tile (tile_plan.cpp decides; tile_kernels.hpp has the
+// other form), and the processor's transforms.
 //
 // The padded data and the scattered kernel are never materialised: the first
 // pass reads x through the per-axis border maps (conv_fft/padding.rs:30-62,
@@ -33,6 +35,7 @@
 #include "device_common.hpp"
 #include "fft_bfly.hpp"
 #include "launch.hpp"
+#include "tile_conv.hpp"
 
 namespace ndc {
 namespace {
@@ -2754,7 +2757,41 @@ ndc_status proc_backward(bool real, int N, const int64_t* sshape, int64_t fl, co
 
 }  // namespace
 
+bool pass_form_fits(const Plan& p, size_t lds) {
+    const bool cplx = p.dtype == NDC_C64 || p.dtype == NDC_C128;
+    const bool dbl = p.dtype == NDC_F64 || p.dtype == NDC_C128;
+    const size_t es = dbl ? 16 : 8;
+    auto fits = [&](int64_t L, int post, int bufs) {
+        return L <= (int64_t(1) << 24) && (size_t(ntw_of(int(L), post, dbl)) + size_t(bufs) * pp_len(int(L))) * es <= lds;
+    };
+    const int last = p.N - 1;
+    const int64_t Fl = p.fft[last];
+    const bool half = !cplx && Fl % 2 == 0;
+    bool ok = half ? fits(Fl / 2, int(Fl), 2) : fits(Fl, 0, 2);
+    // longer rows: two factors, the second with a third line buffer; the pair
+    // nearest the root first
+    for (int64_t d = int64_t(std::sqrt(double(Fl))) + 1; !ok && d >= 2; --d)
+        if (Fl % d == 0) ok = (fits(d, 0, 3) && fits(Fl / d, 0, 2)) || (fits(Fl / d, 0, 3) && fits(d, 0, 2));
+    for (int e = 0; ok && e < last; ++e) {
+        const int64_t F = p.fft[e];
+        ok = fits(F, 0, 3);
+        for (int64_t d = int64_t(std::sqrt(double(F))) + 1; !ok && d >= 2; --d)
+            if (F % d == 0) ok = fits(d, 0, 3) && fits(F / d, 0, 3);
+    }
+    return ok;
+}
+
+const TilePlan* tile_of(const Plan& p, LaunchContext& ctx) {
+    if (!p.tile_known) {
+        auto t = std::make_shared<TilePlan>();
+        if (tile_plan(p, ctx.max_lds(), ctx.cu_count(), t.get()) && pass_form_fits(p, ctx.max_lds())) p.tile = t;
+        p.tile_known = true;
+    }
+    return p.tile.get();
+}
+
 ndc_status launch_fft(const Plan& p, const void* x, const void* k, void* y, LaunchContext& ctx, KernelSpectrum* ks) {
+    if (const TilePlan* t = tile_of(p, ctx)) return launch_tile(p, *t, x, k, y, ctx, ks);
     switch (p.dtype) {
         case NDC_F32: return run_fft<float, float>(p, x, k, y, ctx, ks);
         case NDC_F64: return run_fft<double, double>(p, x, k, y, ctx, ks);
@@ -2764,7 +2801,7 @@ ndc_status launch_fft(const Plan& p, const void* x, const void* k, void* y, Laun
     }
 }
 
-size_t fft_kernel_spectrum_bytes(const Plan& p, size_t lds) {
+static size_t pass_kernel_spectrum_bytes(const Plan& p, size_t lds) {
     const bool cplx = p.dtype == NDC_C64 || p.dtype == NDC_C128;
     const size_t es = (p.dtype == NDC_F64 || p.dtype == NDC_C128) ? 16 : 8;
     const int N = p.N, last = N - 1;
@@ -2780,13 +2817,18 @@ size_t fft_kernel_spectrum_bytes(const Plan& p, size_t lds) {
     return size_t(n) * es;
 }
 
+size_t fft_kernel_spectrum_bytes(const Plan& p, LaunchContext& ctx) {
+    if (const TilePlan* t = tile_of(p, ctx)) return t->spec_bytes;
+    return pass_kernel_spectrum_bytes(p, ctx.max_lds());
+}
+
 size_t fft_workspace_bytes(const Plan& p, size_t lds) {
     const size_t es = (p.dtype == NDC_F64 || p.dtype == NDC_C128) ? 16 : 8;
     const int last = p.N - 1;
     const int64_t Fl = p.fft[last];
     // the two spectra: half-spectrum rows padded to 8 bins, or full rows of
     // the four-step form (all Fl bins kept)
-    size_t spec = fft_kernel_spectrum_bytes(p, lds);
+    size_t spec = pass_kernel_spectrum_bytes(p, lds);
     const bool big = spec == 0;
     if (big) {
         int64_t n = Fl;

@@ -120,7 +120,7 @@ ndc_status launch_fft(const Plan& p, const void* x, const void* k, void* y, Laun
 
 // Bytes of a kept kernel spectrum for the plan, or 0 when its rows are too
 // long for one workgroup (those plans recompute the kernel spectrum per call).
-size_t fft_kernel_spectrum_bytes(const Plan& p, size_t lds);
+size_t fft_kernel_spectrum_bytes(const Plan& p, LaunchContext& ctx);
 
 // Upper bound of the device memory launch_fft (without a kept spectrum)
 // requests through LaunchContext::scratch, twiddles and constant_table for

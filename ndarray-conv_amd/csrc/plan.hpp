@@ -5,6 +5,7 @@
 #pragma once
 
 #include <cstdint>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -13,6 +14,8 @@
 namespace ndc {
 
 constexpr int kMaxRank = NDC_MAX_RANK;
+
+struct TilePlan;
 
 // Codes stored in a border map next to non-negative source indices.
 enum BorderCode : int32_t {
@@ -46,6 +49,10 @@ struct Plan {
     // Element offsets (relative to the data pointer) of the lowest and highest
     // element a strided view touches.
     int64_t x_lo = 0, x_hi = 0, k_lo = 0, k_hi = 0;
+    // The tile form of an FFT convolution, decided by the first launch
+    // (tile_of); a plan belongs to one handle, which one thread uses at a time.
+    mutable std::shared_ptr<const TilePlan> tile;
+    mutable bool tile_known = false;
 };
 
 size_t dtype_size(int dtype);

@@ -1,0 +1,309 @@
+// Which convolutions run as overlap-save tiles (tile_kernels.hpp), on which
+// tile, and the host side of their launches.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cmath>
+#include <cstring>
+#include <string>
+#include <vector>
+
+#include "border1d.hpp"
+#include "tile_conv.hpp"
+#include "tile_fft.hpp"
+
+namespace ndc {
+
+namespace {
+
+using tilefft::Shape;
+
+template <int LH, int LW, int LP>
+std::vector<double> twiddles_of() {
+    using S = Shape<LH, LW, LP>;
+    static constexpr tilefft::Map<S, 5> m5{};
+    static constexpr tilefft::Map<S, 4> m4{};
+    // the table's layout depends on the digits only
+    static_assert(m5.ntw == m4.ntw, "twiddle layout");
+    std::vector<double> t(size_t(2) * m5.ntw + 2);
+    auto fill = [&](int off, int digit, int low) {
+        const int P = 1 << digit, M = 1 << low;
+        for (int k = 1; k < P; ++k)
+            for (int m = 0; m < M; ++m) {
+                const double ang = -2.0 * M_PI * double(k) * double(m) / (double(P) * double(M));
+                t[size_t(2) * (off + (k - 1) * M + m)] = std::cos(ang);
+                t[size_t(2) * (off + (k - 1) * M + m) + 1] = std::sin(ang);
+            }
+    };
+    for (int p = 0; p < S::NP; ++p) {
+        if (m5.wlow[p] > 0 && S::aw[p] > 0) fill(m5.tww[p], S::aw[p], m5.wlow[p]);
+        if (m5.hlow[p] > 0 && S::ah[p] > 0) fill(m5.twh[p], S::ah[p], m5.hlow[p]);
+    }
+    return t;
+}
+
+// The tiles, and what one costs (ns, single precision, MI355X): `lat` from
+// launch to end of a single tile, `point` per complex point while a CU works
+// through many.  Fitted to kernel times of 200x5000, 512x512, 2048x2048,
+// 4096x32768 and 1-D inputs, which it gives within 20%.  Double precision
+// takes 1.8 times as long per point.
+struct Cand {
+    int lh, lw, lp;
+    bool f32, f64;      // built for one convolution per tile
+    bool sum32, sum64;  // built for sums over outer taps
+    double lat, point;
+};
+constexpr Cand kCands[] = {
+    {0, 10, 2, true, true, false, false, 3000, 0.9},  {0, 12, 3, true, true, false, false, 6000, 1.0},
+    {0, 14, 4, true, false, false, false, 22000, 1.6}, {5, 5, 2, true, true, true, true, 3000, 0.9},
+    {6, 6, 3, true, true, true, true, 6000, 1.03},     {5, 7, 3, false, true, true, true, 6500, 1.05},
+    {5, 7, 4, true, false, false, false, 7000, 0.97},  {6, 7, 4, true, false, false, false, 9000, 1.12},
+    {7, 7, 4, true, false, false, false, 20000, 1.9},
+};
+
+// Spans stay below 2^30 bytes, so that a cell's offset is 30 bits and the
+// marker of a cell that is not read (tile_kernels.hpp kNoCell) lies past it.
+constexpr int64_t kSpanMax = int64_t(1) << 30;
+// Inputs up to this size are looked over by every workgroup of a one-launch
+// plan (64 loads per thread at most).
+constexpr int64_t kScanMax = 16384;
+constexpr int64_t kMaxTaps = 16;
+
+bool side_ok(const ndc_border& b, int64_t pad, int64_t n) {
+    switch (side1d(b.tag)) {
+        case kS1Reflect: return pad <= n - 1;
+        case kS1Circular: return pad <= n;
+        default: return true;
+    }
+}
+
+TileDiv div_of(int64_t d) { return TileDiv{uint32_t(d), uint32_t(d == 1 ? 0 : ((int64_t(1) << 32) + d - 1) / d)}; }
+
+void fill_axis(const Plan& p, int i, int64_t es, TileAxis* a, int64_t ystr) {
+    std::memset(a, 0, sizeof(*a));
+    a->n = int32_t(p.x_shape[i]);
+    a->p0 = int32_t(p.pad[i][0]);
+    a->pds = int32_t(p.pds[i]);
+    const int32_t n = a->n;
+    switch (side1d(p.side[i][0].tag)) {
+        case kS1Reflect: a->fa = -1; break;
+        case kS1Circular: a->fa = 1; a->fb = n; break;
+        case kS1Replicate: break;
+        default: a->fconst = 1; break;
+    }
+    switch (side1d(p.side[i][1].tag)) {
+        case kS1Reflect: a->ba = -1; a->bb = 2 * (n - 1); break;
+        case kS1Circular: a->ba = 1; a->bb = -n; break;
+        case kS1Replicate: a->bb = n - 1; break;
+        default: a->bconst = 1; break;
+    }
+    const int64_t st = n > 1 ? p.x_str[i] * es : 0;
+    a->xs = int32_t(st);
+    a->xlo = int32_t(st < 0 ? -st * (n - 1) : 0);
+    // position j of the spectrum holds tap j, or K - 1 - j without the reversal
+    const int64_t K = p.k_shape[i], kt = K > 1 ? p.k_str[i] * es : 0, kd = p.reverse ? kt : -kt;
+    a->ks = int32_t(kd);
+    a->klo = int32_t(kd < 0 ? -kd * (K - 1) : 0);
+    a->d = int32_t(p.dil[i]);
+    a->phases = div_of(a->d);
+    a->stride = div_of(p.stride[i]);
+    a->K = int32_t(p.k_shape[i]);
+    a->s = int32_t(p.stride[i]);
+    a->U = int32_t(p.pds[i] - p.kdil[i] + 1);
+    a->ys = int32_t(ystr * es);
+}
+
+// What the multi-pass transforms take (ns), from the same measurements: a fixed
+// part per rank (their launches) and one per point.  Tiles lose only where
+// few large ones do the work: an 80x80 kernel on 512x512 (36 against 33 us), 16
+// outer taps on 30x60x60 (62 against 40 us).
+double pass_cost(const Plan& p) {
+    double pts = 1;
+    for (int i = 0; i < p.N; ++i) pts *= double(p.fft[i]);
+    if (p.N == 1) return pts <= 20000 ? 8000 + 1.5 * pts : 1e30;   // one launch while a line fits LDS
+    const double each = (dtype_is_complex(p.dtype) ? 2.0 : 1.0) * (p.dtype == NDC_F64 || p.dtype == NDC_C128 ? 1.4 : 1.0);
+    return (p.N == 2 ? 25000 : 36000 + 9000 * (p.N - 3)) + 0.03 * each * pts;
+}
+
+bool const_nonzero(const ndc_border& b) {
+    return side1d(b.tag) == kS1Const && (b.value.re != 0 || b.value.im != 0);
+}
+
+}  // namespace
+
+std::vector<double> tile_twiddles(int lh, int lw, int lp) {
+    switch ((lh * 16 + lw) * 8 + lp) {
+        case (0 * 16 + 10) * 8 + 2: return twiddles_of<0, 10, 2>();
+        case (0 * 16 + 12) * 8 + 3: return twiddles_of<0, 12, 3>();
+        case (0 * 16 + 14) * 8 + 4: return twiddles_of<0, 14, 4>();
+        case (5 * 16 + 5) * 8 + 2: return twiddles_of<5, 5, 2>();
+        case (6 * 16 + 6) * 8 + 3: return twiddles_of<6, 6, 3>();
+        case (5 * 16 + 7) * 8 + 3: return twiddles_of<5, 7, 3>();
+        case (5 * 16 + 7) * 8 + 4: return twiddles_of<5, 7, 4>();
+        case (6 * 16 + 7) * 8 + 4: return twiddles_of<6, 7, 4>();
+        case (7 * 16 + 7) * 8 + 4: return twiddles_of<7, 7, 4>();
+        default: return {};
+    }
+}
+
+bool tile_plan(const Plan& p, size_t lds, int cus, TilePlan* t) {
+    const bool cplx = dtype_is_complex(p.dtype);
+    const bool dbl = p.dtype == NDC_F64 || p.dtype == NDC_C128;
+    const int N = p.N, w = N - 1, h = N - 2;
+    const int64_t es = int64_t(dtype_size(p.dtype)), cs = dbl ? 16 : 8;
+    if ((p.x_hi - p.x_lo + 1) * es >= kSpanMax || (p.k_hi - p.k_lo + 1) * es >= kSpanMax || p.y_numel * es >= kSpanMax) return false;
+    int64_t taps = 1, planes = 1;
+    for (int i = 0; i < N; ++i) {
+        if (!side_ok(p.side[i][0], p.pad[i][0], p.x_shape[i]) || !side_ok(p.side[i][1], p.pad[i][1], p.x_shape[i]))
+            return false;
+        // room for the positions a tile reaches past the padded extent
+        if (p.pds[i] + (int64_t(p.dil[i]) << 14) >= kSpanMax) return false;
+        if (i < h) {
+            taps *= p.k_shape[i];
+            planes *= p.out[i];
+        }
+    }
+    if (taps > kMaxTaps) return false;
+    const bool compact = p.x_hi - p.x_lo + 1 == p.x_numel;
+    const bool one = N == 1 && p.x_numel <= kScanMax;
+    if (one && !compact) return false;
+
+    auto tiles = [&](int i, int lsz, int64_t* V) -> int64_t {
+        *V = (int64_t(1) << lsz) - p.k_shape[i] + 1;
+        const int64_t U = p.pds[i] - p.kdil[i] + 1;
+        const int64_t per = (U + p.dil[i] - 1) / p.dil[i];   // outputs of a phase
+        return *V > 0 ? (per + *V - 1) / *V : 0;
+    };
+    double best = 0;
+    for (const Cand& c : kCands) {
+        if ((N == 1) != (c.lh == 0)) continue;
+        if (!(N > 2 ? (dbl ? c.sum64 : c.sum32) : (dbl ? c.f64 : c.f32))) continue;
+        if (one && c.lw > 12) continue;
+        const int64_t pts = int64_t(1) << (c.lh + c.lw);
+        if (size_t(pts * cs) > lds) continue;
+        int64_t vw, vh = 1;
+        const int64_t nw = tiles(w, c.lw, &vw);
+        const int64_t nh = N == 1 ? 1 : tiles(h, c.lh, &vh);
+        if (nw <= 0 || nh <= 0 || vw * vh * 8 < pts) continue;
+        // real elements: the axis whose number of tiles wastes the smaller
+        // part of its pairs
+        const int64_t cw = nw * p.dil[w], ch = N == 1 ? 1 : nh * p.dil[h];
+        const bool pair_w = ((cw + 1) / 2) * ch <= cw * ((ch + 1) / 2);
+        const int64_t pw = !cplx && pair_w ? (cw + 1) / 2 : cw, ph = !cplx && !pair_w ? (ch + 1) / 2 : ch;
+        if (cw >= kSpanMax || ch >= kSpanMax || double(pw) * double(ph) * double(planes) >= double(kSpanMax)) continue;
+        const int64_t pi = pw * ph, items = pi * planes;
+        // a sum over outer taps transforms once per tap and once back
+        const double trips = N > 2 ? 0.425 * (1.0 + double(taps)) : 1.0;
+        const double cost = (c.lat + c.point * (dbl ? 1.8 : 1.0) * double(pts) * double(items) / cus) * trips +
+                            (one ? 0.0 : 0.6 * c.lat + 3000.0);   // the spectrum and fix-up launches
+        if (best != 0 && cost >= best) continue;
+        best = cost;
+        t->lh = c.lh;
+        t->lw = c.lw;
+        t->lp = c.lp;
+        t->threads = int(pts >> c.lp);
+        t->lds = size_t(pts * cs);
+        t->spec_bytes = size_t(pts * cs) * size_t(taps);
+        std::memset(&t->a, 0, sizeof(t->a));
+        t->a.pair_w = pair_w ? 1 : 0;
+        t->a.ax[0].pairs = div_of(ph);
+        t->a.ax[1].pairs = div_of(pw);
+        t->a.plane_items = div_of(pi);
+        t->a.items = int32_t(items);
+        t->a.ax[0].V = int32_t(vh);
+        t->a.ax[0].tiles = div_of(nh);
+        t->a.ax[1].V = int32_t(vw);
+        t->a.ax[1].tiles = div_of(nw);
+    }
+    if (best == 0 || best > pass_cost(p)) return false;
+
+    TileArgs& a = t->a;
+    t->one = one;
+    a.x_bytes = int32_t((p.x_hi - p.x_lo + 1) * es);
+    a.y_bytes = int32_t(p.y_numel * es);
+    a.ntaps = int32_t(taps);
+    a.nouter = std::max(0, h);
+    a.k_bytes = int32_t((p.k_hi - p.k_lo + 1) * es);
+    t->fills = false;
+    // a single workgroup sees all of x anyway
+    a.scan = one && a.items > 1 ? int32_t(p.x_numel * (cplx ? 2 : 1)) : 0;
+    int64_t ystr[kMaxRank], ys = 1;
+    for (int i = N - 1; i >= 0; --i) {
+        ystr[i] = ys;
+        ys *= p.out[i];
+    }
+    auto axis = [&](int i, TileAxis* dst, int slot) {
+        const int32_t V = dst->V;
+        const TileDiv nt = dst->tiles, np = dst->pairs;
+        fill_axis(p, i, es, dst, ystr[i]);
+        dst->V = V;
+        dst->tiles = nt;
+        dst->pairs = np;
+        for (int s = 0; s < 2; ++s) {
+            a.cst[slot][s][0] = p.side[i][s].value.re;
+            a.cst[slot][s][1] = p.side[i][s].value.im;
+            if (p.pad[i][s] > 0 && const_nonzero(p.side[i][s])) t->fills = true;
+        }
+    };
+    axis(w, &a.ax[1], 1);
+    if (N > 1) {
+        axis(h, &a.ax[0], 0);
+    } else {
+        TileAxis& u = a.ax[0];   // a single row
+        u.n = u.pds = u.d = u.K = u.V = u.U = u.s = 1;
+        u.phases = u.tiles = u.pairs = u.stride = div_of(1);
+        u.fconst = u.bconst = 1;
+    }
+    for (int i = 0; i < h; ++i) {
+        axis(i, &a.outer[i].a, 2 + i);
+        a.outer[i].out = div_of(p.out[i]);
+        a.outer[i].taps = div_of(p.k_shape[i]);
+    }
+    return true;
+}
+
+ndc_status launch_tile(const Plan& p, const TilePlan& t, const void* x, const void* k, void* y, LaunchContext& ctx,
+                       KernelSpectrum* ks) {
+    const bool cplx = dtype_is_complex(p.dtype);
+    const bool dbl = p.dtype == NDC_F64 || p.dtype == NDC_C128;
+    TileArgs a = t.a;
+    a.x = x ? static_cast<const char*>(x) + p.x_lo * int64_t(dtype_size(p.dtype)) : nullptr;
+    a.k = k ? static_cast<const char*>(k) + p.k_lo * int64_t(dtype_size(p.dtype)) : nullptr;
+    a.y = y;
+    if (!t.tw || !t.flag) {
+        const std::string key = "tile:" + std::to_string(t.lh) + ":" + std::to_string(t.lw) + ":" + std::to_string(t.lp) + (dbl ? ":d" : ":f");
+        const std::vector<double> tab = tile_twiddles(t.lh, t.lw, t.lp);
+        const std::vector<float> f(tab.begin(), tab.end());
+        t.tw = dbl ? ctx.constant_table(key, tab.data(), tab.size() * sizeof(double))
+                   : ctx.constant_table(key, f.data(), f.size() * sizeof(float));
+        const uint32_t zeros[2] = {0, 0};
+        t.flag = static_cast<uint32_t*>(const_cast<void*>(ctx.constant_table("tile:flag", zeros, sizeof(zeros))));
+    }
+    a.tw = t.tw;
+    a.flag = t.flag;
+    if (!a.tw || !a.flag) {
+        if (ctx.err.empty()) ctx.err = "tile table allocation failed";
+        return NDC_ERR_OUT_OF_MEMORY;
+    }
+    auto go = [&](int what) {
+        return dbl ? launch_tile_as<double>(t, a, cplx, what, ctx) : launch_tile_as<float>(t, a, cplx, what, ctx);
+    };
+    if (ks) {
+        a.spec = ks->spec;
+        a.have_spec = 1;
+        if (ks->bake) return go(0);
+    } else if (!t.one) {
+        a.spec = ctx.scratch(0, t.spec_bytes);
+        if (!a.spec) {
+            if (ctx.err.empty()) ctx.err = "kernel spectrum allocation failed";
+            return NDC_ERR_OUT_OF_MEMORY;
+        }
+        const ndc_status s = go(0);
+        if (s != NDC_OK) return s;
+    }
+    ndc_status s = go(1);
+    if (s == NDC_OK && !t.one) s = go(2);
+    return s;
+}
+
+}  // namespace ndc
