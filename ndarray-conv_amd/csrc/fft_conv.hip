@@ -2118,6 +2118,8 @@ __global__ void __launch_bounds__(kMaxThreads) line_fft_kernel(LineFftArgs<R> a)
     const bool half = a.mode != 0 && L * 2 == a.n;   // even real line: half-length transform
     const int tot = L * Ct;
     const float rL = 1.0f / float(L);
+    // the c2r load reads the post-processing factors that other threads staged
+    if (a.mode == 2) __syncthreads();
     for (int b = threadIdx.x; b < tot; b += kU * T) {
         C v[kU];
 #pragma unroll

@@ -116,3 +116,19 @@ def test_baked_is_the_same(gpu, shape, k):
     b = nc.conv_fft_bake(x, kv, nc.ConvMode.Same, nc.PaddingMode.Circular)
     y = nc.conv_fft(x, kv, nc.ConvMode.Same, nc.PaddingMode.Circular)
     np.testing.assert_array_equal(nc.conv_fft_with_baked(x, b), y)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_processor_after_other_kernels(gpu, dtype):
+    """The inverse transform's first reads of the factors it stages in LDS,
+    where another kernel has left other values."""
+    rng = np.random.default_rng(8)
+    x, k = rand_array(rng, (300, 400), dtype), rand_array(rng, (9, 9), dtype)
+    p = nc.get_fft_processor(dtype)
+    for n in (32, 100, 250, 1024):
+        a = rand_array(rng, (32, n), dtype)
+        spec = p.forward(a)
+        for _ in range(3):
+            nc.conv_fft(x, k, nc.ConvMode.Same, nc.PaddingMode.Zeros)
+            assert O.relerr(p.backward(spec), a)[0] <= (1e-5 if dtype == np.float32 else 1e-12)
+    p.close()
