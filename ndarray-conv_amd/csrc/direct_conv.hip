@@ -16,6 +16,7 @@
 #include "border1d.hpp"
 #include "device_common.hpp"
 #include "launch.hpp"
+#include "matrix_conv.hpp"
 
 namespace ndc {
 namespace {
@@ -491,6 +492,8 @@ double2 cst_c128(const ndc_value& v) { return cmake<double2>(v.re, v.im); }
 }  // namespace
 
 ndc_status launch_direct(const Plan& p, const void* x, const void* k, void* y, LaunchContext& ctx) {
+    ndc_status s;
+    if (launch_matrix(p, true, x, k, y, ctx, &s)) return s;
     switch (p.dtype) {
         case NDC_F32: return launch_typed<float>(p, x, k, y, ctx, cst_real<float>);
         case NDC_F64: return launch_typed<double>(p, x, k, y, ctx, cst_real<double>);

@@ -25,6 +25,7 @@
 #include "bf16_split.hpp"
 #include "device_common.hpp"
 #include "launch.hpp"
+#include "matrix_conv.hpp"
 
 namespace ndc {
 namespace {
@@ -450,6 +451,22 @@ ndc_status launch_direct_mfma(const Plan& p, const void* x, const void* k, void*
         const int64_t g = gcd64(sx, dx);
         if (((kXB - 1) * sx + 15 * dx) / g + 1 <= kMaxW) return launch_direct(p, x, k, y, ctx);
     }
+    // kernel columns per pass: up to 64 (four K-blocks of 16), fewer when the
+    // staged row (128 outputs plus the dilated column span) would not fit
+    int nkb = 0;
+    for (int cand = 4; cand >= 1; --cand) {
+        const int64_t w = ((kXB - 1) * sx + (16 * cand - 1) * dx) / gcd64(sx, dx) + 1;
+        if (w <= kMaxW) {
+            nkb = cand;
+            break;
+        }
+    }
+    if (!nkb) {
+        ctx.err = "stride/dilation too large for the staged rows of the matrix-core form";
+        return NDC_ERR_UNSUPPORTED;
+    }
+    ndc_status s;
+    if (launch_matrix(p, false, x, k, y, ctx, &s)) return s;
     int64_t offs[kMaxRank + 1];
     const int32_t* maps = ctx.border_maps(p, offs);
     if (!maps) return NDC_ERR_OUT_OF_MEMORY;
@@ -478,21 +495,6 @@ ndc_status launch_direct_mfma(const Plan& p, const void* x, const void* k, void*
     a.rev = p.reverse ? 1 : 0;
     const int Q = int(dy / sy);
     a.gx = int32_t(gcd64(sx, dx));
-    // kernel columns per pass: up to 64 (four K-blocks of 16), fewer when the
-    // staged row (128 outputs plus the dilated column span) would not fit
-    int nkb = 0;
-    for (int cand = 4; cand >= 1; --cand) {
-        const int64_t w = ((kXB - 1) * sx + (16 * cand - 1) * dx) / a.gx + 1;
-        if (w <= kMaxW) {
-            nkb = cand;
-            a.W = int32_t(w);
-            break;
-        }
-    }
-    if (!nkb) {
-        ctx.err = "stride/dilation too large for the staged rows of the matrix-core form";
-        return NDC_ERR_UNSUPPORTED;
-    }
     nkb = std::min(nkb, int((a.KW + 15) / 16));
     a.W = int32_t(((kXB - 1) * sx + (16 * nkb - 1) * dx) / a.gx + 1);
     const bool d1 = dx / a.gx == 1;

@@ -87,6 +87,14 @@ ndc_status launch_tile(const Plan& p, const TilePlan& t, const void* x, const vo
 template <typename R> ndc_status launch_tile_as(const TilePlan& t, const TileArgs& a, bool cplx, int what,
                                                 LaunchContext& ctx);
 
+// For other kernels that read their input through TileAxis (cell_offset):
+// whether every span of the plan is below 2^30 bytes and every pad within its
+// axis, the division constants, and one axis of a plan (ystr: elements of y
+// from one output to the next).
+bool tile_spans_fit(const Plan& p);
+TileDiv tile_div(int64_t d);
+void tile_axis(const Plan& p, int i, int64_t ystr, TileAxis* a);
+
 // Host table of a tile's twiddles, empty for an unknown tile.
 std::vector<double> tile_twiddles(int lh, int lw, int lp);
 

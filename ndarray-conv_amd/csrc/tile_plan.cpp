@@ -77,9 +77,28 @@ bool side_ok(const ndc_border& b, int64_t pad, int64_t n) {
     }
 }
 
-TileDiv div_of(int64_t d) { return TileDiv{uint32_t(d), uint32_t(d == 1 ? 0 : ((int64_t(1) << 32) + d - 1) / d)}; }
+// What the multi-pass transforms take (ns), from the same measurements: a fixed
+// part per rank (their launches) and one per point.  Tiles lose only where
+// few large ones do the work: an 80x80 kernel on 512x512 (36 against 33 us), 16
+// outer taps on 30x60x60 (62 against 40 us).
+double pass_cost(const Plan& p) {
+    double pts = 1;
+    for (int i = 0; i < p.N; ++i) pts *= double(p.fft[i]);
+    if (p.N == 1) return pts <= 20000 ? 8000 + 1.5 * pts : 1e30;   // one launch while a line fits LDS
+    const double each = (dtype_is_complex(p.dtype) ? 2.0 : 1.0) * (p.dtype == NDC_F64 || p.dtype == NDC_C128 ? 1.4 : 1.0);
+    return (p.N == 2 ? 25000 : 36000 + 9000 * (p.N - 3)) + 0.03 * each * pts;
+}
 
-void fill_axis(const Plan& p, int i, int64_t es, TileAxis* a, int64_t ystr) {
+bool const_nonzero(const ndc_border& b) {
+    return side1d(b.tag) == kS1Const && (b.value.re != 0 || b.value.im != 0);
+}
+
+}  // namespace
+
+TileDiv tile_div(int64_t d) { return TileDiv{uint32_t(d), uint32_t(d == 1 ? 0 : ((int64_t(1) << 32) + d - 1) / d)}; }
+
+void tile_axis(const Plan& p, int i, int64_t ystr, TileAxis* a) {
+    const int64_t es = int64_t(dtype_size(p.dtype));
     std::memset(a, 0, sizeof(*a));
     a->n = int32_t(p.x_shape[i]);
     a->p0 = int32_t(p.pad[i][0]);
@@ -105,31 +124,26 @@ void fill_axis(const Plan& p, int i, int64_t es, TileAxis* a, int64_t ystr) {
     a->ks = int32_t(kd);
     a->klo = int32_t(kd < 0 ? -kd * (K - 1) : 0);
     a->d = int32_t(p.dil[i]);
-    a->phases = div_of(a->d);
-    a->stride = div_of(p.stride[i]);
+    a->phases = tile_div(a->d);
+    a->stride = tile_div(p.stride[i]);
     a->K = int32_t(p.k_shape[i]);
     a->s = int32_t(p.stride[i]);
     a->U = int32_t(p.pds[i] - p.kdil[i] + 1);
     a->ys = int32_t(ystr * es);
 }
 
-// What the multi-pass transforms take (ns), from the same measurements: a fixed
-// part per rank (their launches) and one per point.  Tiles lose only where
-// few large ones do the work: an 80x80 kernel on 512x512 (36 against 33 us), 16
-// outer taps on 30x60x60 (62 against 40 us).
-double pass_cost(const Plan& p) {
-    double pts = 1;
-    for (int i = 0; i < p.N; ++i) pts *= double(p.fft[i]);
-    if (p.N == 1) return pts <= 20000 ? 8000 + 1.5 * pts : 1e30;   // one launch while a line fits LDS
-    const double each = (dtype_is_complex(p.dtype) ? 2.0 : 1.0) * (p.dtype == NDC_F64 || p.dtype == NDC_C128 ? 1.4 : 1.0);
-    return (p.N == 2 ? 25000 : 36000 + 9000 * (p.N - 3)) + 0.03 * each * pts;
+bool tile_spans_fit(const Plan& p) {
+    const int64_t es = int64_t(dtype_size(p.dtype));
+    if ((p.x_hi - p.x_lo + 1) * es >= kSpanMax || (p.k_hi - p.k_lo + 1) * es >= kSpanMax || p.y_numel * es >= kSpanMax)
+        return false;
+    for (int i = 0; i < p.N; ++i) {
+        if (!side_ok(p.side[i][0], p.pad[i][0], p.x_shape[i]) || !side_ok(p.side[i][1], p.pad[i][1], p.x_shape[i]))
+            return false;
+        // room for the positions a tile reaches past the padded extent
+        if (p.pds[i] + (int64_t(p.dil[i]) << 14) >= kSpanMax) return false;
+    }
+    return true;
 }
-
-bool const_nonzero(const ndc_border& b) {
-    return side1d(b.tag) == kS1Const && (b.value.re != 0 || b.value.im != 0);
-}
-
-}  // namespace
 
 std::vector<double> tile_twiddles(int lh, int lw, int lp) {
     switch ((lh * 16 + lw) * 8 + lp) {
@@ -151,13 +165,9 @@ bool tile_plan(const Plan& p, size_t lds, int cus, TilePlan* t) {
     const bool dbl = p.dtype == NDC_F64 || p.dtype == NDC_C128;
     const int N = p.N, w = N - 1, h = N - 2;
     const int64_t es = int64_t(dtype_size(p.dtype)), cs = dbl ? 16 : 8;
-    if ((p.x_hi - p.x_lo + 1) * es >= kSpanMax || (p.k_hi - p.k_lo + 1) * es >= kSpanMax || p.y_numel * es >= kSpanMax) return false;
+    if (!tile_spans_fit(p)) return false;
     int64_t taps = 1, planes = 1;
     for (int i = 0; i < N; ++i) {
-        if (!side_ok(p.side[i][0], p.pad[i][0], p.x_shape[i]) || !side_ok(p.side[i][1], p.pad[i][1], p.x_shape[i]))
-            return false;
-        // room for the positions a tile reaches past the padded extent
-        if (p.pds[i] + (int64_t(p.dil[i]) << 14) >= kSpanMax) return false;
         if (i < h) {
             taps *= p.k_shape[i];
             planes *= p.out[i];
@@ -206,14 +216,14 @@ bool tile_plan(const Plan& p, size_t lds, int cus, TilePlan* t) {
         t->spec_bytes = size_t(pts * cs) * size_t(taps);
         std::memset(&t->a, 0, sizeof(t->a));
         t->a.pair_w = pair_w ? 1 : 0;
-        t->a.ax[0].pairs = div_of(ph);
-        t->a.ax[1].pairs = div_of(pw);
-        t->a.plane_items = div_of(pi);
+        t->a.ax[0].pairs = tile_div(ph);
+        t->a.ax[1].pairs = tile_div(pw);
+        t->a.plane_items = tile_div(pi);
         t->a.items = int32_t(items);
         t->a.ax[0].V = int32_t(vh);
-        t->a.ax[0].tiles = div_of(nh);
+        t->a.ax[0].tiles = tile_div(nh);
         t->a.ax[1].V = int32_t(vw);
-        t->a.ax[1].tiles = div_of(nw);
+        t->a.ax[1].tiles = tile_div(nw);
     }
     if (best == 0 || best > pass_cost(p)) return false;
 
@@ -235,7 +245,7 @@ bool tile_plan(const Plan& p, size_t lds, int cus, TilePlan* t) {
     auto axis = [&](int i, TileAxis* dst, int slot) {
         const int32_t V = dst->V;
         const TileDiv nt = dst->tiles, np = dst->pairs;
-        fill_axis(p, i, es, dst, ystr[i]);
+        tile_axis(p, i, ystr[i], dst);
         dst->V = V;
         dst->tiles = nt;
         dst->pairs = np;
@@ -251,13 +261,13 @@ bool tile_plan(const Plan& p, size_t lds, int cus, TilePlan* t) {
     } else {
         TileAxis& u = a.ax[0];   // a single row
         u.n = u.pds = u.d = u.K = u.V = u.U = u.s = 1;
-        u.phases = u.tiles = u.pairs = u.stride = div_of(1);
+        u.phases = u.tiles = u.pairs = u.stride = tile_div(1);
         u.fconst = u.bconst = 1;
     }
     for (int i = 0; i < h; ++i) {
         axis(i, &a.outer[i].a, 2 + i);
-        a.outer[i].out = div_of(p.out[i]);
-        a.outer[i].taps = div_of(p.k_shape[i]);
+        a.outer[i].out = tile_div(p.out[i]);
+        a.outer[i].taps = tile_div(p.k_shape[i]);
     }
     return true;
 }
