@@ -17,6 +17,8 @@
 #include "device_common.hpp"
 #include "launch.hpp"
 #include "matrix_conv.hpp"
+#include "tile_conv.hpp"
+#include "tile_kernels.hpp"
 
 namespace ndc {
 namespace {
@@ -34,8 +36,11 @@ template <typename T> constexpr int kMaxTileY = sizeof(T) > 8 ? 16 : (sizeof(T) 
 template <typename T> constexpr int staged_per_round() { return sizeof(T) > 8 ? 2 : 8; }
 
 // Kernel columns per register window of the sliding form (32 for 4-byte
-// elements, 16 for wider ones, whose windows would spill).
+// elements, 16 for wider ones, whose windows would spill); kernels of up to 8
+// columns take windows of 8 where an element is wider than 4 bytes (5x5 f64
+// taps on 480x640: 1.5 us less).
 template <typename T> constexpr int kCX = sizeof(T) == 4 ? 32 : 16;
+template <typename T> constexpr int kCXSmall = sizeof(T) > 4 ? 8 : kCX<T>;
 
 // A value every lane holds identically (a broadcast LDS read), moved to
 // scalar registers: the zero-tap test becomes a scalar branch and the
@@ -82,6 +87,11 @@ struct DirectArgs {
     int32_t TO;         // element offset of the taps in LDS, after the region, 16-byte aligned
     int32_t KS;         // tap row stride in LDS: KXc rounded up to kCX (zero-filled)
     int32_t ntx, nty;   // tiles per plane
+    // FAST staging: x from its lowest element, and the axes in byte offsets
+    const void* xbase;
+    int32_t x_bytes;
+    int32_t fills;      // some fill writes a constant other than zero
+    TileAxis ta[2];     // rows, columns
 };
 
 // Elements per 16-byte LDS read of the sliding form's taps: 4 for 4-byte
@@ -137,13 +147,77 @@ __device__ __forceinline__ bool plane_source(const DirectArgs<T>& a, int32_t cy,
     return true;
 }
 
+// Raw bits of an element through a buffer: out of its range reads zero.
+template <typename T>
+__device__ __forceinline__ T buffer_elem(__amdgpu_buffer_rsrc_t b, uint32_t off) {
+    if constexpr (sizeof(T) == 1) return __builtin_bit_cast(T, uint8_t(__builtin_amdgcn_raw_buffer_load_b8(b, int(off), 0, 0)));
+    else if constexpr (sizeof(T) == 2) return __builtin_bit_cast(T, uint16_t(__builtin_amdgcn_raw_buffer_load_b16(b, int(off), 0, 0)));
+    else if constexpr (sizeof(T) == 4) return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(b, int(off), 0, 0));
+    else if constexpr (sizeof(T) == 8) return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(b, int(off), 0, 0));
+    else return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b128(b, int(off), 0, 0));
+}
+
+// Byte offsets in x of the region's columns, then rows (tilek::kNoCell where x
+// is not read), so that staging a cell is two LDS reads and an addition instead
+// of two border rules and a 64-bit address.
+template <typename T>
+__device__ __forceinline__ void stage_offsets(uint32_t* offs, const DirectArgs<T>& a, int py0, int px0, bool outer_const) {
+    for (int i = threadIdx.x; i < a.RX + a.RY; i += kThreads)
+        offs[i] = outer_const ? tilek::kNoCell
+                  : i < a.RX ? tilek::cell_offset(a.ta[1], px0 + i * a.gx)
+                             : tilek::cell_offset(a.ta[0], py0 + (i - a.RX) * a.gy);
+}
+
+// Stages the region from those offsets, kU loads a thread in flight.  A 480x640
+// f64 image with 5x5 taps spent 6 of its 17 us on staging 32x64-output tiles.
+template <typename T>
+__device__ __forceinline__ void stage_region(T* region, const uint32_t* offs, const DirectArgs<T>& a, int py0, int px0,
+                                             int xoff, bool outer_const, T ocval) {
+    constexpr int kU = sizeof(T) > 8 ? 4 : 12;
+    const int ay = a.No - 2, ax = a.No - 1;
+    const __amdgpu_buffer_rsrc_t b = tilek::buffer_of(static_cast<const char*>(a.xbase) + xoff, a.x_bytes - xoff);
+    const int n = a.RX * a.RY, dr = kThreads / a.RX, dc = kThreads - dr * a.RX;
+    int r = int(threadIdx.x) / a.RX, c = int(threadIdx.x) - r * a.RX;
+    for (int i0 = threadIdx.x; i0 < n; i0 += kU * kThreads) {
+        T v[kU];
+        int rr[kU], cc[kU];
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+            rr[u] = r;
+            cc[u] = c;
+            v[u] = buffer_elem<T>(b, r < a.RY ? offs[c] + offs[a.RX + r] : tilek::kNoCell);
+            r += dr;
+            c += dc;
+            if (c >= a.RX) {
+                c -= a.RX;
+                ++r;
+            }
+        }
+        if (a.fills) {
+#pragma unroll
+            for (int u = 0; u < kU; ++u) {
+                const int kx = tilek::cell_kind(a.ta[1], px0 + cc[u] * a.gx);
+                const int ky = tilek::cell_kind(a.ta[0], py0 + rr[u] * a.gy);
+                if (kx == 3 || ky == 3) continue;   // beyond what any output reads
+                // the highest axis whose fill wrote a constant wins
+                if (kx) v[u] = a.cst[ax][kx - 1];
+                else if (ky) v[u] = a.cst[ay][ky - 1];
+                else if (outer_const) v[u] = ocval;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kU; ++u)
+            if (i0 + u * kThreads < n) region[i0 + u * kThreads] = v[u];
+    }
+}
+
 // SLIDE (stride equal to dilation along the row, so consecutive outputs read
 // consecutive staged columns): each thread computes kItems (16, 8 or 4)
 // adjacent outputs of one tile row from a register window of
 // kCX + kItems - 1 staged values per kCX kernel columns, instead of one LDS
 // read per product.  The taps of an
 // output are summed in the same order in both forms.
-template <typename T, bool SLIDE, int TY>
+template <typename T, bool SLIDE, int TY, bool FAST, int CX>
 __global__ void __launch_bounds__(kThreads) direct_conv_kernel(DirectArgs<T> a) {
     constexpr int kItems = TY * kTileX / kThreads;
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -151,11 +225,11 @@ __global__ void __launch_bounds__(kThreads) direct_conv_kernel(DirectArgs<T> a) 
     T* taps = region + a.TO;
 
     const int ay = a.No - 2, ax = a.No - 1;
-    int64_t bid = blockIdx.x;
-    const int tx = int(bid % a.ntx);
-    bid /= a.ntx;
-    const int ty = int(bid % a.nty);
-    int64_t outer = bid / a.nty;
+    unsigned bid = blockIdx.x;
+    const int tx = int(bid % unsigned(a.ntx));
+    bid /= unsigned(a.ntx);
+    const int ty = int(bid % unsigned(a.nty));
+    int64_t outer = bid / unsigned(a.nty);
 
     // outer output coordinates (axes 0..No-3)
     int64_t oo[kMaxRank];
@@ -200,7 +274,7 @@ __global__ void __launch_bounds__(kThreads) direct_conv_kernel(DirectArgs<T> a) 
                 rem /= a.K[e];
                 const int64_t pe = oo[e] * a.s[e] + t * a.d[e];
                 const int32_t c = axis_code(a, e, int(pe));
-                if (c >= 0) xoff += int64_t(c) * a.xstr[e];
+                if (c >= 0) xoff += int64_t(c) * a.xstr[e] * (FAST ? int(sizeof(T)) : 1);
                 else if (c == kUnwritten) ounw = true;
                 else if (oc_axis < e) { oc_axis = e; ocval = a.cst[e][c == kConstFront ? 0 : 1]; }
                 koff += (a.rev ? a.K[e] - 1 - t : t) * a.kstr[e];
@@ -220,8 +294,26 @@ __global__ void __launch_bounds__(kThreads) direct_conv_kernel(DirectArgs<T> a) 
                 // out first, then all of the round's loads are issued, then the
                 // values are selected and written, so the loads overlap.
                 constexpr int kSU = staged_per_round<T>();
-                const int nreg = a.RY * a.RX;
+                const int nreg = FAST ? 0 : a.RY * a.RX;
                 const float rRX = 1.0f / float(a.RX);
+                // the first taps travel while the region does
+                T tap0 = Arith<T>::zero();
+                auto tap_at = [&](int i) {
+                    const int cy = i / a.KS, cx = i - cy * a.KS;
+                    if (cx >= kxn) return Arith<T>::zero();
+                    const int64_t ty_ = ky0 + cy, tx_ = kx0 + cx;
+                    const int64_t kiy = a.rev ? a.K[ay] - 1 - ty_ : ty_;
+                    const int64_t kix = a.rev ? a.K[ax] - 1 - tx_ : tx_;
+                    return a.k[koff + kiy * a.kstr[ay] + kix * a.kstr[ax]];
+                };
+                if (int(threadIdx.x) < kyn * a.KS) tap0 = tap_at(threadIdx.x);
+                if constexpr (FAST) {
+                    uint32_t* offs = reinterpret_cast<uint32_t*>(
+                        smem_raw + ((size_t(a.TO + a.KYc * a.KS) * sizeof(T) + 3) & ~size_t(3)));
+                    stage_offsets<T>(offs, a, int(py0), int(px0), oc_axis >= 0);
+                    __syncthreads();
+                    stage_region<T>(region, offs, a, int(py0), int(px0), oc_axis < 0 ? int(xoff) : 0, oc_axis >= 0, ocval);
+                }
                 for (int i0 = threadIdx.x; i0 < nreg; i0 += kSU * kThreads) {
                     int64_t off[kSU];
                     T fill[kSU];
@@ -253,40 +345,30 @@ __global__ void __launch_bounds__(kThreads) direct_conv_kernel(DirectArgs<T> a) 
                 }
                 // stage the kernel taps of this chunk (value of reversed-view tap
                 // t), rows KS apart, zeros past kxn
-                for (int i = threadIdx.x; i < kyn * a.KS; i += kThreads) {
-                    const int cy = i / a.KS, cx = i - cy * a.KS;
-                    T v = Arith<T>::zero();
-                    if (cx < kxn) {
-                        const int64_t ty_ = ky0 + cy, tx_ = kx0 + cx;
-                        const int64_t kiy = a.rev ? a.K[ay] - 1 - ty_ : ty_;
-                        const int64_t kix = a.rev ? a.K[ax] - 1 - tx_ : tx_;
-                        v = a.k[koff + kiy * a.kstr[ay] + kix * a.kstr[ax]];
-                    }
-                    taps[i] = v;
-                }
+                for (int i = threadIdx.x; i < kyn * a.KS; i += kThreads) taps[i] = i < kThreads ? tap0 : tap_at(i);
                 __syncthreads();
                 if constexpr (SLIDE) {
                     for (int cy = 0; cy < kyn; ++cy) {
                         const T* rrow = region + (ly0 * sy_ + cy * dy_) * a.RX + lx;
                         const T* trow = taps + cy * a.KS;
-                        for (int cx0 = 0; cx0 < kxn; cx0 += kCX<T>) {
+                        for (int cx0 = 0; cx0 < kxn; cx0 += CX) {
                             // window values this chunk uses: up to column lx + kxn + kItems - 2 < RX
-                            const int nw = min(kCX<T>, kxn - cx0) + kItems - 1;
-                            T w[kCX<T> + kItems - 1];
+                            const int nw = min(CX, kxn - cx0) + kItems - 1;
+                            T w[CX + kItems - 1];
 #pragma unroll
-                            for (int i = 0; i < kCX<T> + kItems - 1; ++i)
+                            for (int i = 0; i < CX + kItems - 1; ++i)
                                 w[i] = i < nw ? rrow[cx0 + i] : Arith<T>::zero();
                             // the chunk's kCX taps (a broadcast read; trow + cx0 is 16-byte
                             // aligned: TO, KS and cx0 are multiples of vec_elems)
-                            T tv[kCX<T>];
+                            T tv[CX];
                             if constexpr (vec_elems<T>() > 1) {
                                 lds_vec_load(trow + cx0, tv);
                             } else {
 #pragma unroll
-                                for (int c = 0; c < kCX<T>; ++c) tv[c] = trow[cx0 + c];
+                                for (int c = 0; c < CX; ++c) tv[c] = trow[cx0 + c];
                             }
 #pragma unroll
-                            for (int c = 0; c < kCX<T>; ++c) {
+                            for (int c = 0; c < CX; ++c) {
                                 // taps past kxn are the zero padding of the row: skipped below
                                 const T v = wave_uniform(tv[c]);
                                 if (Arith<T>::is_zero(v)) continue;   // zero taps are not in the offset list
@@ -342,18 +424,24 @@ int64_t gcd64(int64_t a, int64_t b) {
 }
 
 // Launches the TY-row form; false when its LDS request does not fit.
-template <typename T, int TY>
-bool launch_tile(LaunchContext& ctx, bool slide, const DirectArgs<T>& a, int64_t nblocks, size_t smem) {
-    const void* kp = slide ? reinterpret_cast<const void*>(&direct_conv_kernel<T, true, TY>)
-                           : reinterpret_cast<const void*>(&direct_conv_kernel<T, false, TY>);
+template <typename T, int TY, bool FAST, int CX>
+bool launch_staged(LaunchContext& ctx, bool slide, const DirectArgs<T>& a, int64_t nblocks, size_t smem) {
+    const void* kp = slide ? reinterpret_cast<const void*>(&direct_conv_kernel<T, true, TY, FAST, CX>)
+                           : reinterpret_cast<const void*>(&direct_conv_kernel<T, false, TY, FAST, kCX<T>>);
     if (!lds_fits(ctx, kp, smem)) return false;
     if (slide)
-        NDC_LAUNCH(ctx, ctx.stream(), (direct_conv_kernel<T, true, TY>),
+        NDC_LAUNCH(ctx, ctx.stream(), (direct_conv_kernel<T, true, TY, FAST, CX>),
             dim3(unsigned(nblocks)), dim3(kThreads), smem, a);
     else
-        NDC_LAUNCH(ctx, ctx.stream(), (direct_conv_kernel<T, false, TY>),
+        NDC_LAUNCH(ctx, ctx.stream(), (direct_conv_kernel<T, false, TY, FAST, kCX<T>>),
             dim3(unsigned(nblocks)), dim3(kThreads), smem, a);
     return true;
+}
+template <typename T, int TY>
+bool launch_tile(LaunchContext& ctx, bool slide, const DirectArgs<T>& a, int64_t nblocks, size_t smem) {
+    if (!a.xbase) return launch_staged<T, TY, false, kCX<T>>(ctx, slide, a, nblocks, smem);
+    return a.KS < kCX<T> ? launch_staged<T, TY, true, kCXSmall<T>>(ctx, slide, a, nblocks, smem)
+                         : launch_staged<T, TY, true, kCX<T>>(ctx, slide, a, nblocks, smem);
 }
 
 template <typename T>
@@ -404,6 +492,26 @@ ndc_status launch_typed(const Plan& p, const void* x, const void* k, void* y, La
     a.y = static_cast<T*>(y);
     a.rev = p.reverse ? 1 : 0;
     const int ay = a.No - 2, ax = a.No - 1;
+    if (tile_spans_fit(p)) {   // offsets of 30 bits, pads within their axes: staged row by row
+        a.x_bytes = int32_t((p.x_hi - p.x_lo + 1) * int64_t(sizeof(T)));
+        a.xbase = static_cast<const T*>(x) + p.x_lo;
+        if (p.N > 1) {
+            tile_axis(p, p.N - 2, 0, &a.ta[0]);
+        } else {
+            a.ta[0].n = a.ta[0].pds = 1;
+            a.ta[0].fconst = a.ta[0].bconst = 1;
+        }
+        tile_axis(p, p.N - 1, 0, &a.ta[1]);
+        int64_t xlo = 0;   // what the outer axes' offsets start from
+        for (int i = 0; i < p.N; ++i) {
+            if (i < p.N - 2 && p.x_str[i] < 0) xlo -= p.x_str[i] * (p.x_shape[i] - 1) * int64_t(sizeof(T));
+            for (int s = 0; s < 2; ++s)
+                if (p.pad[i][s] > 0 && side1d(p.side[i][s].tag) == kS1Const &&
+                    (p.side[i][s].value.re != 0 || p.side[i][s].value.im != 0 || p.side[i][s].value.i != 0))
+                    a.fills = 1;
+        }
+        a.ta[0].xlo += int32_t(xlo);
+    }
     a.nouter = 1;
     a.ktaps_outer = 1;
     for (int e = 0; e < a.No - 2; ++e) {
@@ -414,6 +522,8 @@ ndc_status launch_typed(const Plan& p, const void* x, const void* k, void* y, La
     a.gx = int(gcd64(a.s[ax], a.d[ax]));
     if (a.gy <= 0) a.gy = 1;
     if (a.gx <= 0) a.gx = 1;
+    // the sliding form needs consecutive outputs on consecutive staged columns
+    const bool slide = a.s[ax] == a.d[ax];
     // tile height: the largest unless, for 4-byte elements, 64-row tiles would
     // give under four workgroups per CU or waste over a tenth of the rows
     int ty = kMaxTileY<T>;
@@ -434,8 +544,10 @@ ndc_status launch_typed(const Plan& p, const void* x, const void* k, void* y, La
         // odd row stride: a wave's eight tile rows start on distinct LDS banks
         l.rx = (((kTileX - 1) * a.s[ax] + (kxc - 1) * a.d[ax]) / a.gx + 1) | 1;
         l.to = (l.ry * l.rx + E - 1) / E * E;
-        l.ks = (kxc + kCX<T> - 1) / kCX<T> * kCX<T>;
-        l.total = l.to + kyc * l.ks;
+        // one window of 8 where kernels of up to 8 columns take one
+        const int64_t cx = a.xbase && slide && a.K[ax] <= kCXSmall<T> ? kCXSmall<T> : kCX<T>;
+        l.ks = (kxc + cx - 1) / cx * cx;
+        l.total = l.to + kyc * l.ks + (a.xbase ? ((l.rx + l.ry + 1) * 4 + int64_t(sizeof(T)) - 1) / int64_t(sizeof(T)) : 0);
         return l;
     };
     int64_t kyc = a.K[ay], kxc = a.K[ax];
@@ -462,14 +574,12 @@ ndc_status launch_typed(const Plan& p, const void* x, const void* k, void* y, La
     a.nty = int((a.out[ay] + ty - 1) / ty);
     const int64_t nblocks = a.nouter * a.ntx * a.nty;
     if (nblocks <= 0) return NDC_OK;
-    if (nblocks > (int64_t(1) << 31) - 1) {
+    if (nblocks > (int64_t(1) << 31) - 1 || int64_t(a.ntx) * a.nty > (int64_t(1) << 31) - 1) {
         ctx.err = "direct convolution: output too large for one launch";
         return NDC_ERR_UNSUPPORTED;
     }
     ctx.kbegin("direct_conv", double(sizeof(T)) * double(p.x_numel + p.k_numel + p.y_numel),
                2.0 * double(p.y_numel) * double(p.k_numel));
-    // the sliding form needs consecutive outputs on consecutive staged columns
-    const bool slide = a.s[ax] == a.d[ax];
     if (ty == kMaxTileY<T>) {
         if (!launch_tile<T, kMaxTileY<T>>(ctx, slide, a, nblocks, smem)) return NDC_ERR_UNSUPPORTED;
     } else if constexpr (kMaxTileY<T> == 64) {
