@@ -112,6 +112,22 @@ bool axis_map(int64_t n, int64_t p0, int64_t p1, const ndc_border& front, const 
     return true;
 }
 
+// Whether axis_map succeeds, without the map: of a reflect fill's cells the
+// outermost one reads furthest (front cell 0 reads 2 p0, back cell P - 1 reads p1
+// cells before the last interior one).
+bool axis_fills(int64_t n, int64_t p0, int64_t p1, const ndc_border& front, const ndc_border& back, std::string* err) {
+    const int64_t P = n + p0 + p1;
+    if (front.tag == NDC_BORDER_REFLECT && p0 > 0 && 2 * p0 >= P) {
+        if (err) *err = "reflect front pad reads outside the padded axis (the reference panics)";
+        return false;
+    }
+    if (back.tag == NDC_BORDER_REFLECT && p1 > P - p1 - 1) {
+        if (err) *err = "reflect back pad reads outside the padded axis (the reference panics)";
+        return false;
+    }
+    return true;
+}
+
 void contiguous_strides(const int64_t* shape, int N, int64_t* str) {
     int64_t s = 1;
     for (int i = N - 1; i >= 0; --i) {
@@ -245,12 +261,18 @@ ndc_status make_plan(const ndc_conv_desc* d, int op, Plan* p, std::string* err, 
 
     auto maps = [&](bool fft) -> ndc_status {
         for (int i = 0; i < N; ++i) {
+            if (!build_maps) {
+                std::string e;
+                if (!axis_fills(P.x_shape[i], P.pad[i][0], P.pad[i][1], P.side[i][0], P.side[i][1], &e))
+                    return fail(NDC_ERR_INVALID_ARGUMENT, "axis " + std::to_string(i) + ": " + e);
+                continue;
+            }
             std::vector<int32_t> tmp;
             std::string e;
             const int64_t len = fft ? P.fft[i] : P.pds[i];
             if (!axis_map(P.x_shape[i], P.pad[i][0], P.pad[i][1], P.side[i][0], P.side[i][1], len, &tmp, &e))
                 return fail(NDC_ERR_INVALID_ARGUMENT, "axis " + std::to_string(i) + ": " + e);
-            if (build_maps) P.map[i].swap(tmp);
+            P.map[i].swap(tmp);
         }
         return NDC_OK;
     };

@@ -23,6 +23,7 @@ InvalidArgument.  Every computation runs in libndconv.so; there is no CPU
 fallback.
 """
 import ctypes
+import sys
 import threading
 
 import numpy as np
@@ -357,6 +358,7 @@ class FftProcessor:
         _check(lib.ndc_create(ctypes.byref(h)))
         self._h = h
         self._elem = None if elem is None else np.dtype(elem)
+        self._calls = {}   # prepared calls on GPU tensors (_prepared_call)
 
     def _transform(self, a, forward):
         lib = C.lib()
@@ -504,42 +506,109 @@ def fft_launch_plan(data_shape, kernel_shape, conv_mode, padding_mode=PaddingMod
 _ALGOS = {"auto": C.ALGO_AUTO, "direct": C.ALGO_DIRECT, "bf16": C.ALGO_MFMA_BF16, "bf16x3": C.ALGO_MFMA_BF16X3}
 
 
-def _run(op, data, kernel, conv_mode, padding_mode, processor=None, algo="auto"):
+def _value_key(v):
+    """A pad value by its exact contents; TypeError for kinds whose contents
+    are not known here (their calls are prepared every time)."""
+    if v is None or type(v) in (bool, int, float, complex):
+        return type(v), repr(v)
+    if isinstance(v, np.generic):
+        return v.dtype.str, v.tobytes()
+    raise TypeError
+
+
+def _mode_key(m):
+    return m.tag if m.padding is None else (m.tag, repr(m.padding), repr(m.strides))
+
+
+def _pad_key(p):
+    if p.borders is not None:
+        return p.tag, tuple([(b.tag, _value_key(b.value)) if isinstance(b, _BorderValue) else
+                             tuple([(v.tag, _value_key(v.value)) for v in b]) for b in p.borders])
+    return p.tag if p.value is None else (p.tag, _value_key(p.value))
+
+
+def _torch():
+    return sys.modules["torch"]   # a caller holding a tensor has imported it
+
+
+_raw_stream = None   # torch's current stream of a device index, as an integer
+
+
+def _current_stream(index):
+    global _raw_stream
+    if _raw_stream is None:
+        _raw_stream = getattr(_torch()._C, "_cuda_getCurrentRawStream", None) or \
+            (lambda i: _torch().cuda.current_stream(i).cuda_stream)
+    return _raw_stream(index)
+
+
+# Prepared calls one processor keeps: descriptors of 1.2 KB, dropped together
+# when they are more.
+_MAX_CALLS = 128
+
+
+def _prepared_call(proc, key, op, x, k, dilation, reverse_flag, conv_mode, padding_mode, algo):
+    """The descriptor and output shape of a call on GPU tensors, kept in the
+    processor under everything they depend on (element types, shapes, strides
+    and the values of the options): filling and checking a descriptor takes
+    the host longer than a small convolution takes the GPU."""
+    dtype = _NP_DTYPE[_np_dtype_of(x)]
+    d = C.ConvDesc()
+    _fill_desc(d, x, KernelWithDilation(k, dilation, reverse_flag), conv_mode, padding_mode, dtype, host=False)
+    d.algo = _ALGOS[algo]
+    info = C.PlanInfo()
+    _check(C.lib().ndc_plan(ctypes.byref(d), op, ctypes.byref(info)))
+    call = (d, ctypes.byref(d), tuple(int(info.out_shape[i]) for i in range(len(x.shape))))
+    if key is not None:
+        if len(proc._calls) >= _MAX_CALLS:
+            proc._calls.clear()
+        proc._calls[key] = call
+    return call
+
+
+def _run_gpu(op, x, k, dilation, reverse_flag, conv_mode, padding_mode, proc, algo):
     lib = C.lib()
+    if not (_is_torch(x) and _is_torch(k)) or not x.is_cuda or not k.is_cuda:
+        raise InvalidArgument("torch inputs must both be GPU tensors")
+    if x.dtype != k.dtype:
+        raise InvalidArgument("data and kernel dtypes differ")
+    try:
+        key = (op, algo, x.dtype, x.shape, x.stride(), k.shape, k.stride(), tuple(dilation), reverse_flag,
+               _mode_key(conv_mode), _pad_key(padding_mode))
+    except TypeError:
+        key = None
+    call = proc._calls.get(key) or _prepared_call(proc, key, op, x, k, dilation, reverse_flag, conv_mode, padding_mode,
+                                                  algo)
+    _, d, out_shape = call
+    h = proc.handle
+    y = _torch().empty(out_shape, dtype=x.dtype, device=x.device)
+    _check(lib.ndc_set_stream(h, _current_stream(x.device.index)), h)
+    _check((lib.ndc_conv if op == C.OP_CONV else lib.ndc_conv_fft)(h, d, x.data_ptr(), k.data_ptr(), y.data_ptr()), h)
+    return y
+
+
+def _run(op, data, kernel, conv_mode, padding_mode, processor=None, algo="auto"):
     kwd = _into_kwd(kernel)
     proc = processor or _default_processor()
-    torch_in = _is_torch(data) or _is_torch(kwd.kernel)
-    if torch_in:
-        import torch
-        if not (_is_torch(data) and _is_torch(kwd.kernel)) or not data.is_cuda or not kwd.kernel.is_cuda:
-            raise InvalidArgument("torch inputs must both be GPU tensors")
-        if data.dtype != kwd.kernel.dtype:
-            raise InvalidArgument("data and kernel dtypes differ")
-        x, k = data, kwd.kernel
-    else:
-        x = np.asarray(data)
-        k = np.asarray(kwd.kernel)
-        if x.dtype != k.dtype:
-            raise InvalidArgument("data and kernel dtypes differ")
+    if _is_torch(data) or _is_torch(kwd.kernel):
+        return _run_gpu(op, data, kwd.kernel, kwd.dilation, kwd.reverse_flag, conv_mode, padding_mode, proc, algo)
+    lib = C.lib()
+    x = np.asarray(data)
+    k = np.asarray(kwd.kernel)
+    if x.dtype != k.dtype:
+        raise InvalidArgument("data and kernel dtypes differ")
     dt = _np_dtype_of(x)
     if dt not in _NP_DTYPE:
         raise Unsupported(f"dtype {dt}")
-    dtype = _NP_DTYPE[dt]
     d = C.ConvDesc()
-    _fill_desc(d, x, KernelWithDilation(k, kwd.dilation, kwd.reverse_flag), conv_mode, padding_mode, dtype,
-               host=not torch_in)
+    _fill_desc(d, x, KernelWithDilation(k, kwd.dilation, kwd.reverse_flag), conv_mode, padding_mode, _NP_DTYPE[dt],
+               host=True)
     d.algo = _ALGOS[algo]
     info = C.PlanInfo()
     _check(lib.ndc_plan(ctypes.byref(d), op, ctypes.byref(info)))
     out_shape = tuple(int(info.out_shape[i]) for i in range(len(x.shape)))
     h = proc.handle
     fn = lib.ndc_conv if op == C.OP_CONV else lib.ndc_conv_fft
-    if torch_in:
-        y = torch.empty(out_shape, dtype=x.dtype, device=x.device)
-        _check(lib.ndc_set_stream(h, ctypes.c_void_p(torch.cuda.current_stream(x.device).cuda_stream)), h)
-        _check(fn(h, ctypes.byref(d), ctypes.c_void_p(x.data_ptr()), ctypes.c_void_p(k.data_ptr()),
-                  ctypes.c_void_p(y.data_ptr())), h)
-        return y
     y = np.empty(out_shape, dtype=dt)
     _check(lib.ndc_reset_stream(h), h)
     _check(fn(h, ctypes.byref(d), ctypes.c_void_p(x.ctypes.data), ctypes.c_void_p(k.ctypes.data),
@@ -615,10 +684,9 @@ class Baked:
         if (tuple(x.shape), tuple(x.stride() if self._torch else x.strides), _np_dtype_of(x)) != self._sig:
             raise InvalidArgument("data must have the shape, strides and dtype the kernel was baked for")
         if self._torch:
-            import torch
-            y = torch.empty(self.out_shape, dtype=x.dtype, device=x.device)
-            _check(lib.ndc_set_stream(h, ctypes.c_void_p(torch.cuda.current_stream(x.device).cuda_stream)), h)
-            _check(lib.ndc_conv_fft_with_baked(self._b, ctypes.c_void_p(x.data_ptr()), ctypes.c_void_p(y.data_ptr())), h)
+            y = _torch().empty(self.out_shape, dtype=x.dtype, device=x.device)
+            _check(lib.ndc_set_stream(h, _current_stream(x.device.index)), h)
+            _check(lib.ndc_conv_fft_with_baked(self._b, x.data_ptr(), y.data_ptr()), h)
             return y
         y = np.empty(self.out_shape, dtype=self._dt)
         _check(lib.ndc_reset_stream(h), h)
