@@ -23,7 +23,7 @@ LIB = os.path.join(LIBDIR, "libndconv.so")
 
 SOURCES = ["plan.cpp", "capi.cpp", "batch.cpp", "direct_conv.hip", "fft_conv.hip", "mfma_conv.hip",
            "batch_conv.hip", "noalloc.hip", "tile_plan.cpp", "tile_conv.hip", "tile_conv_f64.hip",
-           "matrix_conv.hip"]
+           "matrix_conv.hip", "batch_tile.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"

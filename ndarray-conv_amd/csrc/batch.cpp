@@ -53,23 +53,30 @@ struct DevMem {
 
 // Throughput costs (ms per item with the device full of workgroups).
 struct CostModel {
-    double fft_item[kBatchClasses];
     double dir_a, dir_b;     // FP32 direct item: dir_a + dir_b * outputs * taps
     double mfma_a, mfma_b;   // BF16x3 matrix-core item: mfma_a + mfma_b * K-blocks
     double mfma6_a, mfma6_b; // BF16x6 matrix-core item, likewise
+    double edge;             // a pair's first and last item more than one inside it
+    // tile runs: tile_a per run (the kernel's transform), tile_b per complex tile
+    double tile_a[kBatchTileClasses], tile_b[kBatchTileClasses];
     bool measured = false;
 };
 
 // Starting point before calibration, and what the calibration falls back to.
 CostModel default_costs() {
     CostModel c;
-    for (int i = 0; i < kBatchClasses; ++i) c.fft_item[i] = 1.2e-5;
+    const double b[kBatchTileClasses] = {4.3e-6, 1.7e-5, 4e-5, 2.9e-4};
+    for (int i = 0; i < kBatchTileClasses; ++i) {
+        c.tile_a[i] = 0.3 * b[i];
+        c.tile_b[i] = b[i];
+    }
     c.dir_a = 2e-6;
     c.dir_b = 6e-11;
     c.mfma_a = 4e-6;
     c.mfma_b = 4e-7;
     c.mfma6_a = 4e-6;
     c.mfma6_b = 8e-7;
+    c.edge = 1e-6;
     return c;
 }
 
@@ -83,26 +90,49 @@ int direct_tile(int s) {
     return std::min(kBatchDirectTile, std::max(cap, 1));
 }
 
-int64_t fft_per(int cls, int64_t kdil, int s) {
-    const int64_t L = 2 * int64_t(batch_lc(cls));
-    if (L < kdil) return 0;
-    return (L - kdil) / s + 1;
-}
-
 double direct_cost(const CostModel& cm, const PairShape& ps, int s) {
     const int64_t tile = direct_tile(s);
     const int64_t nt = (ps.out + tile - 1) / tile;
-    return double(nt) * cm.dir_a + cm.dir_b * double(ps.out) * double(ps.k);
+    return double(nt) * cm.dir_a + double(std::min<int64_t>(nt, 2)) * cm.edge + cm.dir_b * double(ps.out) * double(ps.k);
 }
 
-double fft_cost(const CostModel& cm, const PairShape& ps, int s, int cls) {
-    const int64_t per = fft_per(cls, ps.kdil, s);
-    if (per <= 0) return INFINITY;
-    const int64_t lines = (ps.out + per - 1) / per;
-    // one more line's worth (forward only) for the kernel spectrum
-    return (double(lines) + 0.5) / double(batch_lines(cls)) * cm.fft_item[cls];
+// Outputs per tile and phase, tiles per phase and complex tiles of a pair in
+// tile class c; none when the tile does not take it.
+struct TileSplit {
+    int64_t V = 0, per_phase = 0, total = 0;
+};
+TileSplit tile_split(const PairShape& ps, int d, int c) {
+    TileSplit r;
+    const int64_t N = int64_t(1) << batch_tile_log2(c), reach = ps.pds + int64_t(d) * N;
+    // at least an eighth of a tile is outputs; byte offsets of 30 bits, in the
+    // 64-bit class positions of 31
+    if (ps.k > N * 7 / 8 || reach >= (int64_t(1) << (c == kBatchTileFar ? 31 : 28))) return r;
+    r.V = N - ps.k + 1;
+    const int64_t U = ps.pds - ps.kdil + 1;
+    r.per_phase = ((U + d - 1) / d + r.V - 1) / r.V;
+    r.total = (r.per_phase * d + 1) / 2;
+    return r;
 }
 
+// Workgroups resident at once per CU: 5 of 256 threads (registers), 2 of 512, 1
+// of 1024.
+constexpr int tile_slots(int c) { return c == 0 ? 5 : c == 1 ? 2 : 1; }
+
+// Tiles of a run: long enough to share the kernel's transform, short enough
+// that the chip gets three rounds of runs (at most eight tiles, where the
+// kernel's share is small).
+int64_t run_tiles(int64_t total, int64_t slots) { return std::max<int64_t>(1, std::min<int64_t>(8, total / (3 * slots))); }
+
+// Tiles of a run that a pair's cost assumes before the batch's are known.
+constexpr int kRunTiles = 4;
+
+double tile_cost(const CostModel& cm, const PairShape& ps, int d, int c) {
+    const TileSplit t = tile_split(ps, d, c);
+    if (t.total <= 0) return INFINITY;
+    return cm.tile_b[c] * double(t.total) + cm.tile_a[c] * double((t.total + kRunTiles - 1) / kRunTiles);
+}
+
+constexpr int kMethodTile = -4;     // tile class 0; class c is kMethodTile - c
 constexpr int kMethodDirect = -1;   // FP32 direct items
 constexpr int kMethodMfma = -2;     // BF16x3 matrix-core items
 constexpr int kMethodMfma6 = -3;    // BF16x6 matrix-core items
@@ -128,159 +158,217 @@ double mfma_item_cost(const CostModel& cm, const PairShape& ps, bool six) {
 double mfma_cost(const CostModel& cm, const PairShape& ps, int s, bool six) {
     if (!mfma_eligible(ps, s)) return INFINITY;
     const int64_t nt = (ps.out + kBatchMfmaTile - 1) / kBatchMfmaTile;
-    return double(nt) * mfma_item_cost(cm, ps, six);
+    return double(nt) * mfma_item_cost(cm, ps, six) + double(std::min<int64_t>(nt, 2)) * cm.edge;
 }
 
-// Method per pair: kMethodDirect, kMethodMfma, kMethodMfma6, or an FFT class.
-int choose(const CostModel& cm, const PairShape& ps, int s, int algo, bool repeating_border) {
-    int best_cls = kMethodDirect;
+// The launch that computes a method's pairs: a tile class's, or the queue's.
+int group_of(int method) { return method <= kMethodTile ? kMethodTile - method : kBatchTileClasses; }
+
+// What every pair of a batch shares, and the chip's size.
+struct BatchForm {
+    int s, d;
+    int32_t front, back;   // side tags of border1d.hpp
+    int cus, blocks;       // CUs, resident workgroups of the queue's kernel
+};
+
+// Method of a pair in the queue: kMethodDirect, kMethodMfma or kMethodMfma6.
+int queue_method(const CostModel& cm, const PairShape& ps, int s, int algo, bool repeating_border) {
+    const bool x3 = bf16x3_admitted(ps, repeating_border);
+    if (algo == NDC_BATCH_MFMA && mfma_eligible(ps, s)) return x3 ? kMethodMfma : kMethodMfma6;
+    if (algo == NDC_BATCH_BF16X6 && mfma_eligible(ps, s)) return kMethodMfma6;
+    if (algo == NDC_BATCH_AUTO_BF16X3 && mfma_cost(cm, ps, s, !x3) < direct_cost(cm, ps, s))
+        return x3 ? kMethodMfma : kMethodMfma6;
+    return kMethodDirect;
+}
+
+// Methods of all pairs: a tile class or the queue's method, whichever costs
+// less among the launches that the batch uses.  The costs are those of a full
+// chip; a launch takes about one run or item longer than its work, on a chip
+// that is part empty, so all choices of launches are compared with that added:
+// a few pairs of some length do not get a launch of their own, and a small
+// batch is one launch (509 pairs, 6.3 M outputs: 20 us in one launch of 1024-point
+// tiles, 29 us with 6 pairs in a launch of 4096-point tiles beside it; 4096 pairs, 153 M
+// outputs: 359 to 374 us in one launch of the queue, 386 to 412 us where the
+// short and the long kernels went to tiles).
+std::vector<int> choose(const CostModel& cm, const std::vector<PairShape>& sh, const BatchForm& f, int algo,
+                        bool repeating_border) {
+    constexpr int Q = kBatchTileClasses, G = Q + 1;
+    constexpr double kLaunchMs = 3e-3;
+    const size_t P = sh.size();
+    std::vector<int> m(P), queue(P);
+    std::vector<std::array<double, G>> cost(P);
+    std::vector<std::array<int64_t, Q>> split(P);
+    const bool tiles = algo == NDC_BATCH_AUTO || algo == NDC_BATCH_AUTO_BF16X3 || algo == NDC_BATCH_FFT;
+    std::vector<double> item(P);
+    for (size_t i = 0; i < P; ++i) {
+        const PairShape& ps = sh[i];
+        queue[i] = m[i] = queue_method(cm, ps, f.s, algo, repeating_border);
+        bool any = false;
+        for (int c = 0; c < Q; ++c) {
+            // where the queue's method is a fixed one, tiles take what it does not
+            const bool ok = tiles || (algo != NDC_BATCH_DIRECT && queue[i] == kMethodDirect);
+            split[i][c] = tile_split(ps, f.d, c).total;
+            cost[i][c] = ok ? tile_cost(cm, ps, f.d, c) : INFINITY;
+            any = any || !std::isinf(cost[i][c]);
+        }
+        const bool direct = queue[i] == kMethodDirect, six = queue[i] == kMethodMfma6;
+        cost[i][Q] = algo == NDC_BATCH_FFT && any ? INFINITY
+                     : direct                     ? direct_cost(cm, ps, f.s)
+                                                  : mfma_cost(cm, ps, f.s, six);
+        item[i] = direct ? cm.dir_a + cm.dir_b * double(std::min<int64_t>(direct_tile(f.s), ps.out)) * double(ps.k)
+                         : mfma_item_cost(cm, ps, six);
+    }
     double best = INFINITY;
-    for (int c = 0; c < kBatchClasses; ++c) {
-        const double v = fft_cost(cm, ps, s, c);
-        if (v < best) {
-            best = v;
-            best_cls = c;
+    unsigned best_mask = 0;
+    auto pick = [&](size_t i, unsigned mask) {
+        int g = -1;
+        for (int c = 0; c < G; ++c)
+            if ((mask >> c & 1) && !std::isinf(cost[i][c]) && (g < 0 || cost[i][c] < cost[i][g])) g = c;
+        return g;
+    };
+    std::vector<int> group(P);
+    for (unsigned mask = 1; mask < (1u << G); ++mask) {
+        double work = 0, longest = 0;
+        int64_t total[Q] = {}, runs[Q] = {}, run[Q] = {};
+        unsigned used = 0;
+        bool all = true;
+        for (size_t i = 0; i < P && all; ++i) {
+            group[i] = sh[i].out > 0 ? pick(i, mask) : G;
+            const int g = group[i];
+            if (g == G) continue;
+            all = g >= 0;
+            if (!all) break;
+            used |= 1u << g;
+            if (g == Q) {
+                work += cost[i][Q];
+                longest = std::max(longest, item[i]);
+            } else {
+                total[g] += split[i][g];
+            }
+        }
+        if (!all || used != mask) continue;
+        for (int c = 0; c < Q; ++c) run[c] = run_tiles(total[c], int64_t(f.cus) * tile_slots(c));
+        for (size_t i = 0; i < P; ++i)
+            if (group[i] < Q) runs[group[i]] += (split[i][group[i]] + run[group[i]] - 1) / run[group[i]];
+        for (int c = 0; c < Q; ++c)
+            if (used >> c & 1)
+                work += cm.tile_a[c] * double(runs[c]) + cm.tile_b[c] * double(total[c]) + kLaunchMs +
+                        (cm.tile_a[c] + cm.tile_b[c] * double(run[c])) * double(f.cus * tile_slots(c));
+        if (used >> Q & 1) work += kLaunchMs + longest * double(f.blocks);
+        if (work < best) {
+            best = work;
+            best_mask = mask;
         }
     }
-    if (algo == NDC_BATCH_DIRECT) return kMethodDirect;
-    if (algo == NDC_BATCH_FFT) return best_cls;   // direct when no class holds the dilated kernel
-    if (algo == NDC_BATCH_MFMA && mfma_eligible(ps, s))
-        return bf16x3_admitted(ps, repeating_border) ? kMethodMfma : kMethodMfma6;
-    if (algo == NDC_BATCH_BF16X6 && mfma_eligible(ps, s)) return kMethodMfma6;
-    const double vd = direct_cost(cm, ps, s);
-    int pick = vd <= best ? kMethodDirect : best_cls;
-    if (algo == NDC_BATCH_AUTO_BF16X3) {
-        const bool x3 = bf16x3_admitted(ps, repeating_border);
-        const double vm = mfma_cost(cm, ps, s, !x3);
-        if (vm < std::min(best, vd)) pick = x3 ? kMethodMfma : kMethodMfma6;
+    for (size_t i = 0; i < P; ++i) {
+        const int g = sh[i].out > 0 ? pick(i, best_mask) : Q;
+        m[i] = g == Q ? queue[i] : kMethodTile - g;
     }
-    return pick;
+    return m;
 }
 
 struct Schedule {
-    std::vector<BatchPair> pairs;
     std::vector<BatchItem> items;
-    std::vector<BatchLine> lines;
-    std::vector<int32_t> kpairs;
-    std::vector<BatchKItem> kitems;
-    int64_t ks_total = 0;
-    int32_t nfirst = 0;            // direct and FFT items, ahead of the matrix-core items
+    std::vector<BatchTile> tiles[kBatchTileClasses];   // longest runs first
+    double tile_bytes[kBatchTileClasses] = {};
+    int64_t ntiles = 0;            // complex tiles
+    int32_t nfirst = 0;            // direct items, ahead of the matrix-core items
     double est_ms = 0;
-    double kspec_bytes = 0, main_bytes = 0, main_flops = 0;
+    double main_bytes = 0, main_flops = 0;
 };
 
-// Builds the work queue.  offs[i] = {x, k, y} element offsets of pair i.
+// Tile runs of class c; max_run > 0 gives their length.
+void build_tiles(Schedule& S, const std::vector<PairShape>& sh, const std::vector<std::array<int64_t, 3>>& offs,
+                 const std::vector<int>& method, const BatchForm& f, int c, const CostModel& cm, int64_t max_run) {
+    std::vector<size_t> pairs;
+    std::vector<TileSplit> split;
+    int64_t total = 0;
+    for (size_t i = 0; i < sh.size(); ++i) {
+        if (method[i] != kMethodTile - c || sh[i].out <= 0) continue;
+        pairs.push_back(i);
+        split.push_back(tile_split(sh[i], f.d, c));
+        total += split.back().total;
+    }
+    if (pairs.empty()) return;
+    S.ntiles += total;
+    const int64_t slots = int64_t(f.cus) * tile_slots(c);
+    const int64_t run = max_run > 0 ? max_run : run_tiles(total, slots);
+    for (size_t j = 0; j < pairs.size(); ++j) {
+        const PairShape& ps = sh[pairs[j]];
+        const auto& o = offs[pairs[j]];
+        S.tile_bytes[c] += 4.0 * double(ps.n + ps.k + ps.out);
+        const TileSplit& t = split[j];
+        const int64_t p1 = ps.pds - ps.n - ps.p0;
+        auto wraps = [&](int32_t side, int64_t pad) {
+            return side == kS1Reflect ? pad > ps.n - 1 : side == kS1Circular ? pad > ps.n : false;
+        };
+        const int64_t runs = (t.total + run - 1) / run;   // of equal length, none longer than `run`
+        for (int64_t r = 0; r < runs; ++r) {
+            const int64_t b = t.total * r / runs, e = t.total * (r + 1) / runs;
+            BatchTile it{};
+            it.x_off = o[0];
+            it.k_off = o[1];
+            it.y_off = o[2];
+            it.n = int32_t(ps.n);
+            it.k = int32_t(ps.k);
+            it.p0 = int32_t(ps.p0);
+            it.pds = int32_t(ps.pds);
+            it.out = int32_t(ps.out);
+            it.V = int32_t(t.V);
+            it.tiles = int32_t(t.per_phase);
+            it.first = int32_t(b);
+            it.count = int32_t(e - b);
+            it.wraps = wraps(f.front, ps.p0) || wraps(f.back, p1);
+            S.tiles[c].push_back(it);
+            S.est_ms += cm.tile_a[c] + cm.tile_b[c] * double(e - b);
+        }
+    }
+    std::stable_sort(S.tiles[c].begin(), S.tiles[c].end(),
+                     [](const BatchTile& a, const BatchTile& b) { return a.count > b.count; });
+}
+
+// Builds the tile runs and the work queue.  offs[i] = {x, k, y} element offsets
+// of pair i.
 Schedule build_schedule(const std::vector<PairShape>& sh, const std::vector<std::array<int64_t, 3>>& offs,
-                        const std::vector<int>& method, int s, const CostModel& cm) {
+                        const std::vector<int>& method, const BatchForm& f, const CostModel& cm, int64_t max_run = 0) {
     Schedule S;
-    const size_t P = sh.size();
-    S.pairs.resize(P);
-    std::vector<std::vector<BatchLine>> cls_lines(kBatchClasses);
-    std::vector<std::vector<int32_t>> cls_kpairs(kBatchClasses);
+    for (int c = 0; c < kBatchTileClasses; ++c) build_tiles(S, sh, offs, method, f, c, cm, max_run);
     std::vector<std::pair<double, BatchItem>> work;
-    const int tile = direct_tile(s);
-    // a direct or matrix-core tile record with its pair's metadata
-    auto tile_item = [&](int kind, size_t i, int64_t o, int cnt) {
+    const int tile = direct_tile(f.s);
+    for (size_t i = 0; i < sh.size(); ++i) {
         const PairShape& ps = sh[i];
-        BatchItem it{};
-        it.kind = kind;
-        it.a = int32_t(i);
-        it.b = int32_t(o);
-        it.c = cnt;
-        it.x_off = offs[i][0];
-        it.k_off = offs[i][1];
-        it.y_off = offs[i][2];
-        it.n = int32_t(ps.n);
-        it.k = int32_t(ps.k);
-        it.p0 = int32_t(ps.p0);
-        it.pds = int32_t(ps.pds);
-        return it;
-    };
-    for (size_t i = 0; i < P; ++i) {
-        const PairShape& ps = sh[i];
-        BatchPair& bp = S.pairs[i];
-        bp.x_off = offs[i][0];
-        bp.k_off = offs[i][1];
-        bp.y_off = offs[i][2];
-        bp.n = int32_t(ps.n);
-        bp.k = int32_t(ps.k);
-        bp.p0 = int32_t(ps.p0);
-        bp.pds = int32_t(ps.pds);
-        bp.out = int32_t(ps.out);
-        bp.cls = method[i];
-        bp.ks_off = 0;
-        bp.per = 0;
+        if (method[i] <= kMethodTile) continue;
         S.main_bytes += 4.0 * double(ps.n + ps.out);
         if (ps.out <= 0) continue;
-        if (method[i] == kMethodDirect) {
-            S.main_bytes += 4.0 * double(ps.k);
-            S.main_flops += 2.0 * double(ps.out) * double(ps.k);
-            for (int64_t o = 0; o < ps.out; o += tile) {
-                const int cnt = int(std::min<int64_t>(tile, ps.out - o));
-                work.emplace_back(cm.dir_a + cm.dir_b * double(cnt) * double(ps.k), tile_item(0, i, o, cnt));
-            }
-        } else if (method[i] == kMethodMfma || method[i] == kMethodMfma6) {
-            const bool six = method[i] == kMethodMfma6;
-            S.main_bytes += 4.0 * double(ps.k);
-            S.main_flops += 2.0 * double(ps.out) * double(ps.k);
-            const double c = mfma_item_cost(cm, ps, six);
-            const int kind = six ? kBatchKindMfma6 : kBatchKindMfma;
-            for (int64_t o = 0; o < ps.out; o += kBatchMfmaTile) {
-                const int cnt = int(std::min<int64_t>(kBatchMfmaTile, ps.out - o));
-                work.emplace_back(c, tile_item(kind, i, o, cnt));
-            }
-        } else {
-            const int c = method[i];
-            const int LC = batch_lc(c);
-            bp.per = int32_t(fft_per(c, ps.kdil, s));
-            bp.ks_off = S.ks_total;
-            S.ks_total += LC + 1;
-            cls_kpairs[c].push_back(int32_t(i));
-            S.kspec_bytes += 4.0 * double(ps.k) + 8.0 * double(LC + 1);
-            S.main_bytes += 8.0 * double(LC + 1);   // the kernel spectrum, read once (its blocks share it in cache)
-            for (int64_t o = 0; o < ps.out; o += bp.per) {
-                BatchLine ln{};
-                ln.x_off = bp.x_off;
-                ln.y_off = bp.y_off;
-                ln.ks_off = bp.ks_off;
-                ln.n = bp.n;
-                ln.k = bp.k;
-                ln.p0 = bp.p0;
-                ln.pds = bp.pds;
-                ln.out = bp.out;
-                ln.per = bp.per;
-                ln.o0 = int32_t(o);
-                ln.pair = int32_t(i);
-                cls_lines[c].push_back(ln);
-            }
+        S.main_bytes += 4.0 * double(ps.k);
+        S.main_flops += 2.0 * double(ps.out) * double(ps.k);
+        const bool direct = method[i] == kMethodDirect, six = method[i] == kMethodMfma6;
+        const int64_t step = direct ? tile : kBatchMfmaTile;
+        for (int64_t o = 0; o < ps.out; o += step) {
+            BatchItem it{};   // the tile with its pair's metadata
+            it.kind = direct ? 0 : six ? kBatchKindMfma6 : kBatchKindMfma;
+            it.a = int32_t(i);
+            it.b = int32_t(o);
+            it.c = int32_t(std::min<int64_t>(step, ps.out - o));
+            it.x_off = offs[i][0];
+            it.k_off = offs[i][1];
+            it.y_off = offs[i][2];
+            it.n = int32_t(ps.n);
+            it.k = int32_t(ps.k);
+            it.p0 = int32_t(ps.p0);
+            it.pds = int32_t(ps.pds);
+            work.emplace_back(direct ? cm.dir_a + cm.dir_b * double(it.c) * double(ps.k) : mfma_item_cost(cm, ps, six), it);
         }
-    }
-    for (int c = 0; c < kBatchClasses; ++c) {
-        const int G = batch_lines(c);
-        const int32_t base = int32_t(S.lines.size());
-        const int32_t nl = int32_t(cls_lines[c].size());
-        S.lines.insert(S.lines.end(), cls_lines[c].begin(), cls_lines[c].end());
-        for (int32_t f = 0; f < nl; f += G) {
-            BatchItem it{};
-            it.kind = 1 + c;
-            it.a = base + f;
-            it.b = std::min(G, nl - f);
-            work.emplace_back(cm.fft_item[c], it);
-        }
-        const int32_t kb = int32_t(S.kpairs.size());
-        const int32_t nk = int32_t(cls_kpairs[c].size());
-        S.kpairs.insert(S.kpairs.end(), cls_kpairs[c].begin(), cls_kpairs[c].end());
-        for (int32_t f = 0; f < nk; f += G) S.kitems.push_back(BatchKItem{c, kb + f, std::min(G, nk - f), 0});
     }
     // longest items first: the queue hands them out in this order, so the
-    // tail of the launch is made of the shortest items.  The direct and FFT
-    // items form the first range, the matrix-core items the second.
+    // tail of the launch is made of the shortest items.  The direct items form
+    // the first range, the matrix-core items the second.
     std::stable_sort(work.begin(), work.end(),
                      [](const std::pair<double, BatchItem>& a, const std::pair<double, BatchItem>& b) {
                          return a.first > b.first;
                      });
     const auto first_end = std::stable_partition(work.begin(), work.end(), [](const std::pair<double, BatchItem>& w) {
-        return w.second.kind != kBatchKindMfma && w.second.kind != kBatchKindMfma6;
+        return w.second.kind == 0;
     });
     S.nfirst = int32_t(first_end - work.begin());
     S.items.reserve(work.size());
@@ -293,8 +381,9 @@ Schedule build_schedule(const std::vector<PairShape>& sh, const std::vector<std:
 
 // Device-resident copy of a schedule plus the launch arguments.
 struct DevSchedule {
-    DevMem pairs, items, lines, klines, kitems, kspec, counter, consts;
+    DevMem items, counter, consts, tiles[kBatchTileClasses];
     BatchArgs args{};
+    BatchTileLaunch tl{};
     int grid = 0;
     // Border sides of every pair, and the constant cells the kernels read for
     // pad positions that hold a constant.
@@ -308,49 +397,33 @@ struct DevSchedule {
         args.cback = cback;
         return true;
     }
-    bool upload(const Schedule& S, const float2* tw, int blocks) {
-        std::vector<BatchKLine> kl(S.kpairs.size());
-        for (size_t i = 0; i < kl.size(); ++i) {
-            const BatchPair& p = S.pairs[size_t(S.kpairs[i])];
-            kl[i] = BatchKLine{p.k_off, p.ks_off, p.k, 0};
-        }
-        if (!pairs.upload(S.pairs.data(), S.pairs.size() * sizeof(BatchPair)) ||
-            !items.upload(S.items.data(), S.items.size() * sizeof(BatchItem)) ||
-            !lines.upload(S.lines.data(), S.lines.size() * sizeof(BatchLine)) ||
-            !klines.upload(kl.data(), kl.size() * sizeof(BatchKLine)) ||
-            !kitems.upload(S.kitems.data(), S.kitems.size() * sizeof(BatchKItem)) ||
-            !kspec.ensure(size_t(S.ks_total) * sizeof(float2)) || !counter.ensure(size_t(kBatchHeads) * kBatchQueueStride * sizeof(int32_t)))
+    bool upload(const Schedule& S, LaunchContext& ctx, int blocks) {
+        if (!items.upload(S.items.data(), S.items.size() * sizeof(BatchItem)) ||
+            !counter.ensure(size_t(kBatchHeads) * kBatchQueueStride * sizeof(int32_t)) || !batch_tile_tables(ctx, tl.tw))
             return false;
-        args.pairs = static_cast<const BatchPair*>(pairs.p);
         args.items = static_cast<const BatchItem*>(items.p);
-        args.lines = static_cast<const BatchLine*>(lines.p);
-        args.klines = static_cast<const BatchKLine*>(klines.p);
-        args.kitems = static_cast<const BatchKItem*>(kitems.p);
-        args.kspec = static_cast<float2*>(kspec.p);
         args.counter = static_cast<int32_t*>(counter.p);
-        args.tw = tw;
         args.nitems = int32_t(S.items.size());
         args.nfirst = S.nfirst;
-        args.nkitems = int32_t(S.kitems.size());
+        for (int c = 0; c < kBatchTileClasses; ++c) {
+            if (!tiles[c].upload(S.tiles[c].data(), S.tiles[c].size() * sizeof(BatchTile))) return false;
+            tl.items[c] = static_cast<const BatchTile*>(tiles[c].p);
+            tl.n[c] = int32_t(S.tiles[c].size());
+            tl.bytes[c] = S.tile_bytes[c];
+        }
         grid = int(std::min<int64_t>(int64_t(S.items.size()), int64_t(blocks)));
         return true;
     }
 };
 
-// Quarter-circle tables W_L^r (r < L/4, L = 2 LC) of every class, FP64 on the
-// host, concatenated at batch_tw_offset(c).
-const float2* batch_twiddles(LaunchContext& ctx) {
-    std::vector<float> tab;
-    for (int c = 0; c < kBatchClasses; ++c) {
-        const int LC = batch_lc(c);
-        const double L = 2.0 * LC;
-        for (int r = 0; r < LC / 2; ++r) {
-            const double ang = -2.0 * M_PI * double(r) / L;
-            tab.push_back(float(std::cos(ang)));
-            tab.push_back(float(std::sin(ang)));
-        }
-    }
-    return static_cast<const float2*>(ctx.constant_table("batch_tw", tab.data(), tab.size() * sizeof(float)));
+// The launches of a schedule: the tile runs, which zero the queue's heads, then
+// the queue.
+ndc_status launch_all(const DevSchedule& D, LaunchContext& ctx, hipStream_t st, bool profile, double main_bytes,
+                      double main_flops) {
+    bool runs = false;
+    for (const int32_t n : D.tl.n) runs = runs || n > 0;
+    const ndc_status r = launch_batch_tiles(D.args, D.tl, ctx, st, profile);
+    return r != NDC_OK ? r : launch_batch(D.args, D.grid, !runs, ctx, st, profile, main_bytes, main_flops);
 }
 
 int resident_blocks(LaunchContext& ctx) { return batch_blocks_per_cu() * ctx.cu_count(); }
@@ -359,8 +432,7 @@ int resident_blocks(LaunchContext& ctx) { return batch_blocks_per_cu() * ctx.cu_
 bool time_schedule(LaunchContext& ctx, const Schedule& S, const float* x, const float* k, float* y, int s, int d,
                    double* ms) {
     DevSchedule D;
-    const float2* tw = batch_twiddles(ctx);
-    if (!tw || !D.upload(S, tw, resident_blocks(ctx))) return false;
+    if (!D.upload(S, ctx, resident_blocks(ctx))) return false;
     D.args.x = x;
     D.args.k = k;
     D.args.y = y;
@@ -372,10 +444,10 @@ bool time_schedule(LaunchContext& ctx, const Schedule& S, const float* x, const 
     hipStream_t st = ctx.stream();
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) return false;
-    bool ok = launch_batch(D.args, D.grid, ctx, st, false, 0, 0, 0) == NDC_OK;
+    bool ok = launch_all(D, ctx, st, false, 0, 0) == NDC_OK;
     constexpr int reps = 3;
     ok = ok && hipEventRecord(e0, st) == hipSuccess;
-    for (int r = 0; ok && r < reps; ++r) ok = launch_batch(D.args, D.grid, ctx, st, false, 0, 0, 0) == NDC_OK;
+    for (int r = 0; ok && r < reps; ++r) ok = launch_all(D, ctx, st, false, 0, 0) == NDC_OK;
     ok = ok && hipEventRecord(e1, st) == hipSuccess && hipEventSynchronize(e1) == hipSuccess;
     float t = 0;
     ok = ok && hipEventElapsedTime(&t, e0, e1) == hipSuccess;
@@ -385,79 +457,85 @@ bool time_schedule(LaunchContext& ctx, const Schedule& S, const float* x, const 
     return ok;
 }
 
-// Measures the cost model on the device: synthetic batches of 96 signals of
-// 2^18 samples, one method each (every FFT class; direct at two tap counts).
+// Measures the cost model on the device, on random samples (zeros would let
+// the matrix cores run at clocks that data does not), one method at a time.
+// The batches read and write 25 M samples four times over, which takes long
+// enough that what a launch costs by itself is a few percent.
 bool calibrate(LaunchContext& ctx, int s, int d, CostModel* cm) {
-    constexpr int P = 96;
-    constexpr int64_t N = 1 << 18;
-    float* x = static_cast<float*>(ctx.scratch(0, size_t(P) * N * sizeof(float)));
-    float* y = static_cast<float*>(ctx.scratch(1, size_t(P) * N * sizeof(float)));
-    float* k = static_cast<float*>(ctx.scratch(2, size_t(P) * 1024 * sizeof(float)));
+    constexpr int64_t kSamples = 96 << 18, kTaps = 1024, kTimes = 4;
+    float* x = static_cast<float*>(ctx.scratch(0, size_t(kSamples) * sizeof(float)));
+    float* y = static_cast<float*>(ctx.scratch(1, size_t(kSamples) * sizeof(float)));
+    float* k = static_cast<float*>(ctx.scratch(2, size_t(kTaps) * sizeof(float)));
     if (!x || !y || !k) return false;
-    if (hipMemsetAsync(x, 0, size_t(P) * N * sizeof(float), ctx.stream()) != hipSuccess ||
-        hipMemsetAsync(k, 0, size_t(P) * 1024 * sizeof(float), ctx.stream()) != hipSuccess)
-        return false;
-    auto shapes = [&](int64_t kl) {
+    if (fill_random(x, kSamples, ctx) != NDC_OK || fill_random(k, kTaps, ctx) != NDC_OK) return false;
+    const BatchForm form{s, d, kS1Circular, kS1Circular, ctx.cu_count(), resident_blocks(ctx)};
+    CostModel out = *cm;
+    struct Unit {
+        double ms = 0;       // per tile of a run, or per item
+        double runs = 0;     // runs per tile
+        double work = 0;     // outputs times taps per item
+        double blocks = 0;   // K-blocks of an item
+    };
+    // pairs of n samples and kl taps, all by `method`
+    auto measure = [&](int64_t n, int64_t kl, int method, int64_t run, Unit* u) {
+        const int64_t distinct = kSamples / n;
+        const size_t P = size_t(distinct * kTimes);
         std::vector<PairShape> sh(P);
         std::vector<std::array<int64_t, 3>> offs(P);
-        for (int i = 0; i < P; ++i) {
-            const int64_t kdil = (kl - 1) * d + 1;
-            const int64_t p0 = (kdil - 1) / 2 + ((kdil - 1) % 2), p1 = (kdil - 1) / 2;   // Same
-            const int64_t pds = N + p0 + p1;
-            sh[i] = PairShape{N, kl, p0, pds, (pds - kdil) / s + 1, kdil};
-            offs[i] = {i * N, i * 1024, i * N};
+        const int64_t kdil = (kl - 1) * d + 1;
+        const int64_t p0 = (kdil - 1) / 2 + ((kdil - 1) % 2), p1 = (kdil - 1) / 2;   // Same
+        for (size_t i = 0; i < P; ++i) {
+            sh[i] = PairShape{n, kl, p0, n + p0 + p1, (n + p0 + p1 - kdil) / s + 1, kdil};
+            offs[i] = {int64_t(i) % distinct * n, 0, int64_t(i) % distinct * n};
         }
-        return std::make_pair(sh, offs);
+        const Schedule S = build_schedule(sh, offs, std::vector<int>(P, method), form, out, run);
+        const int c = group_of(method);
+        const double units = c < kBatchTileClasses ? double(S.ntiles) : double(S.items.size());
+        double t = 0;
+        if (units == 0 || !time_schedule(ctx, S, x, k, y, s, d, &t)) return false;
+        u->ms = t / units;
+        u->runs = c < kBatchTileClasses ? double(S.tiles[c].size()) / units : 0;
+        u->work = double(P) * double(sh[0].out) * double(kl) / units;
+        u->blocks = double(mfma_nkb(sh[0]));
+        return true;
     };
-    CostModel out = *cm;
-    for (int c = 0; c < kBatchClasses; ++c) {
-        const int64_t kl = std::max<int64_t>(1, std::min<int64_t>(33, (2 * batch_lc(c) - 1) / (2 * d) + 1));
-        auto so = shapes(kl);
-        std::vector<int> method(P, c);
-        Schedule S = build_schedule(so.first, so.second, method, s, out);
-        double ms = 0;
-        if (!time_schedule(ctx, S, x, k, y, s, d, &ms) || S.items.empty()) return false;
-        out.fft_item[c] = ms / double(S.items.size());
+    constexpr int64_t kLong = 1 << 18;
+    // tile runs: a + b at pairs of one complex tile (their edges are part of a),
+    // b + a / 8 inside long pairs
+    for (int c = 0; c < kBatchTileClasses; ++c) {
+        const int64_t N = int64_t(1) << batch_tile_log2(c), kl = 33;
+        if (int64_t(d) * N >= kLong / 2) continue;
+        Unit one, many;
+        if (!measure(2 * (N - kl + 1) * d, kl, kMethodTile - c, 1, &one) || !measure(kLong, kl, kMethodTile - c, 8, &many))
+            return false;
+        if (many.runs >= 1) continue;
+        out.tile_a[c] = std::max(0.0, (one.ms - many.ms) / (1 - many.runs));
+        out.tile_b[c] = std::max(1e-9, many.ms - out.tile_a[c] * many.runs);
     }
-    double t[2] = {0, 0}, work[2] = {0, 0}, nitems[2] = {0, 0};
-    const int64_t taps[2] = {16, 256};
-    for (int j = 0; j < 2; ++j) {
-        auto so = shapes(taps[j]);
-        std::vector<int> method(P, -1);
-        Schedule S = build_schedule(so.first, so.second, method, s, out);
-        if (!time_schedule(ctx, S, x, k, y, s, d, &t[j])) return false;
-        nitems[j] = double(S.items.size());
-        for (auto& ps : so.first) work[j] += double(ps.out) * double(ps.k);
+    // direct items: a + b work, from two tap counts
+    Unit u[2];
+    if (!measure(kLong, 16, kMethodDirect, 0, &u[0]) || !measure(kLong, 256, kMethodDirect, 0, &u[1])) return false;
+    if (u[1].work > u[0].work) {
+        out.dir_b = std::max(1e-14, (u[1].ms - u[0].ms) / (u[1].work - u[0].work));
+        out.dir_a = std::max(0.0, u[0].ms - out.dir_b * u[0].work);
     }
-    // t = nitems a + work b, from the two measurements
-    const double det = nitems[0] * work[1] - nitems[1] * work[0];
-    if (det != 0) {
-        out.dir_b = std::max(1e-14, (nitems[0] * t[1] - nitems[1] * t[0]) / det);
-        out.dir_a = std::max(0.0, (t[0] - work[0] * out.dir_b) / nitems[0]);
-    }
-    // matrix-core items (stride 1 only): t = nitems (a + b nkb) at two kernel
-    // lengths, for each split
+    // matrix-core items (stride 1 only): a + b K-blocks at two kernel lengths,
+    // for each split; and what the first and last of a pair cost more
     if (s == 1) {
         const int64_t kcap = (kBatchMfmaMaxKdil - 1) / d + 1;
-        const int64_t mt[2] = {std::min<int64_t>(8, kcap), std::min<int64_t>(512, kcap)};
         for (int six = 0; six < 2; ++six) {
-            double tm[2] = {0, 0}, nm[2] = {0, 0}, kbm[2] = {0, 0};
-            for (int j = 0; j < 2; ++j) {
-                auto so = shapes(mt[j]);
-                std::vector<int> method(P, six ? kMethodMfma6 : kMethodMfma);
-                Schedule S = build_schedule(so.first, so.second, method, s, out);
-                if (!time_schedule(ctx, S, x, k, y, s, d, &tm[j]) || S.items.empty()) return false;
-                nm[j] = double(S.items.size());
-                kbm[j] = double(mfma_nkb(so.first[0]));
-            }
-            const double pi0 = tm[0] / nm[0], pi1 = tm[1] / nm[1];   // ms per item
-            if (kbm[1] > kbm[0]) {
-                const double b = std::max(1e-12, (pi1 - pi0) / (kbm[1] - kbm[0]));
-                const double a = std::max(0.0, pi0 - b * kbm[0]);
+            const int method = six ? kMethodMfma6 : kMethodMfma;
+            if (!measure(kLong, std::min<int64_t>(8, kcap), method, 0, &u[0]) ||
+                !measure(kLong, std::min<int64_t>(512, kcap), method, 0, &u[1]))
+                return false;
+            if (u[1].blocks > u[0].blocks) {
+                const double b = std::max(1e-12, (u[1].ms - u[0].ms) / (u[1].blocks - u[0].blocks));
                 (six ? out.mfma6_b : out.mfma_b) = b;
-                (six ? out.mfma6_a : out.mfma_a) = a;
+                (six ? out.mfma6_a : out.mfma_a) = std::max(0.0, u[0].ms - b * u[0].blocks);
             }
         }
+        if (!measure(2 * kBatchMfmaTile, std::min<int64_t>(8, kcap), kMethodMfma6, 0, &u[1])) return false;
+        out.edge = std::max(0.0, u[1].ms - out.mfma6_a - out.mfma6_b * u[1].blocks);
     }
     out.measured = true;
     *cm = out;
@@ -466,7 +544,7 @@ bool calibrate(LaunchContext& ctx, int s, int d, CostModel* cm) {
 
 // The cost model of this handle for strides/dilation (s, d), measured once.
 CostModel cost_model(LaunchContext& ctx, int s, int d, bool measure) {
-    const std::string key = "batch_costs3:" + std::to_string(s) + ":" + std::to_string(d);
+    const std::string key = "batch_costs4:" + std::to_string(s) + ":" + std::to_string(d);
     std::string& m = ctx.memo(key);
     CostModel cm = default_costs();
     if (m.size() == sizeof(CostModel)) {
@@ -536,7 +614,7 @@ struct Batch {
         a.k = k;
         a.y = y;
         D.args = a;
-        return launch_batch(a, D.grid, *ctx, st, profile, S.kspec_bytes, S.main_bytes, S.main_flops);
+        return launch_all(D, *ctx, st, profile, S.main_bytes, S.main_flops);
     }
 };
 
@@ -591,16 +669,14 @@ ndc_status batch_create(ndc_handle h, const ndc_batch_desc* d, Batch** out) {
         if (int64_t(b->s) >= (int64_t(1) << 20) || int64_t(b->d) >= (int64_t(1) << 20))
             return fail(h, NDC_ERR_UNSUPPORTED, "stride or dilation too large for the batch kernels");
         b->cm = cost_model(*ctx, b->s, b->d, b->algo == NDC_BATCH_AUTO || b->algo == NDC_BATCH_AUTO_BF16X3);
-        b->method.resize(size_t(P));
         auto repeats = [](const ndc_border& side) {
             return side.tag == NDC_BORDER_REPLICATE || (side.tag == NDC_BORDER_CONST && side.value.re != 0.0);
         };
         const bool rb = repeats(front) || repeats(back);
-        for (int64_t i = 0; i < P; ++i)
-            b->method[size_t(i)] = choose(b->cm, b->shapes[size_t(i)], b->s, b->algo, rb);
-        b->S = build_schedule(b->shapes, b->offs, b->method, b->s, b->cm);
-        const float2* tw = batch_twiddles(*ctx);
-        if (!tw || !b->D.upload(b->S, tw, resident_blocks(*ctx)))
+        const BatchForm form{b->s, b->d, side1d(front.tag), side1d(back.tag), ctx->cu_count(), resident_blocks(*ctx)};
+        b->method = choose(b->cm, b->shapes, form, b->algo, rb);
+        b->S = build_schedule(b->shapes, b->offs, b->method, form, b->cm);
+        if (!b->D.upload(b->S, *ctx, resident_blocks(*ctx)))
             return fail(h, NDC_ERR_OUT_OF_MEMORY, "batch metadata upload failed");
         BatchArgs& a = b->D.args;
         a.s = b->s;
@@ -686,19 +762,23 @@ void append(std::string& s, const char* fmt, double v) {
 std::string batch_report(const Batch& b) {
     std::string r = "{\"algo\": " + std::to_string(b.algo) + ", \"pairs\": " + std::to_string(b.shapes.size());
     r += ", \"outputs\": " + std::to_string(b.y_total);
-    r += ", \"items\": " + std::to_string(b.S.items.size()) + ", \"lines\": " + std::to_string(b.S.lines.size());
-    r += ", \"kernel_spectra\": " + std::to_string(b.S.kpairs.size());
+    size_t runs = 0;
+    for (const auto& t : b.S.tiles) runs += t.size();
+    r += ", \"items\": " + std::to_string(b.S.items.size()) + ", \"lines\": " + std::to_string(b.S.ntiles);
+    r += ", \"kernel_spectra\": " + std::to_string(runs);   // one per run
     r += ", \"grid\": " + std::to_string(b.D.grid);
     r += ", \"blocks_per_cu\": " + std::to_string(batch_blocks_per_cu());
     append(r, ", \"est_ms\": %.6f", b.S.est_ms);
     append(r, ", \"main_bytes\": %.1f", b.S.main_bytes);
-    append(r, ", \"kspec_bytes\": %.1f", b.S.kspec_bytes);
     append(r, ", \"main_flops\": %.1f", b.S.main_flops);
     r += ", \"costs\": {\"measured\": ";
     r += b.cm.measured ? "true" : "false";
-    r += ", \"fft_item_ms\": [";
-    for (int c = 0; c < kBatchClasses; ++c) append(r, c ? ", %.4e" : "%.4e", b.cm.fft_item[c]);
+    r += ", \"tile_run_ms\": [";
+    for (int c = 0; c < kBatchTileClasses; ++c) append(r, c ? ", %.4e" : "%.4e", b.cm.tile_a[c]);
+    r += "], \"tile_ms\": [";
+    for (int c = 0; c < kBatchTileClasses; ++c) append(r, c ? ", %.4e" : "%.4e", b.cm.tile_b[c]);
     r += "]";
+    append(r, ", \"edge_ms\": %.4e", b.cm.edge);
     append(r, ", \"direct_item_ms\": %.4e", b.cm.dir_a);
     append(r, ", \"direct_mac_ms\": %.4e", b.cm.dir_b);
     append(r, ", \"mfma_item_ms\": %.4e", b.cm.mfma_a);
@@ -714,7 +794,7 @@ std::string batch_report(const Batch& b) {
         const std::string name = m == kMethodDirect ? "direct_fp32"
                                  : m == kMethodMfma  ? "direct_bf16x3"
                                  : m == kMethodMfma6 ? "direct_bf16x6"
-                                                     : "fft" + std::to_string(2 * batch_lc(m));
+                                                     : "tile" + std::to_string(1 << batch_tile_log2(kMethodTile - m));
         bk[{kb, nb}][name] += 1;
     }
     r += ", \"buckets\": [";

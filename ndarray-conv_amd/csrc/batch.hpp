@@ -5,13 +5,11 @@
 // (conv_fft/mod.rs:185-292): ConvMode and PaddingMode are shared by the
 // batch, lengths differ per pair.  Each pair is computed by one of
 //   - direct items: a tile of outputs, FP32 multiply-adds over the taps;
-//   - overlap-save FFT items: blocks of outputs, each from one real FFT of
-//     length L = 2 * LC (LC = 256 .. 4096 complex points) of a window of the
-//     padded signal, multiplied by the pair's kernel spectrum (computed by a
-//     pre-pass at the same L) and transformed back.  Overlap-save computes the
-//     same linear correlation as the reference's single FFT of the whole padded
-//     signal, only blocked: window position u >= kdil - 1 of a block holds
-//     full-correlation index block_start + u.
+//   - matrix-core items: a tile of outputs from split BF16 products;
+//   - tile runs (batch_tile.hip, launches of their own): FP32 overlap-save, two
+//     real tiles per complex transform, the kernel's spectrum in registers.
+//     Overlap-save computes the same linear correlation as the reference's
+//     single FFT of the whole padded signal, only blocked.
 // The choice per pair comes from a cost model whose constants are measured
 // on the device (the autotuner).
 #pragma once
@@ -24,19 +22,18 @@
 
 #include "launch.hpp"
 #include "ndconv.h"
+#include "tile_conv.hpp"
 
 namespace ndc {
 
 constexpr int kBatchThreads = 256;
-constexpr int kBatchClasses = 5;             // LC = 256 << c, c = 0..4
-constexpr int kBatchPoints = 4096;           // complex points per FFT item (G lines of LC)
 constexpr int kBatchDirectTile = 2048;       // outputs per direct item (8 per thread)
 constexpr int kBatchWindow = 6144;           // LDS window capacity of a direct item (floats)
 constexpr int kBatchTapChunk = 1024;         // taps staged per round of a direct item
 constexpr int kBatchMfmaTile = 4096;         // outputs per matrix-core item (1024 per wave)
 constexpr int kBatchMfmaMaxKdil = 1024;      // longest dilated kernel of a matrix-core item (LDS)
-constexpr int kBatchKindMfma = 1 + kBatchClasses;    // BF16x3 matrix-core tile (two-term split)
-constexpr int kBatchKindMfma6 = 2 + kBatchClasses;   // BF16x6 matrix-core tile (three-term split)
+constexpr int kBatchKindMfma = 1;            // BF16x3 matrix-core tile (two-term split)
+constexpr int kBatchKindMfma6 = 2;           // BF16x6 matrix-core tile (three-term split)
 // Fewest kernel taps for which the autotuned and matrix-core batch forms use
 // BF16x3.  Its products carry about 16 significant bits (each within
 // 3 * 2^-16 of the exact product); an output summed from a few products keeps
@@ -48,7 +45,7 @@ constexpr int kBatchKindMfma6 = 2 + kBatchClasses;   // BF16x6 matrix-core tile 
 constexpr int kBf16x3MinTaps = 32;
 
 // The work queue is two ranges of the item list, each longest-first: the
-// direct and FFT items [0, nfirst), then the matrix-core items [nfirst,
+// direct items [0, nfirst), then the matrix-core items [nfirst,
 // nitems).  Workgroups below nfirst drain the first range, then all drain
 // the second.  Each
 // range is kBatchQueues sub-queues: sub-queue q of a range starting at lo
@@ -65,27 +62,8 @@ constexpr int kBatchHeads = 2 * kBatchQueues;
 // below 1 / d).
 constexpr uint32_t batch_dmul(int d) { return uint32_t(((uint64_t(1) << 31) + uint64_t(d) - 1) / uint64_t(d)); }
 
-constexpr int batch_lc(int cls) { return 256 << cls; }
-constexpr int batch_lines(int cls) { return kBatchPoints / batch_lc(cls); }
-// Quarter-circle twiddle tables of all classes, concatenated: class c has
-// LC/2 = 128 << c entries.
-constexpr int batch_tw_offset(int cls) { return 128 * ((1 << cls) - 1); }
-
-// Per-pair metadata read by the kernels (64 bytes).
-struct BatchPair {
-    int64_t x_off, k_off, y_off;   // element offsets into the packed x, k, y
-    int64_t ks_off;                // complex offset of the kernel spectrum (FFT pairs)
-    int32_t n, k;                  // signal and kernel length
-    int32_t p0, pds;               // front pad, padded length n + p0 + p1
-    int32_t out;                   // output length
-    int32_t per;                   // outputs per FFT block
-    int32_t cls;                   // FFT class, or -1 for direct
-    int32_t pad_;
-};
-
 // One unit of the work queue (64 bytes).
 //   kind 0: direct tile  a = pair, b = first output, c = output count
-//   kind 1 + cls: FFT    a = first line, b = line count (<= batch_lines(cls))
 //   kind kBatchKindMfma / kBatchKindMfma6: BF16x3 / BF16x6 matrix-core tile,
 //       a = pair, b = first output, c = count
 // Direct and matrix-core tiles carry their pair's metadata, so a workgroup
@@ -98,23 +76,28 @@ struct BatchItem {
 };
 static_assert(sizeof(BatchItem) == 64, "work-queue records are 16 dwords");
 
-// One overlap-save block with its pair's metadata: first output o0, outputs
-// per block, and what the pair's kernel spectrum and signal need.
-struct BatchLine {
-    int64_t x_off, y_off, ks_off;
-    int32_t n, k, p0, pds, out, per, o0, pair;
+// A run of consecutive complex tiles of one pair (batch_tile.hip, 64 bytes):
+// tiles 2 q and 2 q + 1 of every q in [first, first + count).
+struct BatchTile {
+    int64_t x_off, k_off, y_off;
+    int32_t n, k, p0, pds, out;    // the pair's lengths, front pad, padded and output length
+    int32_t V, tiles;              // outputs per tile and phase, tiles per phase
+    int32_t first, count;
+    int32_t wraps;                 // a pad repeats x or reads the other pad
 };
+static_assert(sizeof(BatchTile) == 64, "one record, one scalar load");
 
-// Kernel-spectrum pre-pass work: up to batch_lines(cls) pairs of one class,
-// klines [first, first + count).
-struct BatchKItem {
-    int32_t cls, first, count, pad_;
-};
+// Tile classes by points.  The last addresses in 64 bits, for pairs of 2^28
+// samples and more and for kernels that no other class holds.
+constexpr int kBatchTileClasses = 4;
+constexpr int kBatchTileFar = kBatchTileClasses - 1;
+constexpr int batch_tile_log2(int c) { return c == 0 ? 10 : 11 + c; }   // 1024, 4096, 8192, 16384
 
-// What the pre-pass reads of a pair, in pre-pass order (24 bytes, one load).
-struct BatchKLine {
-    int64_t k_off, ks_off;         // kernel offset into k, complex offset of its spectrum
-    int32_t k, pad_;               // kernel length
+struct BatchTileLaunch {
+    const BatchTile* items[kBatchTileClasses] = {};
+    int32_t n[kBatchTileClasses] = {};
+    double bytes[kBatchTileClasses] = {};
+    const void* tw[kBatchTileClasses] = {};
 };
 
 // Shared launch parameters of a batch.
@@ -122,31 +105,34 @@ struct BatchArgs {
     const float* x;
     const float* k;
     float* y;
-    const BatchPair* pairs;
     const BatchItem* items;
-    const BatchLine* lines;
-    const BatchKLine* klines;      // pairs of the kernel-spectrum pre-pass, grouped by class
-    const BatchKItem* kitems;
-    float2* kspec;
-    int32_t* counter;              // kBatchHeads sub-queue heads (kBatchQueueStride apart), reset by the pre-pass
-    const float2* tw;              // W_L^r, r < L/4, of class c at batch_tw_offset(c) (L = 2 LC)
+    int32_t* counter;              // kBatchHeads sub-queue heads (kBatchQueueStride apart), zero at the launch
     const float* consts;           // {0, cfront, cback, 0}: the cells constant pad positions read
-    int32_t nitems, nkitems;
-    int32_t nfirst;                // items of the first range (direct and FFT)
+    int32_t nitems;
+    int32_t nfirst;                // items of the first range (direct)
     int32_t s, d, rev;
     uint32_t dmul;                 // batch_dmul(d)
     int32_t front, back;           // side tags of border1d.hpp
     float cfront, cback;           // constants of Const sides
 };
 
-// Device launchers (batch_conv.hip).
+// Device launchers.  With `profile` each launch is bracketed for ctx's
+// per-kernel profile (not while capturing); the byte/flop counts are the
+// algorithmic traffic of each launch.
+//
+// The queue (batch_conv.hip); `reset` zeroes its heads in a launch before it.
 size_t batch_lds_bytes();
 int batch_blocks_per_cu();
-// Pre-pass then persistent main launch on `stream`.  With `profile` each
-// launch is bracketed for ctx's per-kernel profile (not while capturing);
-// the byte/flop counts are the algorithmic traffic of each launch.
-ndc_status launch_batch(const BatchArgs& a, int grid, LaunchContext& ctx, hipStream_t stream, bool profile,
-                        double kspec_bytes, double main_bytes, double main_flops);
+ndc_status launch_batch(const BatchArgs& a, int grid, bool reset, LaunchContext& ctx, hipStream_t stream, bool profile,
+                        double main_bytes, double main_flops);
+// The tile runs (batch_tile.hip), each launch zeroing the queue's heads, and
+// their twiddle tables.
+bool batch_tile_tables(LaunchContext& ctx, const void* tw[kBatchTileClasses]);
+ndc_status launch_batch_tiles(const BatchArgs& a, const BatchTileLaunch& l, LaunchContext& ctx, hipStream_t stream,
+                              bool profile);
+
+// n samples of Uniform[-1, 1) (batch_conv.hip), for the cost model's measurements.
+ndc_status fill_random(float* p, int64_t n, LaunchContext& ctx);
 
 // Services of the handle behind an ndc_handle (capi.cpp).
 LaunchContext* handle_context(ndc_handle h);

@@ -1,17 +1,5 @@
-// Kernels of the batched rank-1 path: a kernel-spectrum pre-pass and one
-// persistent launch that drains the work queue (direct tiles and
-// overlap-save FFT blocks of all pairs).
-//
-// FFT items hold kBatchPoints complex points in LDS: G = kBatchPoints / LC
-// lines of LC points, each line the half-length complex view
-// z[n] = w[2n] + i w[2n+1] of a real window of L = 2 LC samples.  A line is
-// transformed by radix-16 Stockham passes with the 16 points of a butterfly
-// in registers (the last pass is radix 2/4/8/16 to reach LC), LDS only being
-// used to exchange between passes.  The padded layout i + i/16 keeps the
-// stride-16 accesses of the first pass free of bank conflicts.  The window is
-// read from global memory with the border remap fused into the load, and only
-// the cropped, strided outputs are written back.  Twiddles W_L^r come from a
-// quarter-circle table generated in FP64 on the host and staged in LDS.
+// The work queue's kernel of the batched rank-1 path: one persistent launch
+// that drains the direct tiles and the matrix-core tiles of all pairs.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -22,19 +10,12 @@
 #include "batch.hpp"
 #include "bf16_split.hpp"
 #include "border1d.hpp"
-#include "fft_bfly.hpp"
 
 namespace ndc {
 namespace {
 
-using namespace fftb;
-using C = float2;
-
 constexpr int T = kBatchThreads;
-constexpr int kTwSlots = 2048;                                   // L/4 for the largest class
-constexpr int kDataSlots = kBatchPoints + kBatchPoints / 16;     // padded FFT data
 constexpr int kWinSlots = kBatchWindow + kBatchWindow / 8;       // padded direct window
-constexpr size_t kFftLdsBytes = size_t(kTwSlots + kDataSlots) * sizeof(C);
 
 __device__ __forceinline__ int padh(int e) { return e + 8 * (e >> 5); }   // 16 bytes of padding per 64
 
@@ -78,10 +59,9 @@ struct MfmaLds {
     static constexpr size_t bytes = size_t(P * win_slots + P * term) * 2;
 };
 
-// dynamic LDS of both kernels: the larger of the FFT layout and BF16x6 staging
-constexpr size_t kLdsBytes = ((kFftLdsBytes > MfmaLds<3>::bytes ? kFftLdsBytes : MfmaLds<3>::bytes) + 255) & ~size_t(255);
-static_assert(size_t(kWinSlots + kBatchTapChunk) * sizeof(float) <= size_t(kDataSlots) * sizeof(C),
-              "direct-item staging must fit the FFT data region");
+// dynamic LDS of the queue's kernel: BF16x6 staging, the largest
+constexpr size_t kLdsBytes = (MfmaLds<3>::bytes + 255) & ~size_t(255);
+static_assert(size_t(kWinSlots + kBatchTapChunk) * sizeof(float) <= kLdsBytes, "direct-item staging must fit");
 
 // threadIdx.x behind an empty volatile asm: inside the persistent loop it is
 // re-read per item, so the compiler cannot hoist the address arithmetic of
@@ -92,7 +72,6 @@ __device__ __forceinline__ int tid() {
     return t;
 }
 
-__device__ __forceinline__ int padi(int i) { return i + (i >> 4); }
 __device__ __forceinline__ int padw(int i) { return i + (i >> 3); }
 
 // st(e, f(e)) for e < n, with U values of f (global loads) in flight per
@@ -114,301 +93,24 @@ __device__ __forceinline__ void staged(int n, F&& f, S&& st) {
     }
 }
 
-// W_L^e from the quarter table q[r] = W_L^r, r < L/4 (L a power of two).
-__device__ __forceinline__ C twl(const C* q, int e, int L) {
-    e &= L - 1;
-    const int q4 = L >> 2;
-    const int quad = e / q4;
-    const C v = q[e & (q4 - 1)];
-    switch (quad) {
-        case 0: return v;
-        case 1: return cmake<C>(v.y, -v.x);     // * -i
-        case 2: return cmake<C>(-v.x, -v.y);    // * -1
-        default: return cmake<C>(-v.y, v.x);    // * i
-    }
-}
-
-// v[r] *= W_L^(r E) (conjugated for the inverse), r = 1 .. R-1; powers
-// beyond 1, 2, 4, 8 are products of at most three looked-up factors.
-template <int R>
-__device__ __forceinline__ void twiddle(C* v, int E, const C* q, int L, bool inv) {
-    C w[16];
-    w[1] = twl(q, E, L);
-    if constexpr (R > 2) {
-        w[2] = twl(q, 2 * E, L);
-        w[3] = cmul(w[2], w[1]);
-    }
-    if constexpr (R > 4) {
-        w[4] = twl(q, 4 * E, L);
-        w[5] = cmul(w[4], w[1]);
-        w[6] = cmul(w[4], w[2]);
-        w[7] = cmul(w[4], w[3]);
-    }
-    if constexpr (R > 8) {
-        w[8] = twl(q, 8 * E, L);
-#pragma unroll
-        for (int r = 9; r < 16; ++r) w[r] = cmul(w[8], w[r - 8]);
-    }
-#pragma unroll
-    for (int r = 1; r < R; ++r) v[r] = cmulc(v[r], w[r], inv);
-}
-
-// One radix-R Stockham pass, in place, over the G lines of an item in LDS:
-// butterfly j of a line reads points j + r LC/R, applies W_(Ns R)^(r k)
-// (k = j mod Ns), and writes (j - k) R + k + r Ns.  Ends with a barrier.
-template <int LC, int R>
-__device__ __forceinline__ void pass(C* buf, const C* q, int Ns, bool inv) {
-    constexpr int NB = 16 / R;
-    constexpr int BPL = LC / R;
-    constexpr int LS = LC + LC / 16;
-    constexpr int L = 2 * LC;
-    C v[16];
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-        const int beta = tid() + b * T;
-        const int g = beta / BPL, j = beta % BPL;
-#pragma unroll
-        for (int r = 0; r < R; ++r) v[b * R + r] = buf[g * LS + padi(j + r * BPL)];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-        const int beta = tid() + b * T;
-        const int g = beta / BPL, j = beta % BPL;
-        const int k = j & (Ns - 1);
-        if (Ns > 1) twiddle<R>(v + b * R, k * (L / (Ns * R)), q, L, inv);
-        bfly<R>(v + b * R, inv);
-        const int ob = (j - k) * R + k;
-#pragma unroll
-        for (int r = 0; r < R; ++r) buf[g * LS + padi(ob + r * Ns)] = v[b * R + r];
-    }
-    __syncthreads();
-}
-
-template <int LC> struct LastRadix { static constexpr int value = LC / 256; };
-template <> struct LastRadix<256> { static constexpr int value = 16; };
-
-// Transform of the G lines in LDS (natural order in and out): radix 16,
-// radix 16, then the radix that completes LC.
-template <int LC>
-__device__ __forceinline__ void fft_lds(C* buf, const C* q, bool inv) {
-    pass<LC, 16>(buf, q, 1, inv);
-    pass<LC, 16>(buf, q, 16, inv);
-    if constexpr (LC > 256) pass<LC, LastRadix<LC>::value>(buf, q, 256, inv);
-}
-
-// Real sample u of line g in the padded layout (the complex view's point
-// u/2, real part for even u).
-template <int LC>
-__device__ __forceinline__ int real_slot(int g, int u) {
-    constexpr int LS = LC + LC / 16;
-    return 2 * (g * LS + padi(u >> 1)) + (u & 1);
-}
-
-// X[m] of a real line from its half-length spectrum: zk = Z[m], zo = Z[LC-m].
-__device__ __forceinline__ C r2c(C zk, C zo, C w) {
-    const C zc = cconj(zo);
-    const C e = cscale(cadd(zk, zc), 0.5f);
-    const C o = cmul_negi(cscale(csub(zk, zc), 0.5f));
-    return cadd(e, cmul(o, w));
-}
-
-// Half-length inverse input from A = P[m], B = conj P[LC-m].
-__device__ __forceinline__ C c2r(C A, C B, C w) {
-    return cadd(cadd(A, B), cmul_i(cmul(csub(A, B), cconj(w))));
-}
-
-// Per-line context of an item, staged in LDS.
-struct LineCtx {
-    int64_t x_off, y_off, ks_off, k_off;
-    int64_t src;                   // x offset of window sample 0 when the window is all interior
-    int32_t n, k, p0, pds, out, per, o0, valid;
-    int32_t interior, pad_;
-};
-
 // Address of padded position P: an element of x, or the cell of a.consts
 // holding the position's constant (zero past the padded end and for cells the
 // fill never writes).  Address arithmetic only, so that a window's loads can
 // all be issued before the first one returns: a load inside the border
 // branches makes the compiler wait for it before the next position.
-__device__ __forceinline__ const float* pad_ptr(const BatchArgs& a, const LineCtx& c, int64_t P) {
+__device__ __forceinline__ const float* pad_ptr(const BatchArgs& a, const BatchItem& c, int64_t P) {
     if (P >= c.pds) return a.consts;
     const int64_t s = resolve1d<int64_t>(P, c.n, c.p0, a.front, a.back);
     if (s >= 0) return a.x + c.x_off + s;
     return a.consts + (s == kConstFront ? 1 : s == kConstBack ? 2 : 0);
 }
 
-__device__ __forceinline__ float pad_value(const BatchArgs& a, const LineCtx& c, int64_t P) { return *pad_ptr(a, c, P); }
+__device__ __forceinline__ float pad_value(const BatchArgs& a, const BatchItem& c, int64_t P) { return *pad_ptr(a, c, P); }
 
 // Tap t of the correlation form out[o] = sum_t pad[o s + t d] kc[t]:
 // kc[t] = k[K-1-t] for a convolution (reverse), k[t] for no_reverse.
 __device__ __forceinline__ float corr_tap(const BatchArgs& a, int64_t k_off, int K, int t) {
     return a.k[k_off + (a.rev ? K - 1 - t : t)];
-}
-
-// span: window length in samples (the interior test covers [o0 s, o0 s + span)).
-__device__ __forceinline__ void load_line_ctx(const BatchArgs& a, LineCtx* lc, int G, int first, int count, int span) {
-    const int g = tid();
-    if (g < G) {
-        LineCtx c{};
-        c.valid = g < count;
-        if (c.valid) {
-            // a data line's record carries its pair's metadata: one load
-            const BatchLine ln = a.lines[first + g];
-            c.o0 = ln.o0;
-            c.x_off = ln.x_off;
-            c.y_off = ln.y_off;
-            c.ks_off = ln.ks_off;
-            c.n = ln.n;
-            c.k = ln.k;
-            c.p0 = ln.p0;
-            c.pds = ln.pds;
-            c.out = ln.out;
-            c.per = ln.per;
-            const int64_t P0 = int64_t(c.o0) * a.s;
-            c.interior = P0 >= c.p0 && P0 + span <= int64_t(c.p0) + c.n;
-            c.src = c.x_off + P0 - c.p0;
-        }
-        lc[g] = c;
-    }
-}
-
-// Writes the real samples of the G lines: sample u of line g is *addr(c, u)
-// (addr returns a readable address for every line, valid or not).  Each
-// thread loads its L / T samples of every line, all in flight at once.
-template <int LC, typename F>
-__device__ __forceinline__ void load_reals(float* fb, const LineCtx* lc, F&& addr) {
-    constexpr int G = kBatchPoints / LC;
-    constexpr int L = 2 * LC;
-    constexpr int J = L / T;
-    static_assert(L % T == 0, "a line is whole rounds of the workgroup");
-    const int t = tid();
-    float v[G * J];
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-        const LineCtx& c = lc[g];
-#pragma unroll
-        for (int j = 0; j < J; ++j) v[g * J + j] = *addr(c, t + j * T);
-    }
-#pragma unroll
-    for (int g = 0; g < G; ++g)
-#pragma unroll
-        for (int j = 0; j < J; ++j) fb[real_slot<LC>(g, t + j * T)] = v[g * J + j];
-    __syncthreads();
-}
-
-template <int LC>
-__device__ __forceinline__ void fft_item(const BatchArgs& a, const BatchItem& it, const C* q, C* buf, LineCtx* lc) {
-    constexpr int G = kBatchPoints / LC;
-    constexpr int LS = LC + LC / 16;
-    constexpr int L = 2 * LC;
-    constexpr int H = LC / 2 + 1;
-    load_line_ctx(a, lc, G, it.a, it.b, L);
-    __syncthreads();
-    const int s = a.s;
-    float* fb = reinterpret_cast<float*>(buf);
-    // window of padded positions [o0 s, o0 s + L), border remap fused in
-    load_reals<LC>(fb, lc, [&](const LineCtx& c, int u) -> const float* {
-        if (!c.valid) return a.consts;
-        return c.interior ? a.x + c.src + u : pad_ptr(a, c, int64_t(c.o0) * s + u);
-    });
-    // the kernel-spectrum bins this thread multiplies, loaded while the
-    // forward transform runs
-    constexpr int NI = (G * H + T - 1) / T;
-    C kmv[NI], kpv[NI];
-#pragma unroll
-    for (int r = 0; r < NI; ++r) {
-        const int idx = tid() + r * T;
-        kmv[r] = kpv[r] = cmake<C>(0.f, 0.f);
-        if (idx < G * H) {
-            const int g = idx / H, m = idx - g * H;
-            const LineCtx& c = lc[g];
-            if (c.valid) {
-                kmv[r] = a.kspec[c.ks_off + m];
-                kpv[r] = a.kspec[c.ks_off + LC - m];
-            }
-        }
-    }
-    fft_lds<LC>(buf, q, false);
-    // spectrum product, bins m and LC - m together
-#pragma unroll
-    for (int r = 0; r < NI; ++r) {
-        const int idx = tid() + r * T;
-        if (idx >= G * H) break;
-        const int g = idx / H, m = idx - g * H;
-        const LineCtx& c = lc[g];
-        if (!c.valid) continue;
-        C* Z = buf + g * LS;
-        const int mp = LC - m;
-        const C zm = Z[padi(m)];
-        const C zp = Z[padi(mp == LC ? 0 : mp)];
-        const C wm = twl(q, m, L), wp = twl(q, mp, L);
-        C Pm = cmul(r2c(zm, zp, wm), kmv[r]);
-        C Pp = cmul(r2c(zp, zm, wp), kpv[r]);
-        if (m == 0) {   // imaginary parts of DC and Nyquist are ignored by c2r
-            Pm.y = 0.f;
-            Pp.y = 0.f;
-        }
-        Z[padi(m)] = c2r(Pm, cconj(Pp), wm);
-        if (mp != m && mp < LC) Z[padi(mp)] = c2r(Pp, cconj(Pm), wp);
-    }
-    __syncthreads();
-    fft_lds<LC>(buf, q, true);
-    // crop and stride: output o0 + j is window sample kdil - 1 + j s (< L);
-    // every thread reads its L / T candidates of each line first (clamped
-    // into the line), then stores the ones that are outputs
-    constexpr int J = L / T;
-    const int t = tid();
-    float v[G * J];
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-        const int kdil = lc[g].valid ? (lc[g].k - 1) * a.d + 1 : 1;
-#pragma unroll
-        for (int j = 0; j < J; ++j) {
-            const int u = kdil - 1 + (t + j * T) * s;
-            v[g * J + j] = fb[real_slot<LC>(g, u < L ? u : L - 1)];
-        }
-    }
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-        const LineCtx& c = lc[g];
-        const int cnt = !c.valid ? 0 : c.per < c.out - c.o0 ? c.per : c.out - c.o0;
-        float* y = a.y + c.y_off + c.o0;
-#pragma unroll
-        for (int j = 0; j < J; ++j)
-            if (t + j * T < cnt) y[t + j * T] = v[g * J + j];
-    }
-}
-
-// The lines' context (valid, k, k_off, ks_off) is in lc, and the class's
-// twiddle table in q.
-template <int LC>
-__device__ __forceinline__ void kspec_item(const BatchArgs& a, const C* q, C* buf, const LineCtx* lc) {
-    constexpr int G = kBatchPoints / LC;
-    constexpr int LS = LC + LC / 16;
-    constexpr int L = 2 * LC;
-    const int d = a.d;
-    float* fb = reinterpret_cast<float*>(buf);
-    // scattered kernel of the reference's FFT path (conv_fft/padding.rs:78-111):
-    // k[i] at i d (reverse) or (K-1-i) d (no_reverse)
-    // u / d as the high word of 2u dmul (exact: u < 2 LC <= 8192, and a pair
-    // whose dilation passes 2^18 has one tap, whose only position is u = 0)
-    load_reals<LC>(fb, lc, [&](const LineCtx& c, int u) -> const float* {
-        const int i = int(__umulhi(uint32_t(u) << 1, a.dmul));
-        if (!c.valid || u != i * d || i >= c.k) return a.consts;
-        return a.k + c.k_off + (a.rev ? i : c.k - 1 - i);
-    });
-    fft_lds<LC>(buf, q, false);
-    const float scale = 1.0f / float(L);   // the inverse normalisation, folded in
-    for (int idx = tid(); idx < G * (LC + 1); idx += T) {
-        const int g = idx / (LC + 1), m = idx - g * (LC + 1);
-        const LineCtx& c = lc[g];
-        if (!c.valid) continue;
-        const C* Z = buf + g * LS;
-        const C zm = Z[padi(m == LC ? 0 : m)];
-        const C zp = Z[padi(m == 0 ? 0 : LC - m)];
-        a.kspec[c.ks_off + m] = cscale(r2c(zm, zp, twl(q, m, L)), scale);
-    }
 }
 
 // Direct tile: outputs [o0, o0 + cnt) of one pair, taps staged in chunks.
@@ -424,7 +126,7 @@ __device__ __forceinline__ void direct_item(const BatchArgs& a, const BatchItem&
     float acc[8];
 #pragma unroll
     for (int m = 0; m < 8; ++m) acc[m] = 0.f;
-    LineCtx c{};
+    BatchItem c{};
     c.x_off = p.x_off;
     c.n = p.n;
     c.p0 = p.p0;
@@ -539,7 +241,7 @@ __device__ __forceinline__ void mfma_stage_load(const BatchArgs& a, const BatchI
     const int nkb = (kdil + 31 + 15) / 16;
     const int W = kBatchMfmaTile + 16 * nkb + 32;
     const int64_t o0 = p.b;
-    LineCtx c{};
+    BatchItem c{};
     c.x_off = p.x_off;
     c.n = p.n;
     c.p0 = p.p0;
@@ -765,78 +467,17 @@ __device__ __forceinline__ void mfma_item(const BatchArgs& a, const BatchItem& p
     __builtin_amdgcn_s_waitcnt(kWaitVmcnt16);
 }
 
-// BF16x3 staging fits the FFT data region (the twiddle table stays); BF16x6
-// staging takes the whole dynamic allocation, twiddles included.
-static_assert(MfmaLds<2>::bytes <= size_t(kDataSlots) * sizeof(C), "BF16x3 staging must fit the FFT data region");
-static_assert(MfmaLds<3>::bytes <= kLdsBytes, "BF16x6 staging must fit the dynamic LDS");
-
-// A class's quarter table (n = LC/2 <= kTwSlots points): every load of a
-// thread is issued before its first LDS store.  A plain copy loop waits for
-// each load before the next, eight serial round trips for the largest class.
-__device__ __forceinline__ void stage_tw(C* dst, const C* src, int n) {
-    constexpr int U = kTwSlots / T;
-    static_assert(kTwSlots % T == 0 && batch_lc(kBatchClasses - 1) / 2 <= kTwSlots, "one round per thread slot");
-    C v[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-        const int i = tid() + u * T;
-        if (i < n) v[u] = src[i];
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-        const int i = tid() + u * T;
-        if (i < n) dst[i] = v[u];
-    }
-}
-
-__global__ void __launch_bounds__(kBatchThreads) batch_kspec_kernel(BatchArgs a) {
-    extern __shared__ C smem[];
-    __shared__ LineCtx lc[16];
-    if (blockIdx.x == 0 && threadIdx.x < kBatchHeads) a.counter[threadIdx.x * kBatchQueueStride] = 0;   // sub-queue heads
-    if (int(blockIdx.x) >= a.nkitems) return;
-    const BatchKItem it = a.kitems[blockIdx.x];
-    C* q = smem;
-    C* buf = smem + kTwSlots;
-    const int LC = batch_lc(it.cls);
-    const int G = kBatchPoints / LC;
-    // the lines' records and the twiddle table in flight together
-    const int g = tid();
-    const bool valid = g < G && g < it.count;
-    BatchKLine kl{};
-    if (valid) kl = a.klines[it.first + g];
-    stage_tw(q, a.tw + batch_tw_offset(it.cls), LC / 2);
-    if (g < G) {
-        LineCtx c{};
-        c.valid = valid;
-        c.k_off = kl.k_off;
-        c.ks_off = kl.ks_off;
-        c.k = kl.k;
-        lc[g] = c;
-    }
-    __syncthreads();
-    switch (it.cls) {
-        case 0: kspec_item<256>(a, q, buf, lc); break;
-        case 1: kspec_item<512>(a, q, buf, lc); break;
-        case 2: kspec_item<1024>(a, q, buf, lc); break;
-        case 3: kspec_item<2048>(a, q, buf, lc); break;
-        default: kspec_item<4096>(a, q, buf, lc); break;
-    }
-}
-
-// LDS of the persistent loop beside the dynamic allocation: the FFT lines'
-// context and the queue ring.
-__shared__ LineCtx g_lc[16];
+// LDS of the persistent loop beside the dynamic allocation: the queue ring.
 __shared__ int g_item[3];
 __shared__ BatchItem g_rec[3];
 
 // Persistent: the workgroup takes items of one range of the queue until the
-// range is empty (the only exit, reached by every workgroup): the direct and
-// FFT items (M false) or the matrix-core items (M true).  The matrix-core
-// range's loop is a function of its own, called once per workgroup, so the
-// FFT code's registers do not crowd it: in one loop with the FFT code the
-// matrix-core items' scalar values spilled to vector lanes (about a fifth of
-// their vector instructions).  The first range's loop stays in the kernel,
-// which has the larger scalar register budget (no call convention).
+// range is empty (the only exit, reached by every workgroup): the direct items
+// (M false) or the matrix-core items (M true).  The matrix-core range's loop is
+// a function of its own, called once per workgroup, so the other items'
+// registers do not crowd it: in one loop with them the matrix-core items'
+// scalar values spilled to vector lanes.  The first range's loop stays in the
+// kernel, which has the larger scalar register budget (no call convention).
 typedef const __attribute__((address_space(4))) BatchArgs* KernargArgs;
 
 // The launch arguments, field by field from the kernel argument segment
@@ -857,17 +498,10 @@ __device__ __forceinline__ BatchArgs kernel_args(KernargArgs arg) {
     a.x = ap->x;
     a.k = ap->k;
     a.y = ap->y;
-    a.pairs = ap->pairs;
     a.items = ap->items;
-    a.lines = ap->lines;
-    a.klines = ap->klines;
-    a.kitems = ap->kitems;
-    a.kspec = ap->kspec;
     a.counter = ap->counter;
-    a.tw = ap->tw;
     a.consts = ap->consts;
     a.nitems = ap->nitems;
-    a.nkitems = ap->nkitems;
     a.nfirst = ap->nfirst;
     a.s = ap->s;
     a.d = ap->d;
@@ -883,15 +517,11 @@ __device__ __forceinline__ BatchArgs kernel_args(KernargArgs arg) {
 template <bool M>
 __device__ __forceinline__ void drain(KernargArgs ap) {
     const BatchArgs a = kernel_args(ap);
-    extern __shared__ C smem[];
-    LineCtx* lc = g_lc;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     int* s_item = g_item;
     BatchItem* s_rec = g_rec;
-    C* q = smem;
-    C* buf = smem + kTwSlots;
-    float* win = reinterpret_cast<float*>(buf);
+    float* win = reinterpret_cast<float*>(smem);
     float* taps = win + kWinSlots;
-    int cur = -1;   // class whose twiddle table is in LDS
     const int lo = M ? a.nfirst : 0, hi = M ? a.nitems : a.nfirst;
     if (lo >= hi) return;   // uniform: an empty range costs no queue pops
     int32_t* heads = a.counter + (M ? kBatchQueues * kBatchQueueStride : 0);
@@ -951,33 +581,16 @@ __device__ __forceinline__ void drain(KernargArgs ap) {
             if (threadIdx.x == 0) next3 = ticket();
         };
         const BatchItem& it = s_rec[r0];
-        const int kind = it.kind;
         if constexpr (M) {
             // every item of this range is a matrix-core item
             const BatchItem* next = s_item[r1] < hi ? &s_rec[r1] : nullptr;
-            if (kind == kBatchKindMfma)
-                mfma_item<2>(a, it, reinterpret_cast<uint16_t*>(buf), st, have, next, advance);
+            if (it.kind == kBatchKindMfma)
+                mfma_item<2>(a, it, reinterpret_cast<uint16_t*>(smem), st, have, next, advance);
             else
                 mfma_item<3>(a, it, reinterpret_cast<uint16_t*>(smem), st, have, next, advance);
         } else {
             advance();
-            if (kind == 0) {
-                direct_item(a, it, win, taps);
-            } else {
-                const int cls = kind - 1;
-                if (cls != cur) {
-                    stage_tw(q, a.tw + batch_tw_offset(cls), batch_lc(cls) / 2);
-                    cur = cls;
-                    __syncthreads();
-                }
-                switch (cls) {
-                    case 0: fft_item<256>(a, it, q, buf, lc); break;
-                    case 1: fft_item<512>(a, it, q, buf, lc); break;
-                    case 2: fft_item<1024>(a, it, q, buf, lc); break;
-                    case 3: fft_item<2048>(a, it, q, buf, lc); break;
-                    default: fft_item<4096>(a, it, q, buf, lc); break;
-                }
-            }
+            direct_item(a, it, win, taps);
             __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);   // the queue's reads, on every lane (as above)
         }
         // Every item kind passes a barrier after all threads have read the
@@ -992,6 +605,19 @@ __device__ __forceinline__ void drain(KernargArgs ap) {
         if (threadIdx.x == 0) s_item[r0] = resolve(next3);
         __syncthreads();
         r0 = r1;
+    }
+}
+
+__global__ void __launch_bounds__(64) batch_reset_kernel(int32_t* heads) {
+    if (threadIdx.x < kBatchHeads) heads[threadIdx.x * kBatchQueueStride] = 0;
+}
+
+__global__ void __launch_bounds__(256) fill_random_kernel(float* p, int64_t n) {
+    for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < n; i += int64_t(gridDim.x) * 256) {
+        uint32_t h = uint32_t(i) * 0x9E3779B9u + 1u;   // a multiplicative hash
+        h = (h ^ (h >> 16)) * 0x85EBCA6Bu;
+        h ^= h >> 13;
+        p[i] = float(int32_t(h)) * 0x1p-31f;
     }
 }
 
@@ -1022,27 +648,26 @@ int batch_blocks_per_cu() {
     return n > 0 ? n : 1;
 }
 
-ndc_status launch_batch(const BatchArgs& a, int grid, LaunchContext& ctx, hipStream_t stream, bool profile,
-                        double kspec_bytes, double main_bytes, double main_flops) {
-    if (!lds_fits(ctx, reinterpret_cast<const void*>(batch_kspec_kernel), kLdsBytes) ||
-        !lds_fits(ctx, reinterpret_cast<const void*>(batch_main_kernel), kLdsBytes))
-        return NDC_ERR_UNSUPPORTED;
-    const int kgrid = a.nkitems > 0 ? a.nkitems : 1;
-    if (profile) ctx.kbegin("batch_kspec", kspec_bytes, 0);
-    NDC_LAUNCH(ctx, stream, batch_kspec_kernel, dim3(kgrid), dim3(kBatchThreads), kLdsBytes, a);
+ndc_status fill_random(float* p, int64_t n, LaunchContext& ctx) {
+    NDC_LAUNCH(ctx, ctx.stream(), fill_random_kernel, dim3(1024), dim3(256), 0, p, n);
+    return hipGetLastError() == hipSuccess ? NDC_OK : NDC_ERR_DEVICE;
+}
+
+ndc_status launch_batch(const BatchArgs& a, int grid, bool reset, LaunchContext& ctx, hipStream_t stream, bool profile,
+                        double main_bytes, double main_flops) {
+    if (!lds_fits(ctx, reinterpret_cast<const void*>(batch_main_kernel), kLdsBytes)) return NDC_ERR_UNSUPPORTED;
+    if (a.nitems <= 0 || grid <= 0) return NDC_OK;
+    if (reset) {
+        if (profile) ctx.kbegin("batch_reset", 0, 0);
+        NDC_LAUNCH(ctx, stream, batch_reset_kernel, dim3(1), dim3(64), 0, a.counter);
+        if (profile) ctx.kend();
+    }
+    if (profile) ctx.kbegin("batch_main", main_bytes, main_flops);
+    NDC_LAUNCH(ctx, stream, batch_main_kernel, dim3(grid), dim3(kBatchThreads), kLdsBytes, a);
     if (profile) ctx.kend();
     if (hipGetLastError() != hipSuccess) {
-        ctx.err = "batch_kspec launch failed";
+        ctx.err = "batch_main launch failed";
         return NDC_ERR_DEVICE;
-    }
-    if (a.nitems > 0 && grid > 0) {
-        if (profile) ctx.kbegin("batch_main", main_bytes, main_flops);
-        NDC_LAUNCH(ctx, stream, batch_main_kernel, dim3(grid), dim3(kBatchThreads), kLdsBytes, a);
-        if (profile) ctx.kend();
-        if (hipGetLastError() != hipSuccess) {
-            ctx.err = "batch_main launch failed";
-            return NDC_ERR_DEVICE;
-        }
     }
     return NDC_OK;
 }

@@ -62,6 +62,8 @@ NDC_TILE_SHAPE(0, 10, 2, 5, NDC_B(0, 0, 0, 0, 0), NDC_B(2, 2, 2, 2, 2), NDC_B(16
                NDC_B(7, 0, 14, 14, 0, 0))
 NDC_TILE_SHAPE(0, 12, 3, 4, NDC_B(0, 0, 0, 0), NDC_B(3, 3, 3, 3), NDC_B(8, 17, 17, 3, 0, 0, 30),
                NDC_B(9, 1, 0, 0, 15, 0, 2, 0))
+NDC_TILE_SHAPE(0, 13, 3, 5, NDC_B(0, 0, 0, 0, 0), NDC_B(3, 3, 2, 2, 3), NDC_B(9, 29, 0, 0, 5, 0, 11, 0),
+               NDC_B(2, 0, 8, 0, 0, 4, 0, 1, 0))
 NDC_TILE_SHAPE(0, 14, 4, 4, NDC_B(0, 0, 0, 0), NDC_B(4, 4, 4, 2), NDC_B(0, 0, 16, 1, 8, 4, 2, 0, 0),
                NDC_B(0, 0, 0, 8, 1, 8, 2, 4, 0, 2))
 NDC_TILE_SHAPE(6, 6, 3, 4, NDC_B(3, 0, 3, 0), NDC_B(0, 3, 0, 3), NDC_B(8, 17, 17, 3, 0, 0, 30),

@@ -149,6 +149,7 @@ std::vector<double> tile_twiddles(int lh, int lw, int lp) {
     switch ((lh * 16 + lw) * 8 + lp) {
         case (0 * 16 + 10) * 8 + 2: return twiddles_of<0, 10, 2>();
         case (0 * 16 + 12) * 8 + 3: return twiddles_of<0, 12, 3>();
+        case (0 * 16 + 13) * 8 + 3: return twiddles_of<0, 13, 3>();
         case (0 * 16 + 14) * 8 + 4: return twiddles_of<0, 14, 4>();
         case (5 * 16 + 5) * 8 + 2: return twiddles_of<5, 5, 2>();
         case (6 * 16 + 6) * 8 + 3: return twiddles_of<6, 6, 3>();
