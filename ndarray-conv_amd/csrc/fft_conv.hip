@@ -79,6 +79,10 @@ struct LinePlan {
 __host__ __device__ __forceinline__ int pp(int t) { return t; }
 // LDS slots a line of L elements spans in that layout.
 __host__ __device__ __forceinline__ int pp_len(int L) { return L; }
+// The padded layout, one spare slot after every 16 elements, of the buffer
+// that a first stage writes and the second reads (line_fft_kernel).
+__host__ __device__ __forceinline__ int pd(int t) { return t + (t >> 4); }
+__host__ __device__ __forceinline__ int pd_len(int L) { return L + (L >> 4); }
 
 // ---------------------------------------------------------------------------
 // Stockham stages over lines in LDS: element (line b, index t) at b*ls + pp(t)*es.
@@ -2035,9 +2039,7 @@ struct LineFftArgs {
     int64_t outer, inner;
     int32_t n;           // elements along the axis: complex length (c2c) or real length F (r2c, c2r)
     int32_t H;           // F/2 + 1 (r2c, c2r)
-    int32_t mode;        // 0 c2c, 1 r2c, 2 c2r
     int32_t Ct;          // lines per block: along inner (columns) or consecutive rows (inner == 1)
-    int32_t inv;
     int32_t ntiles;      // column tiles per outer index
     int32_t nblocks;     // grid size
     R scale;
@@ -2051,147 +2053,451 @@ struct LineFftArgs {
     // processor's axis rotation fused into its first inverse or last forward
     // transform instead of a transpose pass
     int32_t in_lines, out_lines;
+    int32_t fused;       // the first stage reads global memory (see line_fft_kernel)
+    int32_t fused_last;  // and the last writes it
+    int32_t staged;      // twiddles staged in LDS
+    int32_t ls, lsd;     // slots between lines, in the padded buffer lsd
+    // bytes between the lines and the transformed points of the input and output
+    uint32_t in_line, in_step, out_line, out_step;
     LinePlan<R> pl;      // complex length transformed: F/2 for even real lines, else n
 };
 
-template <typename R>
+// What a line transform's first stage reads and its last writes.
+enum LineKind { kColsFwd, kColsInv, kRowsFwd, kRowsInv, kRealFwd, kRealInv };
+
+template <typename R, int KIND>
+struct LineIo {
+    using C = Cx<R>;
+    static constexpr bool kCols = KIND <= kColsInv;
+    static constexpr bool kInv = KIND == kColsInv || KIND == kRowsInv || KIND == kRealInv;
+    const LineFftArgs<R>& a;
+    int64_t first;    // index of the block's first line: inner index, or row
+    int64_t base;     // its element 0 (columns)
+    int64_t o;        // outer index (columns)
+    int lines;        // lines the array has of the block's
+    bool half;        // an even real line, transformed at half its length
+    const char* src;  // the block's first element, in and out
+    char* dst;
+
+    __device__ __forceinline__ C load(int b, int j) const {
+        if (b >= lines) return cmake<C>(R(0), R(0));
+        if constexpr (kCols) {
+            return a.in_lines ? a.in[(o * a.inner + first + b) * a.n + j] : a.in[base + int64_t(j) * a.inner + b];
+        } else if constexpr (KIND == kRealFwd) {
+            const R* x = a.rin + (first + b) * a.n;
+            return half ? cmake<C>(x[2 * j], x[2 * j + 1]) : cmake<C>(x[j], R(0));
+        } else if constexpr (KIND == kRealInv) {
+            // bins of the full (odd) or half-length (even) inverse
+            const C* X = a.in + (first + b) * a.H;
+            if (half) {
+                C A = X[j], B = cconj(X[a.pl.L - j]);
+                if (j == 0) {   // imaginary parts of DC and Nyquist are ignored
+                    A.y = R(0);
+                    B.y = R(0);
+                }
+                return c2r_pre(A, B, j, a.pl.tw + a.pl.post);
+            }
+            C Y = j < a.H ? X[j] : cconj(X[a.n - j]);
+            if (j == 0) Y.y = R(0);
+            return Y;
+        } else {
+            return *reinterpret_cast<const C*>(src + (uint32_t(b) * a.in_line + uint32_t(j) * uint32_t(sizeof(C))));
+        }
+    }
+    __device__ __forceinline__ void store(int b, int j, C v) const {
+        if (b >= lines) return;
+        if constexpr (kCols) {
+            v = cscale(v, a.scale);
+            if (a.twN) {
+                const C w = a.twN[int64_t(j) * ((first + b) / a.tw_inner)];
+                v = cmul(v, kInv ? cconj(w) : w);
+            }
+            if (a.out_lines) a.out[(o * a.inner + first + b) * a.n + j] = v;
+            else a.out[base + int64_t(j) * a.inner + b] = v;
+        } else if constexpr (KIND == kRealInv) {
+            R* y = a.rout + (first + b) * a.n;
+            if (half) {
+                y[2 * j] = v.x * a.scale;
+                y[2 * j + 1] = v.y * a.scale;
+            } else {
+                y[j] = v.x * a.scale;
+            }
+        } else {
+            *reinterpret_cast<C*>(dst + (uint32_t(b) * a.out_line + uint32_t(j) * uint32_t(sizeof(C)))) = cscale(v, a.scale);
+        }
+    }
+};
+
+// Item `it` of a stage: line b and butterfly (or element) j, the lines fastest
+// for columns (a power of two of them).
+template <bool COLS>
+__device__ __forceinline__ void line_item(int it, int n, int nlines, float rn, int* b, int* j) {
+    if (COLS) {
+        *j = it >> __builtin_ctz(unsigned(nlines));
+        *b = it & (nlines - 1);
+    } else if (nlines == 1) {
+        *b = 0;
+        *j = it;
+    } else {
+        *b = fdiv(it, n, rn);
+        *j = it - *b * n;
+    }
+}
+
+// 8 bytes of two reals that need not be aligned to 8.
+typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
+typedef double f64x2u __attribute__((ext_vector_type(2), aligned(8)));
+__device__ __forceinline__ float2 load_pair(const char* p, float) {
+    const f32x2u v = *reinterpret_cast<const f32x2u*>(p);
+    return cmake<float2>(v.x, v.y);
+}
+__device__ __forceinline__ double2 load_pair(const char* p, double) {
+    const f64x2u v = *reinterpret_cast<const f64x2u*>(p);
+    return cmake<double2>(v.x, v.y);
+}
+__device__ __forceinline__ void store_pair(char* p, float2 v) { *reinterpret_cast<f32x2u*>(p) = f32x2u{v.x, v.y}; }
+__device__ __forceinline__ void store_pair(char* p, double2 v) { *reinterpret_cast<f64x2u*>(p) = f64x2u{v.x, v.y}; }
+
+// First stage, from global memory: its P points are a butterfly's loads, each
+// at a uniform base plus the thread's 32-bit offset.
+template <typename R, int P, int KIND>
+__device__ __forceinline__ void stage_first(const LineIo<R, KIND>& io, Cx<R>* dst, int nlines, int ls, int T) {
+    using C = Cx<R>;
+    using Io = LineIo<R, KIND>;
+    const LineFftArgs<R>& a = io.a;
+    const int nbf = a.pl.L / P;
+    const float rn = 1.0f / float(nbf);
+    for (int it = threadIdx.x; it < nbf * nlines; it += T) {
+        int b, j;
+        line_item<Io::kCols>(it, nbf, nlines, rn, &b, &j);
+        const int bl = b < io.lines ? b : io.lines - 1;   // lines past the last are not stored
+        C v[P];
+        if constexpr (KIND == kRealInv) {
+            const char* X = reinterpret_cast<const char*>(a.in + io.first * a.H);
+            const char* W = reinterpret_cast<const char*>(a.pl.tw + a.pl.post);
+            const uint32_t row = uint32_t(bl) * a.in_line, up = uint32_t(j) * uint32_t(sizeof(C));
+            const uint32_t down = row + uint32_t(a.pl.L - j) * uint32_t(sizeof(C));
+            C B[P], w[P];
+#pragma unroll
+            for (int r = 0; r < P; ++r) {
+                const size_t step = size_t(r) * nbf * sizeof(C);
+                v[r] = *reinterpret_cast<const C*>(X + step + (row + up));
+                B[r] = *reinterpret_cast<const C*>(X - step + down);
+                w[r] = *reinterpret_cast<const C*>(W + step + up);
+            }
+            if (j == 0) {   // imaginary parts of DC and Nyquist are ignored
+                v[0].y = R(0);
+                B[0].y = R(0);
+            }
+#pragma unroll
+            for (int r = 0; r < P; ++r) v[r] = c2r_pre(v[r], cconj(B[r]), 0, &w[r]);
+        } else {
+            const uint32_t off = uint32_t(bl) * a.in_line + uint32_t(j) * a.in_step;
+            const size_t step = size_t(nbf) * a.in_step;
+#pragma unroll
+            for (int r = 0; r < P; ++r) {
+                const char* p = io.src + size_t(r) * step;
+                if constexpr (KIND == kRealFwd) v[r] = load_pair(p + off, R(0));
+                else v[r] = *reinterpret_cast<const C*>(p + off);
+            }
+        }
+        bfly<P>(v, Io::kInv);
+        C* d = dst + b * ls;
+        if constexpr ((P & (P - 1)) == 0) {
+            d += pd(j * P);
+#pragma unroll
+            for (int r = 0; r < P; ++r) d[r] = v[r];
+        } else {
+#pragma unroll
+            for (int r = 0; r < P; ++r) d[pd(j * P + r)] = v[r];
+        }
+    }
+}
+
+// The P points of a butterfly in LDS, n slots apart.
+template <int P, bool PADDED, typename C>
+__device__ __forceinline__ void read_points(C* v, const C* s, int j, int n) {
+    if (PADDED && (n & 15) == 0) {   // uniform
+        s += pd(j);
+        const int step = pd(n);
+#pragma unroll
+        for (int r = 0; r < P; ++r) v[r] = s[r * step];
+    } else {
+#pragma unroll
+        for (int r = 0; r < P; ++r) v[r] = s[PADDED ? pd(j + r * n) : j + r * n];
+    }
+}
+
+// A stage between the first and the last.
+template <typename R, int P, int KIND, bool PADDED>
+__device__ __forceinline__ void stage_middle(const LineIo<R, KIND>& io, const Cx<R>* src, Cx<R>* dst, int Ns, int nlines,
+                                             int sls, int ls, const Cx<R>* twb, int T) {
+    using C = Cx<R>;
+    using Io = LineIo<R, KIND>;
+    const int nbf = io.a.pl.L / P;
+    const float rn = 1.0f / float(nbf), rns = 1.0f / float(Ns);
+    for (int it = threadIdx.x; it < nbf * nlines; it += T) {
+        int b, j;
+        line_item<Io::kCols>(it, nbf, nlines, rn, &b, &j);
+        const int q = (Ns & (Ns - 1)) == 0 ? j >> __builtin_ctz(unsigned(Ns)) : fdiv(j, Ns, rns);
+        const int k = j - q * Ns;
+        C v[P], w[P];
+        read_points<P, PADDED>(v, src + b * sls, j, nbf);
+#pragma unroll
+        for (int r = 1; r < P; ++r) w[r] = twb[k + (r - 1) * Ns];
+        __builtin_amdgcn_sched_barrier(0);   // all reads before the arithmetic
+#pragma unroll
+        for (int r = 1; r < P; ++r) v[r] = cmulc(v[r], w[r], Io::kInv);
+        bfly<P>(v, Io::kInv);
+        C* d = dst + b * ls + q * Ns * P + k;
+#pragma unroll
+        for (int r = 0; r < P; ++r) d[r * Ns] = v[r];
+    }
+}
+
+// Last stage, to global memory, of r2c to LDS (and the barrier before it, behind
+// which the twiddles of a thread's first butterfly travel).
+template <typename R, int P, int KIND, bool PADDED>
+__device__ __forceinline__ void stage_last(const LineIo<R, KIND>& io, const Cx<R>* src, Cx<R>* dst, int nlines, int ls,
+                                           int dls, const Cx<R>* twg, int T) {
+    using C = Cx<R>;
+    using Io = LineIo<R, KIND>;
+    const LineFftArgs<R>& a = io.a;
+    const int nbf = a.pl.L / P;
+    const float rn = 1.0f / float(nbf);
+    C w[P];
+    auto twiddles = [&](int it, int* b, int* j) {
+        line_item<Io::kCols>(it, nbf, nlines, rn, b, j);
+        if (it < nbf * nlines) {
+#pragma unroll
+            for (int r = 1; r < P; ++r)
+                w[r] = *reinterpret_cast<const C*>(reinterpret_cast<const char*>(twg + (r - 1) * nbf) + uint32_t(*j) * sizeof(C));
+        }
+    };
+    int b, j;
+    twiddles(threadIdx.x, &b, &j);
+    __syncthreads();
+    for (int it = threadIdx.x; it < nbf * nlines; it += T) {
+        if (it != int(threadIdx.x)) twiddles(it, &b, &j);
+        C v[P];
+        read_points<P, PADDED>(v, src + b * ls, j, nbf);
+#pragma unroll
+        for (int r = 1; r < P; ++r) v[r] = cmulc(v[r], w[r], Io::kInv);
+        bfly<P>(v, Io::kInv);
+        if constexpr (KIND == kRealFwd) {
+            C* d = dst + b * dls + j;
+#pragma unroll
+            for (int r = 0; r < P; ++r) d[r * nbf] = v[r];
+            continue;
+        }
+        if (b >= io.lines) continue;
+        if (Io::kCols && a.twN) {   // all factors before the first store, which could alias them
+            const int64_t j2 = (io.first + b) / a.tw_inner;
+#pragma unroll
+            for (int r = 0; r < P; ++r) w[r] = a.twN[(j + r * nbf) * j2];
+#pragma unroll
+            for (int r = 0; r < P; ++r) v[r] = cmulc(v[r], w[r], Io::kInv);
+        }
+        const uint32_t off = uint32_t(b) * a.out_line + uint32_t(j) * a.out_step;
+        const size_t step = size_t(nbf) * a.out_step;
+#pragma unroll
+        for (int r = 0; r < P; ++r) {
+            char* p = io.dst + size_t(r) * step;
+            const C y = cscale(v[r], a.scale);
+            if constexpr (KIND == kRealInv) store_pair(p + off, y);
+            else *reinterpret_cast<C*>(p + off) = y;
+        }
+    }
+}
+
+// Line transforms of one axis.  The first stage reads global memory and the
+// last writes it, save for r2c, whose bins need two points of the spectrum each;
+// the stages between go through two LDS buffers, a line's points together.  The
+// twiddles of those are staged in LDS while the first stage's data travels; the
+// last stage's and the real lines' factors, each used once, are read where they
+// are used.  What bounds it is the instructions of one wave after another: a
+// block is all that a CU has, so a butterfly's cost is its address arithmetic
+// (uniform bases and 32-bit offsets) and its latency.  Transforms of 256 x 5120
+// reals, forward and back: 39.0 us with every stage in LDS between a copy in and
+// a copy out, 31.5 now; of 4096 x 4096 0.48 ms and 0.20.  What is left out (lines of fewer than two stages, a first or last
+// radix without a butterfly, odd real lines, offsets past 32 bits) is copied in
+// and out.
+template <typename R, int KIND>
 __global__ void __launch_bounds__(kMaxThreads) line_fft_kernel(LineFftArgs<R> a) {
     using C = Cx<R>;
+    using Io = LineIo<R, KIND>;
     extern __shared__ unsigned char smem_raw[];
-    const int L = a.pl.L;
-    const int Ct = a.Ct;
-    const int PLl = pp_len(L);   // LDS slots per line
+    const int L = a.pl.L, nst = a.pl.nst, nlines = a.Ct, T = blockDim.x;
+    const int ls = a.ls, lsd = a.lsd;
     C* tw = reinterpret_cast<C*>(smem_raw);
-    C* b0 = tw + a.pl.ntw;
-    C* b1 = b0 + PLl * Ct;
-    const int T = blockDim.x;
-    const bool inv = a.inv != 0;
-    stage_table(tw, a.pl.tw, a.pl.ntw, T);
-    if (a.inner > 1) {
-        // columns: Ct lines at consecutive inner indices, element (c, j) at pp(j)*Ct + c
-        const int64_t g = xcd_slot(blockIdx.x, a.nblocks);   // neighbouring tiles on one XCD
-        const int64_t o = g / a.ntiles;
-        const int64_t i0 = int64_t(g % a.ntiles) * Ct;
-        const int nc = int(imin64(Ct, a.inner - i0));
-        const int64_t base = o * int64_t(a.n) * a.inner + i0;
-        const float rC = 1.0f / float(Ct);
-        for (int b = threadIdx.x; b < L * Ct; b += kU * T) {
+    C* b0 = tw + a.staged;
+    C* b1 = b0 + lsd * nlines;
+    Io io{a, 0, 0, 0, 0, KIND >= kRealFwd && L * 2 == a.n, nullptr, nullptr};
+    if constexpr (Io::kCols) {
+        const int g = int(xcd_slot(blockIdx.x, a.nblocks));   // neighbouring tiles on one XCD
+        const int o = g / a.ntiles;
+        io.o = o;
+        io.first = int64_t(g - o * a.ntiles) * nlines;
+        io.base = io.o * int64_t(a.n) * a.inner + io.first;
+        io.lines = int(imin64(nlines, a.inner - io.first));
+        const int64_t whole = (io.o * a.inner + io.first) * a.n;   // of lines that are contiguous
+        io.src = reinterpret_cast<const char*>(a.in + (a.in_lines ? whole : io.base));
+        io.dst = reinterpret_cast<char*>(a.out + (a.out_lines ? whole : io.base));
+    } else {
+        io.first = int64_t(blockIdx.x) * nlines;
+        io.lines = int(imin64(nlines, a.outer - io.first));
+        io.src = KIND == kRealFwd ? reinterpret_cast<const char*>(a.rin + io.first * a.n)
+                                  : reinterpret_cast<const char*>(a.in + io.first * a.n);
+        io.dst = KIND == kRealInv ? reinterpret_cast<char*>(a.rout + io.first * a.n)
+                                  : reinterpret_cast<char*>(a.out + io.first * a.n);
+    }
+    TableStage<C> tab;
+    tab.begin(a.pl.tw, a.staged, T);
+    const float rn = 1.0f / float(L);
+    if (a.fused) {
+        switch (a.pl.rad[0]) {
+#define NDC_STAGE(PP) case PP: stage_first<R, PP, KIND>(io, b0, nlines, lsd, T); break;
+            NDC_STAGE(2) NDC_STAGE(3) NDC_STAGE(4) NDC_STAGE(5) NDC_STAGE(7)
+            case 16: if constexpr (sizeof(R) == 4) stage_first<R, 16, KIND>(io, b0, nlines, lsd, T); break;
+            default: stage_first<R, 8, KIND>(io, b0, nlines, lsd, T); break;
+#undef NDC_STAGE
+        }
+    } else {
+        for (int base = threadIdx.x; base < L * nlines; base += kU * T) {
             C v[kU];
 #pragma unroll
             for (int u = 0; u < kU; ++u) {
-                const int it = b + u * T;
-                v[u] = cmake<C>(R(0), R(0));
-                if (it < L * Ct) {
-                    const int j = fdiv(it, Ct, rC), c = it - j * Ct;
-                    if (c < nc)
-                        v[u] = a.in_lines ? a.in[(o * a.inner + i0 + c) * a.n + j] : a.in[base + int64_t(j) * a.inner + c];
-                }
+                int b, j;
+                line_item<Io::kCols>(base + u * T, L, nlines, rn, &b, &j);
+                if (base + u * T < L * nlines) v[u] = io.load(b, j);
             }
 #pragma unroll
             for (int u = 0; u < kU; ++u) {
-                const int it = b + u * T;
-                if (it < L * Ct) {
-                    const int j = fdiv(it, Ct, rC), c = it - j * Ct;
-                    b0[pp(j) * Ct + c] = v[u];
-                }
+                int b, j;
+                line_item<Io::kCols>(base + u * T, L, nlines, rn, &b, &j);
+                if (base + u * T < L * nlines) b0[b * lsd + j] = v[u];
             }
+        }
+    }
+    tab.end(tw, a.pl.tw, a.staged, T);
+    int Ns = a.pl.rad[0], cur = 0;
+    for (int s = 1; a.fused && s < nst - a.fused_last; ++s) {
+        __syncthreads();
+        const int P = a.pl.rad[s];
+        const C* src = cur ? b1 : b0;
+        C* dst = cur ? b0 : b1;
+        const int sls = cur ? ls : lsd, dls = cur ? lsd : ls;
+        const C* twb = tw + a.pl.base[s];
+        switch (P) {
+#define NDC_STAGE(PP)                                                                                      \
+    case PP:                                                                                               \
+    if (s == 1) stage_middle<R, PP, KIND, true>(io, src, dst, Ns, nlines, sls, dls, twb, T);           \
+    else stage_middle<R, PP, KIND, false>(io, src, dst, Ns, nlines, sls, dls, twb, T);                 \
+    break;
+            NDC_STAGE(2)
+            NDC_STAGE(3)
+            NDC_STAGE(4)
+            NDC_STAGE(5)
+            NDC_STAGE(7)
+            case 16:
+                if constexpr (sizeof(R) == 4) {
+                    if (s == 1) stage_middle<R, 16, KIND, true>(io, src, dst, Ns, nlines, sls, dls, twb, T);
+                    else stage_middle<R, 16, KIND, false>(io, src, dst, Ns, nlines, sls, dls, twb, T);
+                }
+                break;
+            case 8:
+                if (s == 1) stage_middle<R, 8, KIND, true>(io, src, dst, Ns, nlines, sls, dls, twb, T);
+                else stage_middle<R, 8, KIND, false>(io, src, dst, Ns, nlines, sls, dls, twb, T);
+                break;
+            default:   // past the second stage; the buffers' lines are equally far apart
+                stage_generic<R, false, Io::kInv>(src, dst, L, Ns, P, nlines, ls, 1, twb, tw + a.pl.wp[s], T);
+                break;
+#undef NDC_STAGE
+        }
+        cur ^= 1;
+        Ns *= P;
+    }
+    if (!a.fused) {   // both buffers' lines are ls slots apart
+        __syncthreads();
+        cur = fft_lines_dir<R, false, Io::kInv>(b0, b1, a.pl, tw, nlines, ls, 1, T);
+    }
+    const C* res = cur ? b1 : b0;
+    int rls = cur ? ls : lsd;
+    if (a.fused_last) {
+        C* dst = cur ? b0 : b1;
+        const int dls = cur ? lsd : ls;
+        const C* twg = a.pl.tw + a.pl.base[nst - 1];
+        switch (a.pl.rad[nst - 1]) {
+#define NDC_STAGE(PP)                                                                \
+    case PP:                                                                         \
+        if (nst == 2) stage_last<R, PP, KIND, true>(io, res, dst, nlines, rls, dls, twg, T);   \
+        else stage_last<R, PP, KIND, false>(io, res, dst, nlines, rls, dls, twg, T);           \
+        break;
+            NDC_STAGE(2)
+            NDC_STAGE(3)
+            NDC_STAGE(4)
+            NDC_STAGE(5)
+            NDC_STAGE(7)
+            case 16:
+                if constexpr (sizeof(R) == 4) {
+                    if (nst == 2) stage_last<R, 16, KIND, true>(io, res, dst, nlines, rls, dls, twg, T);
+                    else stage_last<R, 16, KIND, false>(io, res, dst, nlines, rls, dls, twg, T);
+                }
+                break;
+            default:
+                if (nst == 2) stage_last<R, 8, KIND, true>(io, res, dst, nlines, rls, dls, twg, T);
+                else stage_last<R, 8, KIND, false>(io, res, dst, nlines, rls, dls, twg, T);
+                break;
+#undef NDC_STAGE
+        }
+        if constexpr (KIND != kRealFwd) return;
+        res = dst;
+        rls = dls;
+    }
+    if constexpr (KIND == kRealFwd) {
+        if (io.half) {
+            // bins k and L - k of each line from the same two points:
+            // X[L - k] = conj(E - W^k O) where X[k] = E + W^k O
+            const int half = L / 2 + 1, total = half * nlines;
+            const C* wpost = a.pl.tw + a.pl.post;
+            const float rh = 1.0f / float(half);
+            C w[kU];   // travel behind the barrier
+#pragma unroll
+            for (int u = 0; u < kU; ++u) {
+                int b, k;
+                line_item<false>(threadIdx.x + u * T, half, nlines, rh, &b, &k);
+                if (int(threadIdx.x) + u * T < total) w[u] = wpost[k];
+            }
+            __syncthreads();
+            auto bins = [&](int it, C wk, bool have) {
+                int b, k;
+                line_item<false>(it, half, nlines, rh, &b, &k);
+                if (it >= total || b >= io.lines) return;
+                if (!have) wk = wpost[k];
+                const C* Z = res + b * rls;
+                const C zk = Z[k], zm = cconj(Z[k == 0 ? 0 : L - k]);
+                const C e = cscale(cadd(zk, zm), R(0.5));
+                const C t = cmul(cmul_negi(cscale(csub(zk, zm), R(0.5))), wk);
+                C* y = a.out + (io.first + b) * a.H;
+                y[k] = cscale(cadd(e, t), a.scale);
+                y[L - k] = cscale(cconj(csub(e, t)), a.scale);
+            };
+#pragma unroll
+            for (int u = 0; u < kU; ++u) bins(threadIdx.x + u * T, w[u], true);
+            for (int it = threadIdx.x + kU * T; it < total; it += T) bins(it, w[0], false);
+            return;
         }
         __syncthreads();
-        const C* res = fft_lines<R, true>(b0, b1, a.pl, tw, Ct, 1, Ct, inv, T) ? b1 : b0;
-        for (int it = threadIdx.x; it < L * Ct; it += T) {
-            const int j = fdiv(it, Ct, rC), c = it - j * Ct;
-            if (c >= nc) continue;
-            C v = cscale(res[pp(j) * Ct + c], a.scale);
-            if (a.twN) {
-                const int64_t j2 = (i0 + c) / a.tw_inner;
-                const C w = a.twN[int64_t(j) * j2];
-                v = cmul(v, inv ? cconj(w) : w);
-            }
-            if (a.out_lines) a.out[(o * a.inner + i0 + c) * a.n + j] = v;
-            else a.out[base + int64_t(j) * a.inner + c] = v;
-        }
-        return;
-    }
-    // rows: Ct consecutive rows, element (b, j) at b*PLl + pp(j)
-    const int64_t r0 = int64_t(blockIdx.x) * Ct;
-    const int nr = int(imin64(Ct, a.outer - r0));
-    const bool half = a.mode != 0 && L * 2 == a.n;   // even real line: half-length transform
-    const int tot = L * Ct;
-    const float rL = 1.0f / float(L);
-    // the c2r load reads the post-processing factors that other threads staged
-    if (a.mode == 2) __syncthreads();
-    for (int b = threadIdx.x; b < tot; b += kU * T) {
-        C v[kU];
-#pragma unroll
-        for (int u = 0; u < kU; ++u) {
-            const int it = b + u * T;
-            v[u] = cmake<C>(R(0), R(0));
-            if (it < tot) {
-                const int rb = fdiv(it, L, rL), j = it - rb * L;
-                if (rb < nr) {
-                    const int64_t row = r0 + rb;
-                    if (a.mode == 0) {
-                        v[u] = a.in[row * a.n + j];
-                    } else if (a.mode == 1) {
-                        const R* x = a.rin + row * a.n;
-                        v[u] = half ? cmake<C>(x[2 * j], x[2 * j + 1]) : cmake<C>(x[j], R(0));
-                    } else {
-                        // c2r: bins of the full (odd) or half-length (even) inverse
-                        const C* X = a.in + row * a.H;
-                        if (half) {
-                            const int M = L;
-                            C A = X[j], B = cconj(X[M - j]);
-                            if (j == 0) {   // imaginary parts of DC and Nyquist are ignored
-                                A.y = R(0);
-                                B.y = R(0);
-                            }
-                            v[u] = c2r_pre(A, B, j, tw + a.pl.post);
-                        } else {
-                            C Y = j < a.H ? X[j] : cconj(X[a.n - j]);
-                            if (j == 0) Y.y = R(0);
-                            v[u] = Y;
-                        }
-                    }
-                }
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < kU; ++u) {
-            const int it = b + u * T;
-            if (it < tot) {
-                const int rb = fdiv(it, L, rL), j = it - rb * L;
-                b0[rb * PLl + pp(j)] = v[u];
-            }
-        }
-    }
-    __syncthreads();
-    const C* res = fft_lines<R, false>(b0, b1, a.pl, tw, Ct, PLl, 1, inv, T) ? b1 : b0;
-    if (a.mode == 0) {
-        for (int it = threadIdx.x; it < tot; it += T) {
-            const int rb = fdiv(it, L, rL), j = it - rb * L;
-            if (rb < nr) a.out[(r0 + rb) * a.n + j] = cscale(res[rb * PLl + pp(j)], a.scale);
-        }
-    } else if (a.mode == 1) {
-        const int Hb = a.H;
-        for (int it = threadIdx.x; it < Ct * Hb; it += T) {
-            const int rb = it / Hb, k = it - rb * Hb;
-            if (rb >= nr) continue;
-            const C* Z = res + rb * PLl;
-            const C X = half ? r2c_bin(Z, L, k, tw + a.pl.post) : Z[pp(k)];
-            a.out[(r0 + rb) * Hb + k] = cscale(X, a.scale);
+        for (int it = threadIdx.x; it < nlines * a.H; it += T) {
+            const int b = it / a.H, k = it - b * a.H;
+            if (b < io.lines) a.out[(io.first + b) * a.H + k] = cscale(res[b * rls + k], a.scale);
         }
     } else {
-        for (int it = threadIdx.x; it < tot; it += T) {
-            const int rb = fdiv(it, L, rL), j = it - rb * L;
-            if (rb >= nr) continue;
-            R* y = a.rout + (r0 + rb) * a.n;
-            const C zj = res[rb * PLl + pp(j)];
-            if (half) {
-                y[2 * j] = zj.x * a.scale;
-                y[2 * j + 1] = zj.y * a.scale;
-            } else {
-                y[j] = zj.x * a.scale;
-            }
+        __syncthreads();
+        for (int it = threadIdx.x; it < L * nlines; it += T) {
+            int b, j;
+            line_item<Io::kCols>(it, L, nlines, rn, &b, &j);
+            io.store(b, j, res[b * rls + j]);
         }
     }
 }
@@ -2355,41 +2661,89 @@ ndc_status line_fft(LaunchContext& ctx, int mode, bool inv, const void* in, void
     a.inner = inner;
     a.n = n;
     a.H = n / 2 + 1;
-    a.mode = mode;
-    a.inv = inv ? 1 : 0;
     a.scale = scale;
     a.twN = twN;
     a.tw_inner = tw_inner;
     a.in_lines = (io & kInLines) ? 1 : 0;
     a.out_lines = (io & kOutLines) ? 1 : 0;
+    const LineKind kind = mode == 1 ? kRealFwd : mode == 2 ? kRealInv
+                          : inner > 1 ? (inv ? kColsInv : kColsFwd) : inv ? kRowsInv : kRowsFwd;
+    const int nst = a.pl.nst;
+    auto butterfly = [&](int P) { return fixed_radix(P) && (P != 16 || sizeof(R) == 4); };
     const size_t es = sizeof(C);
+    const uint64_t row = uint64_t(n) * (mode ? sizeof(R) : es), col = uint64_t(inner) * es;
+    const bool cols = kind <= kColsInv;
+    const uint64_t in_step = cols && !a.in_lines ? col : es, out_step = cols && !a.out_lines ? col : es;
+    a.in_step = uint32_t(in_step);
+    a.out_step = uint32_t(out_step);
+    a.in_line = uint32_t(cols && !a.in_lines ? es : kind == kRealInv ? uint64_t(a.H) * es : row);
+    a.out_line = uint32_t(cols && !a.out_lines ? es : row);
+    // a butterfly's points are at most half a line apart, 16 lines are in a block
+    const bool near = uint64_t(L) / 2 * std::max(in_step, out_step) + 16 * (row + es) < (uint64_t(1) << 32);
+    a.fused = near && nst >= 2 && butterfly(a.pl.rad[0]) && butterfly(a.pl.rad[1]) && (mode == 0 || half);
+    a.fused_last = a.fused && butterfly(a.pl.rad[nst - 1]);
     const size_t lds = ctx.max_lds();
+    a.staged = a.fused_last ? a.pl.base[nst - 1] : a.pl.post >= 0 ? a.pl.post : a.pl.ntw;
+    if (a.fused && (size_t(a.staged) + size_t(pd_len(L)) * 2) * es > lds) a.fused = a.fused_last = 0;
+    if (!a.fused) a.staged = a.pl.post >= 0 ? a.pl.post : a.pl.ntw;
+    // Slots of a line in the two buffers, the second where a stage writes it.
+    // Lines 64 / Ct slots apart modulo the 32 of the banks: the lanes of a wave,
+    // which take 64 / Ct points each of Ct lines, touch every bank twice.
+    auto slots = [&](int len, int ct) { return ct == 1 ? len : len + ((64 / ct - len) % 32 + 32) % 32; };
+    const bool two = !a.fused_last || nst > 2 || kind == kRealFwd;
+    const int len0 = a.fused ? pd_len(L) : L, len1 = a.fused_last ? L : len0;
+    auto smem_of = [&](int ct) {
+        return (size_t(a.staged) + size_t(slots(len0, ct) + (two ? slots(len1, ct) : 0)) * ct) * es;
+    };
     int Ct = 1;
     int64_t blocks = 0;
     if (inner > 1) {
-        Ct = int(std::min<int64_t>(16, inner));
-        while (Ct > 1 && (size_t(a.pl.ntw) + size_t(2) * pp_len(L) * Ct) * es > lds) Ct /= 2;
+        Ct = inner >= 16 ? 16 : inner >= 8 ? 8 : inner >= 4 ? 4 : 2;
+        while (Ct > 1 && smem_of(Ct) > lds) Ct /= 2;
+        // down to 32 bytes of consecutive lines where CUs would be left with less
+        // than two blocks of a small array (256 x 2561 bins, 5 MB, forward and back:
+        // 38.7 us at 16 lines, 36.0 at 8, 34.2 at 4; a pass over 13 MB in lines of 250
+        // to 400 took 14 us at 16 and 20 at 4)
+        const bool small = outer * inner * int64_t(n) * int64_t(es) <= int64_t(8) << 20;
+        while (small && Ct > 4 && outer * ((inner + Ct - 1) / Ct) < 2 * ctx.cu_count()) Ct /= 2;
         a.ntiles = int32_t((inner + Ct - 1) / Ct);
         blocks = outer * a.ntiles;
     } else {
         Ct = int(std::max<int64_t>(1, std::min<int64_t>(kMaxLpb, 512 / std::max(1, L))));
-        while (Ct > 1 && (size_t(a.pl.ntw) + size_t(2) * pp_len(L) * Ct) * es > lds) Ct /= 2;
+        while (Ct > 1 && smem_of(Ct) > lds) Ct /= 2;
         blocks = (outer + Ct - 1) / Ct;
     }
     a.Ct = Ct;
-    const size_t smem = (size_t(a.pl.ntw) + size_t(2) * pp_len(L) * Ct) * es;
-    if (smem > lds || !lds_fits(ctx, reinterpret_cast<const void*>(&line_fft_kernel<R>), smem)) {
-        ctx.err = "line longer than the LDS transform supports";
-        return NDC_ERR_UNSUPPORTED;
-    }
+    a.ls = slots(len1, Ct);
+    a.lsd = slots(len0, Ct);
     if (blocks <= 0) return NDC_OK;
     a.nblocks = int32_t(blocks);
-    const double bytes = double(outer) * double(inner) * double(n) * double(es) * 2.0;
-    ctx.kbegin("fft_processor_lines", bytes, 5.0 * double(outer) * double(inner) * L * std::log2(double(std::max(2, L))));
-    NDC_LAUNCH(ctx, ctx.stream(), (line_fft_kernel<R>),
-        dim3(unsigned(blocks)), dim3(threads_for(int64_t(L) * Ct)), smem, a);
-    ctx.kend();
-    return check_launch(ctx, "processor line transform");
+    // a thread per butterfly of the smallest radix, or one for two points
+    int least = L;
+    for (int q = 0; q < nst; ++q) least = std::min(least, a.pl.rad[q]);
+    const int64_t want = int64_t(L / std::max(2, least)) * Ct;
+    const int T = a.fused_last ? int(std::max<int64_t>(128, std::min<int64_t>(kMaxThreads, (want + 63) / 64 * 64)))
+                          : threads_for(int64_t(L) * Ct);
+    const double bytes = double(outer) * double(inner) * double(n) * double(sizeof(C)) * 2.0;
+    auto go = [&](auto kernel) -> ndc_status {
+        if (smem_of(Ct) > lds || !lds_fits(ctx, reinterpret_cast<const void*>(kernel), smem_of(Ct))) {
+            ctx.err = "line longer than the LDS transform supports";
+            return NDC_ERR_UNSUPPORTED;
+        }
+        ctx.kbegin("fft_processor_lines", bytes,
+                   5.0 * double(outer) * double(inner) * L * std::log2(double(std::max(2, L))));
+        NDC_LAUNCH(ctx, ctx.stream(), kernel, dim3(unsigned(blocks)), dim3(T), smem_of(Ct), a);
+        ctx.kend();
+        return check_launch(ctx, "processor line transform");
+    };
+    switch (kind) {
+        case kColsFwd: return go(&line_fft_kernel<R, kColsFwd>);
+        case kColsInv: return go(&line_fft_kernel<R, kColsInv>);
+        case kRowsFwd: return go(&line_fft_kernel<R, kRowsFwd>);
+        case kRowsInv: return go(&line_fft_kernel<R, kRowsInv>);
+        case kRealFwd: return go(&line_fft_kernel<R, kRealFwd>);
+        default: return go(&line_fft_kernel<R, kRealInv>);
+    }
 }
 
 inline unsigned grid_for(int64_t total) {
