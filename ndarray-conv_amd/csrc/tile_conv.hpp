@@ -36,6 +36,8 @@ struct TileAxis {
 struct TileOuter {
     TileAxis a;
     TileDiv out, taps;
+    TileDiv cells;        // cells of x
+    int32_t step;         // planes of x from one cell to the next
 };
 
 constexpr int kMaxTileOuter = kMaxRank - 2;
@@ -45,10 +47,12 @@ struct TileArgs {
     const void* k;
     void* y;
     void* spec;           // kernel spectra, one per outer tap: [tap][register][thread]
+    void* xspec;          // spectra of x's tiles, [plane][tile][register][thread]; null when not kept
     const void* tw;
     uint32_t* flag;       // [0] set when an output is not finite, [1] counts the fix-up's blocks
     int32_t x_bytes, k_bytes, y_bytes;
     int32_t nouter, ntaps;
+    int32_t xitems;       // complex tiles of all planes of x
     int32_t items;        // complex tiles of the launch
     TileDiv plane_items;  // complex tiles per outer output position
     int32_t pair_w;       // real elements: a complex tile is two neighbours along w (else along h)
@@ -67,6 +71,7 @@ struct TilePlan {
     bool fills = false;      // some fill writes a constant other than zero
     TileArgs a;              // shape part; pointers unset
     size_t spec_bytes = 0;
+    size_t xspec_bytes = 0;  // rank 3 and up: kept spectra of x's tiles (0: transformed once per tap)
     size_t lds = 0;
     int threads = 0;
     // device tables of the handle the plan belongs to, looked up by the first launch

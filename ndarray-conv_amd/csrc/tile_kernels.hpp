@@ -296,10 +296,11 @@ struct TileIo {
 // or (oc) the constant that the plane consists of.
 struct OuterCell {
     int ko, xo, oc;
+    int xp;         // the plane's number in x
     double re, im;
 };
 __device__ __forceinline__ OuterCell outer_cell(const TileArgs& a, int plane, int tap) {
-    OuterCell c{0, 0, 0, 0, 0};
+    OuterCell c{0, 0, 0, 0, 0, 0};
     for (int i = a.nouter - 1; i >= 0; --i) {
         const TileOuter& o = a.outer[i];
         int pos, k;
@@ -316,6 +317,9 @@ __device__ __forceinline__ OuterCell outer_cell(const TileArgs& a, int plane, in
             }
         } else {
             c.xo += int(cell_offset(o.a, P));
+            const int rel = P - o.a.p0;
+            const int m = rel < 0 ? o.a.fa : rel >= o.a.n ? o.a.ba : 1;
+            c.xp += (m * rel + (rel < 0 ? o.a.fb : rel >= o.a.n ? o.a.bb : 0)) * o.step;
         }
     }
     if (c.oc) c.xo = 0;
@@ -424,6 +428,96 @@ __global__ void __launch_bounds__(S::T) tile_sum_kernel(TileArgs a) {
     Io::store(acc, a, buffer_of(static_cast<char*>(a.y) + yo, a.y_bytes - yo), p, t);
 }
 
+// The spectra of the kernel's outer taps (unless kept ones are given) and of
+// every plane of x, one workgroup each, for tile_acc_kernel.
+template <typename R, class S, bool CPLX>
+__global__ void __launch_bounds__(S::T) tile_fwd_kernel(TileArgs a) {
+    using C = Cx<R>;
+    using Io = TileIo<R, S, CPLX, false>;
+    using F = TileFft<R, S>;
+    extern __shared__ unsigned char smem_raw[];
+    C* lds = reinterpret_cast<C*>(smem_raw);
+    const int t = threadIdx.x, nk = a.have_spec ? 0 : a.ntaps;
+    const auto tw = F::load_tw(a.tw, t);
+    C v[S::PPT];
+    C* out;
+    if (int(blockIdx.x) < nk) {   // uniform
+        Io::load_kernel(v, a, outer_cell(a, 0, int(blockIdx.x)).ko, t);
+        out = static_cast<C*>(a.spec) + size_t(blockIdx.x) * S::N + t;
+    } else {
+        const int item = xcd_item(int(blockIdx.x) - nk, a.xitems);
+        int q, xo = 0;
+        int plane = div_by(a.plane_items, item, &q);
+        for (int i = a.nouter - 1; i >= 0; --i) {
+            int cell;
+            plane = div_by(a.outer[i].cells, plane, &cell);
+            xo += cell * a.outer[i].a.xs + a.outer[i].a.xlo;
+        }
+        Io::load(v, a, buffer_of(static_cast<const char*>(a.x) + xo, a.x_bytes - xo), tile_pair<CPLX>(a, q), t, 0,
+                 cmake<C>(R(0), R(0)));
+        out = static_cast<C*>(a.xspec) + size_t(item) * S::N + t;
+    }
+    F::forward(v, lds, tw, t);
+#pragma unroll
+    for (int r = 0; r < S::PPT; ++r) out[r * S::T] = v[r];
+}
+
+// tile_sum_kernel from kept spectra of x: a tile of x is transformed once and
+// not once for every tap and output plane that reads it, and the chain of a
+// workgroup is one transform long instead of one per tap.  For fills of zero.
+// 10x100x200, 5x11x31 taps: c64 30.6 -> 24.7 us a call, f32 35.3 -> 22.8, f64 43.6 ->
+// 28.2; 32x64x64, 9x9x9 taps, f32: 27.4 -> 19.5.
+template <typename R, class S, bool CPLX>
+__global__ void __launch_bounds__(S::T) tile_acc_kernel(TileArgs a) {
+    using C = Cx<R>;
+    extern __shared__ unsigned char smem_raw[];
+    C* lds = reinterpret_cast<C*>(smem_raw);
+    const int t = threadIdx.x;
+    int q;
+    const int plane = div_by(a.plane_items, xcd_item(int(blockIdx.x), a.items), &q);
+    const auto tw = TileFft<R, S>::load_tw(a.tw, t);
+    C acc[S::PPT], nx[S::PPT], nk[S::PPT];
+#pragma unroll
+    for (int r = 0; r < S::PPT; ++r) acc[r] = cmake<C>(R(0), R(0));
+    // loads the next tap from `tap` on whose plane is not all zero
+    auto fetch = [&](int tap) {
+        for (; tap < a.ntaps; ++tap) {
+            const OuterCell oc = outer_cell(a, plane, tap);
+            if (oc.oc) continue;
+            const C* sx = static_cast<const C*>(a.xspec) + (size_t(oc.xp) * a.plane_items.d + q) * S::N + t;
+            const C* sk = static_cast<const C*>(a.spec) + size_t(tap) * S::N + t;
+#pragma unroll
+            for (int r = 0; r < S::PPT; ++r) {
+                nx[r] = sx[r * S::T];
+                nk[r] = sk[r * S::T];
+            }
+            break;
+        }
+        return tap;
+    };
+    int tap = fetch(0);
+    while (tap < a.ntaps) {
+        C v[S::PPT], k[S::PPT];
+#pragma unroll
+        for (int r = 0; r < S::PPT; ++r) {
+            v[r] = nx[r];
+            k[r] = nk[r];
+        }
+        tap = fetch(tap + 1);
+#pragma unroll
+        for (int r = 0; r < S::PPT; ++r) acc[r] = cadd(acc[r], cmul(v[r], k[r]));
+    }
+    TileFft<R, S>::inverse(acc, lds, tw, t);
+    if (nonfinite(acc[0].x) || nonfinite(acc[0].y)) a.flag[0] = 1;
+    int yo = 0, pl = plane;
+    for (int i = a.nouter - 1; i >= 0; --i) {
+        int pos;
+        pl = div_by(a.outer[i].out, pl, &pos);
+        yo += pos * a.outer[i].a.ys;
+    }
+    TileIo<R, S, CPLX, false>::store(acc, a, buffer_of(static_cast<char*>(a.y) + yo, a.y_bytes - yo), tile_pair<CPLX>(a, q), t);
+}
+
 // Small inputs in one launch: the workgroup transforms the kernel itself
 // (unless a kept spectrum is given) and, when there is more than one, looks
 // the whole input over for non-finite values, so that no fix-up launch is
@@ -502,9 +596,14 @@ ndc_status launch_conv(const TilePlan& p, const TileArgs& a, LaunchContext& ctx)
         return NDC_ERR_UNSUPPORTED;
     }
     if (a.nouter) {
-        if constexpr (S::LH != 0 && S::LP < 4)
+        if constexpr (S::LH != 0 && S::LP < 4) {
+            if constexpr (!FILLS)
+                if (a.xspec)
+                    return go(tile_acc_kernel<R, S, CPLX>, "tile_conv_sum", a.items,
+                              double(p.xspec_bytes) + double(a.y_bytes) + double(p.spec_bytes), fft * a.items);
             return go(tile_sum_kernel<R, S, CPLX, FILLS>, "tile_conv_sum", a.items, io + double(p.spec_bytes),
                       (1.0 + a.ntaps) * fft * a.items);
+        }
         return NDC_ERR_UNSUPPORTED;
     }
     if constexpr (sizeof(R) == 8 || !(S::LH == 5 && S::LP == 3))
@@ -518,6 +617,17 @@ ndc_status launch_shape(const TilePlan& p, const TileArgs& a, int what, LaunchCo
     if (what == 1)
         return p.fills ? launch_conv<R, S, CPLX, true>(p, a, ctx) : launch_conv<R, S, CPLX, false>(p, a, ctx);
     const size_t smem = size_t(S::N) * sizeof(Cx<R>);
+    if (what == 3) {
+        if constexpr (S::LH != 0 && S::LP < 4) {
+            const int blocks = a.xitems + (a.have_spec ? 0 : a.ntaps);
+            ctx.kbegin("tile_forward", double(a.x_bytes) + double(p.xspec_bytes), 5.0 * S::N * S::LN * blocks);
+            if (!lds_fits(ctx, reinterpret_cast<const void*>(&tile_fwd_kernel<R, S, CPLX>), smem)) return NDC_ERR_UNSUPPORTED;
+            NDC_LAUNCH(ctx, ctx.stream(), (tile_fwd_kernel<R, S, CPLX>), dim3(unsigned(blocks)), dim3(S::T), smem, a);
+            ctx.kend();
+            return NDC_OK;
+        }
+        return NDC_ERR_UNSUPPORTED;
+    }
     ctx.kbegin("tile_spec", double(a.k_bytes) + double(p.spec_bytes), 5.0 * S::N * S::LN * a.ntaps);
     if (!lds_fits(ctx, reinterpret_cast<const void*>(&tile_spec_kernel<R, S, CPLX>), smem)) return NDC_ERR_UNSUPPORTED;
     NDC_LAUNCH(ctx, ctx.stream(), (tile_spec_kernel<R, S, CPLX>), dim3(unsigned(a.ntaps)), dim3(S::T), smem, a);
@@ -548,7 +658,8 @@ ndc_status launch_any(const TilePlan& p, const TileArgs& a, int what, LaunchCont
     return NDC_ERR_UNSUPPORTED;
 }
 
-// what: 0 the kernel spectra, 1 the convolution, 2 the fix-up
+// what: 0 the kernel spectra, 1 the convolution, 2 the fix-up, 3 the spectra of
+// kernel and x
 template <typename R>
 ndc_status launch_tile_r(const TilePlan& p, const TileArgs& a, bool cplx, int what, LaunchContext& ctx) {
     ndc_status s = NDC_OK;

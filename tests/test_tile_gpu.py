@@ -132,3 +132,20 @@ def test_processor_after_other_kernels(gpu, dtype):
             nc.conv_fft(x, k, nc.ConvMode.Same, nc.PaddingMode.Zeros)
             assert O.relerr(p.backward(spec), a)[0] <= (1e-5 if dtype == np.float32 else 1e-12)
     p.close()
+
+
+# outer taps from kept spectra of x's tiles (fills of zero and repeating sides, x small) and
+# transformed per tap (constant fills, x large): strides, dilation, views, several outer axes
+@pytest.mark.parametrize("pm", ["zeros", "reflect", "circular", "replicate", ("const", 0.5)])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.complex64, np.complex128])
+@pytest.mark.parametrize("shape,k,mode,dil", [((4, 40, 50), (3, 5, 7), "same", 1), ((9, 33, 31), (4, 3, 9), "full", 2),
+                                              ((7, 60, 45), (3, 9, 5), ("custom", [3, 4, 2], [2, 3, 1]), 1),
+                                              ((3, 4, 30, 41), (2, 3, 5, 6), "same", 1), ((16, 20, 20), (16, 3, 3), "valid", 1),
+                                              ((40, 200, 260), (5, 3, 3), "same", 1)])
+def test_outer_taps(gpu, dtype, shape, k, mode, dil, pm):
+    rng = np.random.default_rng(sum(shape) + sum(k))
+    x = rand_array(rng, tuple(2 * n for n in shape), dtype)[tuple(slice(None, None, -2) for _ in shape)]
+    try:
+        check(x, rand_array(rng, k, dtype), mode, pm, dil)
+    except O.OracleError:
+        pytest.skip("refused by the reference")
