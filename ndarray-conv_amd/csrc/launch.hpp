@@ -122,9 +122,11 @@ ndc_status launch_fft(const Plan& p, const void* x, const void* k, void* y, Laun
 // long for one workgroup (those plans recompute the kernel spectrum per call).
 size_t fft_kernel_spectrum_bytes(const Plan& p, LaunchContext& ctx);
 
-// Upper bound of the device memory launch_fft (without a kept spectrum)
-// requests through LaunchContext::scratch, twiddles and constant_table for
-// the plan, alignment included.
+// Upper bound of the device memory the whole-array form (without a kept
+// spectrum) requests through LaunchContext::scratch, twiddles and
+// constant_table for the plan, alignment included.  The tile form, whose
+// spectra and tables take at most 10 MB, is asked for by the same bound, so
+// that the allocation-free entry point takes and refuses what it always did.
 size_t fft_workspace_bytes(const Plan& p, size_t lds);
 
 // The processor's plain N-d transforms (processor/real.rs, complex.rs) on

@@ -758,7 +758,7 @@ class BatchPlan:
     Each pair has the semantics of one conv_fft call (conv_fft/mod.rs:113-118)
     with the shared ConvMode, PaddingMode, dilation and reverse flag.  Signals,
     kernels and outputs are packed back to back in pair order.  algo: "auto"
-    (a device-measured cost model picks FP32 direct or FP32 overlap-save FFT per
+    (a device-measured cost model picks FP32 direct or FP32 overlap-save FFT tiles per
     pair), "auto_bf16x3" (the same choice with the matrix-core direct forms:
     BF16x3 for kernels of at least 32 taps, BF16x6 below), "fft", "direct"
     (FP32), "bf16x3" (matrix cores for every eligible pair, BF16x3 or BF16x6 by
