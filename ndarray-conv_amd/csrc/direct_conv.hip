@@ -27,8 +27,8 @@ constexpr int kThreads = 256;
 constexpr int kTileX = 64;           // outputs per tile row: one wavefront
 // Largest tile height (a kernel template argument TY; kTileX * TY / kThreads
 // outputs per thread): 64 for elements up to 4 bytes, 32 for 8-byte and 16 for
-// 16-byte elements, whose wider windows would spill.  4-byte launches use 32
-// rows when 64 would leave the chip underfilled or waste rows.
+// 16-byte elements, whose wider windows would spill.  Launches that would
+// leave the chip underfilled, or waste rows, use 32 or 16.
 template <typename T> constexpr int kMaxTileY = sizeof(T) > 8 ? 16 : (sizeof(T) > 4 ? 32 : 64);
 
 // Region cells staged per thread per round (fewer for 16-byte elements, which
@@ -531,6 +531,20 @@ ndc_status launch_typed(const Plan& p, const void* x, const void* k, void* y, La
         const int64_t ntx = (a.out[ax] + kTileX - 1) / kTileX, nty = (a.out[ay] + 63) / 64;
         if (a.nouter * ntx * nty < 4 * int64_t(ctx.cu_count()) || (nty * 64 - a.out[ay]) * 10 > a.out[ay]) ty = 32;
     }
+    // Half the rows again where 32 would be mostly empty (rank 1: 3 M f64, 31 taps
+    // 401 -> 265 us), where the chip would be left without a block a CU (a block's
+    // staging and taps are what such a launch takes: 300x300 c64, 7x7 taps 14.8 ->
+    // 11.6; 500x700 f64, 31x31 72 -> 62), and for 8-byte elements and few taps
+    // while a CU has few blocks (f64, 5x5: 480x640 10.5 -> 9.0, 1000x1000 14.7 ->
+    // 12.0; c64 1000x1000, 7x7 20.3 -> 17.7).  Past that the halo rows that 16 rows
+    // stage twice as often cost more: c64 3000x3000, 7x7 91 -> 106; f64 2000x2000,
+    // 8x8 42 -> 44; 100x300x300, 3x3x3 105 -> 153; 1500x1500, 31x31 169 -> 204.
+    if (ty == 32) {
+        const int64_t ntx = (a.out[ax] + kTileX - 1) / kTileX, nty = (a.out[ay] + 31) / 32;
+        const int64_t blocks = a.nouter * ntx * nty, cus = ctx.cu_count();
+        const bool few = sizeof(T) == 8 && a.ktaps_outer == 1 && a.K[ay] * a.K[ax] <= 49 && blocks < 4 * cus;
+        if (a.out[ay] <= 16 || blocks < cus || few) ty = 16;
+    }
     // Choose the kernel chunk so that region + taps fit the LDS budget.  LDS
     // layout: the region (RY rows of RX, the staged width rounded up to odd),
     // then the taps in rows of KS (a multiple of kCX, zero-filled), 16-byte
@@ -582,8 +596,10 @@ ndc_status launch_typed(const Plan& p, const void* x, const void* k, void* y, La
                2.0 * double(p.y_numel) * double(p.k_numel));
     if (ty == kMaxTileY<T>) {
         if (!launch_tile<T, kMaxTileY<T>>(ctx, slide, a, nblocks, smem)) return NDC_ERR_UNSUPPORTED;
-    } else if constexpr (kMaxTileY<T> == 64) {
-        if (!launch_tile<T, 32>(ctx, slide, a, nblocks, smem)) return NDC_ERR_UNSUPPORTED;
+    } else if constexpr (kMaxTileY<T> > 16) {
+        const bool ok = ty == 16 ? launch_tile<T, 16>(ctx, slide, a, nblocks, smem)
+                                 : launch_tile<T, 32>(ctx, slide, a, nblocks, smem);
+        if (!ok) return NDC_ERR_UNSUPPORTED;
     }
     ctx.kend();
     hipError_t e = hipGetLastError();
