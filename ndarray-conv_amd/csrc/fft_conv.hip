@@ -2310,18 +2310,18 @@ __device__ __forceinline__ void stage_last(const LineIo<R, KIND>& io, const Cx<R
     }
 }
 
-// Line transforms of one axis.  The first stage reads global memory and the
-// last writes it, save for r2c, whose bins need two points of the spectrum each;
-// the stages between go through two LDS buffers, a line's points together.  The
+// Line transforms of one axis.  The first stage reads global memory and the last
+// writes it, save for r2c, whose bins need two points of the spectrum each; the
+// stages between go through two LDS buffers, a line's points together.  The
 // twiddles of those are staged in LDS while the first stage's data travels; the
-// last stage's and the real lines' factors, each used once, are read where they
-// are used.  What bounds it is the instructions of one wave after another: a
-// block is all that a CU has, so a butterfly's cost is its address arithmetic
-// (uniform bases and 32-bit offsets) and its latency.  Transforms of 256 x 5120
-// reals, forward and back: 39.0 us with every stage in LDS between a copy in and
-// a copy out, 31.5 now; of 4096 x 4096 0.48 ms and 0.20.  What is left out (lines of fewer than two stages, a first or last
-// radix without a butterfly, odd real lines, offsets past 32 bits) is copied in
-// and out.
+// last stage's and the real lines' factors, each used once, are read where they are
+// used.  What bounds it is the instructions of one wave after another: a block is
+// all that a CU has, so a butterfly's cost is its address arithmetic (uniform bases
+// and 32-bit offsets) and its latency.  Transforms of 256 x 5120 reals, forward and
+// back: 39.0 us with every stage in LDS between a copy in and a copy out, 30.6 now;
+// of 4096 x 4096 0.48 ms and 0.20.  What is left out (lines of fewer than two
+// stages, a first or second radix without a butterfly, odd real lines, offsets past
+// 32 bits) is copied in and out.
 template <typename R, int KIND>
 __global__ void __launch_bounds__(kMaxThreads) line_fft_kernel(LineFftArgs<R> a) {
     using C = Cx<R>;
