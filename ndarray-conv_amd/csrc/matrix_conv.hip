@@ -125,7 +125,7 @@ __global__ void __launch_bounds__(64 * NW) matrix_conv_kernel(MatArgs a) {
     constexpr bool kFloat = KIND <= kBf16x3;
     constexpr int NC = (W + 63) / 64;
     extern __shared__ __align__(16) unsigned char smem[];
-    __shared__ int32_t s_exact;
+    __shared__ int32_t s_bad[NW];   // by wave: it staged a non-finite value
     unsigned char* region = smem;                              // [plane][row][W]
     const int plane = a.NR * W * T::ESZ;
     uint32_t* taps = reinterpret_cast<uint32_t*>(smem + PL * plane);   // [KH][KWp], element bits
@@ -142,7 +142,6 @@ __global__ void __launch_bounds__(64 * NW) matrix_conv_kernel(MatArgs a) {
     const int y0 = ty * NW * R, x0 = tx * kTileX;               // first output of the phase
     const int py0 = a.ax[0].d * y0 + fy, px0 = a.ax[1].d * x0 + fx;
 
-    if (t == 0) s_exact = 0;
     const __amdgpu_buffer_rsrc_t px = buffer_of(a.x, a.x_bytes);
     // ---- the region: a wave stages every fourth row, a lane every 64th column
     uint32_t co[NC];
@@ -209,8 +208,48 @@ __global__ void __launch_bounds__(64 * NW) matrix_conv_kernel(MatArgs a) {
         if (kFloat) bad |= not_finite<KIND>(v);
         taps[i] = v;
     }
-    if (bad) s_exact = 1;
+    // every wave writes its own word, so the words need no clearing before
+    if constexpr (kFloat) {
+        const bool any = __ballot(bad) != 0;
+        if (lane == 0) s_bad[wave] = any;
+    }
     __syncthreads();
+
+    // A non-finite value makes a matrix product non-finite even where the
+    // reference's sum skips it (zero taps, the band's zeros).  Such workgroups
+    // compute their outputs as the reference does, and only so: FP32, the view's
+    // taps in row-major order, zero taps skipped, separate multiply and add
+    // (conv/mod.rs:177-197, dilation/mod.rs:34-60).
+    if constexpr (kFloat) {
+        int exact = 0;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) exact |= s_bad[w];
+        if (__builtin_amdgcn_readfirstlane(exact)) {
+            const __amdgpu_buffer_rsrc_t py = buffer_of(a.y, a.y_bytes);
+            for (int e = t; e < NW * R * kTileX; e += kThreads) {
+                const int yo = a.os[0] * (y0 + e / kTileX) + fy, xo = a.os[1] * (x0 + e % kTileX) + fx;
+                if (yo >= a.ax[0].U || xo >= a.ax[1].U) continue;
+                const int py_ = py0 + a.ax[0].d * (e / kTileX), px_ = px0 + a.ax[1].d * (e % kTileX);
+                float sum = 0.0f;
+                for (int r = 0; r < KH; ++r) {
+                    const int pr = py_ + a.ax[0].d * r;
+                    for (int c = 0; c < KW; ++c) {
+                        const float kv = __builtin_bit_cast(float, taps[r * a.KWp + c]);
+                        if (kv == 0.0f) continue;
+                        const int pc = px_ + a.ax[1].d * c;
+                        float v = __builtin_bit_cast(float, load_bits<float>(px, cell_offset(a.ax[0], pr) + cell_offset(a.ax[1], pc)));
+                        const int kr = cell_kind(a.ax[0], pr), kc = cell_kind(a.ax[1], pc);
+                        if (kc) v = a.cst[1][kc - 1];
+                        else if (kr) v = a.cst[0][kr - 1];
+                        sum = __fadd_rn(sum, __fmul_rn(v, kv));
+                    }
+                }
+                store_bits<float>(py, uint32_t(yo) * uint32_t(a.ax[0].ys) + uint32_t(xo) * uint32_t(a.ax[1].ys),
+                                  __builtin_bit_cast(uint32_t, sum));
+            }
+            return;
+        }
+    }
 
     if constexpr (KIND == kF32) {
         // copy j of a kernel row holds k[c - j] at c, so a lane of column j
@@ -372,37 +411,6 @@ __global__ void __launch_bounds__(64 * NW) matrix_conv_kernel(MatArgs a) {
                 for (int q = 0; q < T::ACC; ++q) v += uint32_t(acc[y][q][i]) << (8 * q);
                 store_bits<E>(py, yr + yc[i], v);
             }
-        }
-    }
-
-    // A non-finite value makes a matrix product non-finite even where the
-    // reference's sum skips it (zero taps, the band's zeros).  Such workgroups
-    // recompute their outputs as the reference does: FP32, the view's taps in
-    // row-major order, zero taps skipped, separate multiply and add
-    // (conv/mod.rs:177-197, dilation/mod.rs:34-60).
-    if constexpr (kFloat) {
-        if (!s_exact) return;   // written before the barrier above
-        const __amdgpu_buffer_rsrc_t py = buffer_of(a.y, a.y_bytes);
-        for (int e = t; e < NW * R * kTileX; e += kThreads) {
-            const int yo = a.os[0] * (y0 + e / kTileX) + fy, xo = a.os[1] * (x0 + e % kTileX) + fx;
-            if (yo >= a.ax[0].U || xo >= a.ax[1].U) continue;
-            const int py_ = py0 + a.ax[0].d * (e / kTileX), px_ = px0 + a.ax[1].d * (e % kTileX);
-            float sum = 0.0f;
-            for (int r = 0; r < KH; ++r) {
-                const int pr = py_ + a.ax[0].d * r;
-                for (int c = 0; c < KW; ++c) {
-                    const float kv = __builtin_bit_cast(float, taps[r * a.KWp + c]);
-                    if (kv == 0.0f) continue;
-                    const int pc = px_ + a.ax[1].d * c;
-                    float v = __builtin_bit_cast(float, load_bits<float>(px, cell_offset(a.ax[0], pr) + cell_offset(a.ax[1], pc)));
-                    const int kr = cell_kind(a.ax[0], pr), kc = cell_kind(a.ax[1], pc);
-                    if (kc) v = a.cst[1][kc - 1];
-                    else if (kr) v = a.cst[0][kr - 1];
-                    sum = __fadd_rn(sum, __fmul_rn(v, kv));
-                }
-            }
-            store_bits<float>(py, uint32_t(yo) * uint32_t(a.ax[0].ys) + uint32_t(xo) * uint32_t(a.ax[1].ys),
-                              __builtin_bit_cast(uint32_t, sum));
         }
     }
 }
