@@ -90,6 +90,7 @@ struct DirectArgs {
     // FAST staging: x from its lowest element, and the axes in byte offsets
     const void* xbase;
     int32_t x_bytes;
+    int32_t xlo;        // where the outer axes' element 0 lies: no plane starts below the lowest element
     int32_t fills;      // some fill writes a constant other than zero
     TileAxis ta[2];     // rows, columns
 };
@@ -266,7 +267,7 @@ __global__ void __launch_bounds__(kThreads) direct_conv_kernel(DirectArgs<T> a) 
         int oc_axis = -1;
         T ocval = Arith<T>::zero();
         bool ounw = false;
-        int64_t xoff = 0, koff = 0;
+        int64_t xoff = FAST ? a.xlo : 0, koff = 0;
         {
             int64_t rem = to;
             for (int e = a.No - 3; e >= 0; --e) {
@@ -510,7 +511,7 @@ ndc_status launch_typed(const Plan& p, const void* x, const void* k, void* y, La
                     (p.side[i][s].value.re != 0 || p.side[i][s].value.im != 0 || p.side[i][s].value.i != 0))
                     a.fills = 1;
         }
-        a.ta[0].xlo += int32_t(xlo);
+        a.xlo = int32_t(xlo);
     }
     a.nouter = 1;
     a.ktaps_outer = 1;
