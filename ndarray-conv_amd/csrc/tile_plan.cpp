@@ -143,8 +143,10 @@ bool tile_spans_fit(const Plan& p) {
     for (int i = 0; i < p.N; ++i) {
         if (!side_ok(p.side[i][0], p.pad[i][0], p.x_shape[i]) || !side_ok(p.side[i][1], p.pad[i][1], p.x_shape[i]))
             return false;
-        // room for the positions a tile reaches past the padded extent
-        if (p.pds[i] + (int64_t(p.dil[i]) << 14) >= kSpanMax) return false;
+        // room for the positions a tile reaches past the padded extent; a single
+        // tap may have any dilation, and direct convolution takes dilation 0
+        if (p.dil[i] < 1 || p.dil[i] >= kSpanMax >> 14 || p.pds[i] + (p.dil[i] << 14) >= kSpanMax) return false;
+        if (p.stride[i] >= kSpanMax) return false;
     }
     return true;
 }

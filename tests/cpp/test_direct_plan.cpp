@@ -2,7 +2,6 @@
 // recorded instead of made (LaunchContext::dry_run).  Arguments: dtype, then
 // "n k dilation stride" for each axis.  Prints the status, and the dynamic LDS
 // bytes, grid and block of each launch.
-#define __HIP_PLATFORM_AMD__ 1
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>

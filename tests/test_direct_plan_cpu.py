@@ -1,0 +1,43 @@
+"""Launches of direct convolutions planned on the host (tests/cpp/test_direct_plan.cpp):
+what the entry point accepts, it launches."""
+import os
+import subprocess
+
+import pytest
+
+from conftest import ROOT
+
+LIBDIR = os.path.join(ROOT, "ndarray-conv_amd", "lib")
+EXE = os.path.join(ROOT, "ndarray-conv_amd", "_build", "test_direct_plan")
+F32, F64, C128, I32 = 0, 1, 3, 6   # ndconv.h
+
+
+@pytest.fixture(scope="module")
+def exe():
+    if not os.path.exists(os.path.join(LIBDIR, "libndconv.so")):
+        pytest.skip("libndconv.so not built")
+    os.makedirs(os.path.dirname(EXE), exist_ok=True)
+    cmd = ["/opt/rocm/bin/amdclang++", "-std=c++17", "-O1", "-w", "-D__HIP_PLATFORM_AMD__", f"-I{ROOT}/include",
+           f"-I{ROOT}/ndarray-conv_amd/csrc", "-I/opt/rocm/include",
+           os.path.join(ROOT, "tests", "cpp", "test_direct_plan.cpp"), "-o", EXE, f"-L{LIBDIR}", "-lndconv",
+           "-L/opt/rocm/lib", "-lamdhip64", f"-Wl,-rpath,{LIBDIR}"]
+    subprocess.run(cmd, check=True, capture_output=True, text=True)
+    return EXE
+
+
+def launches(exe, dtype, *axes):
+    """(LDS bytes, grid, block) of each launch; axes are (n, k, dilation, stride)."""
+    r = subprocess.run([exe, str(dtype)] + [str(v) for a in axes for v in a], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, (r.returncode, r.stdout, r.stderr)
+    return [tuple(int(v) for v in line.split()[1:]) for line in r.stdout.splitlines() if line.startswith("launch")]
+
+
+@pytest.mark.parametrize("dtype", [F32, F64, I32])
+@pytest.mark.parametrize("axes", [[(100, 3, 0, 1)], [(100, 3, 1, 1), (100, 3, 0, 1)], [(100, 3, 0, 1), (100, 3, 1, 1)],
+                                  [(5, 2, 0, 1), (40, 3, 1, 1), (50, 3, 1, 1)],
+                                  # dilations of a single tap, past every offset the kernels form
+                                  [(100, 1, 1 << 16, 1), (100, 3, 1, 1)], [(100, 1, 1 << 31, 1)],
+                                  [(100, 1, 1 << 50, 1), (100, 3, 1, 1)], [(100, 1, 1 << 49, 1)]])
+def test_any_dilation_is_planned(exe, dtype, axes):
+    """conv takes dilation 0 (every tap meets the same sample) and any dilation of one tap."""
+    assert len(launches(exe, dtype, *axes)) == 1

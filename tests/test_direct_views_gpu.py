@@ -1,6 +1,6 @@
-"""Direct convolution of large views reversed along an outer axis: the planes
-of such a view start below its first element, and padding cells are still not
-read from the array."""
+"""Direct convolution away from the usual plans: large views reversed along an
+outer axis, whose planes start below the first element (padding cells are
+still not read from the array), and dilations of 0 or past every offset."""
 import numpy as np
 import pytest
 
@@ -20,3 +20,14 @@ def test_reversed_planes_of_600_mib(gpu, pm):
     mode = ("explicit", [[0, 0], [1, 1], [1, 1]], [100, 1, 1])
     got = nc.conv(x[::-1], k, conv_mode(mode), padding_mode(pm))
     np.testing.assert_array_equal(got, O.conv(x[::-1][::100], k, ("explicit", mode[1], [1, 1, 1]), pm))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.int32, np.int8])
+@pytest.mark.parametrize("shape,ks,dil", [((90,), (3,), 0), ((40, 270), (3, 4), [0, 1]), ((40, 270), (3, 4), [2, 0]),
+                                          ((40, 270), (1, 4), [1 << 50, 1]), ((4, 20, 30), (2, 3, 2), [0, 1, 0])])
+def test_any_dilation(gpu, dtype, shape, ks, dil):
+    """Dilation 0 (every tap meets the same sample) and any dilation of one tap."""
+    rng = np.random.default_rng(4)
+    x, k = rng.integers(-9, 10, shape).astype(dtype), rng.integers(-9, 10, ks).astype(dtype)
+    got = nc.conv(x, nc.with_dilation(k, dil), conv_mode("same"), padding_mode("replicate"))
+    np.testing.assert_array_equal(got, O.conv(x, k, "same", "replicate", dil))   # whole numbers: exact in every type
