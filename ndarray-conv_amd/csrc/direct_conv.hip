@@ -565,16 +565,24 @@ ndc_status launch_typed(const Plan& p, const void* x, const void* k, void* y, La
         l.total = l.to + kyc * l.ks + (a.xbase ? ((l.rx + l.ry + 1) * 4 + int64_t(sizeof(T)) - 1) / int64_t(sizeof(T)) : 0);
         return l;
     };
-    int64_t kyc = a.K[ay], kxc = a.K[ax];
-    for (;;) {
-        const size_t bytes = size_t(layout(kyc, kxc).total) * sizeof(T);
-        if (bytes <= budget || (kyc == 1 && kxc == 1)) break;
-        if (kyc >= kxc && kyc > 1) kyc = (kyc + 1) / 2;
-        else if (kxc > 1) kxc = (kxc + 1) / 2;
-        else kyc = (kyc + 1) / 2;
+    int64_t kyc = 0, kxc = 0;
+    auto choose_chunk = [&]() -> size_t {
+        kyc = a.K[ay];
+        kxc = a.K[ax];
+        for (;;) {
+            const size_t bytes = size_t(layout(kyc, kxc).total) * sizeof(T);
+            if (bytes <= budget || (kyc == 1 && kxc == 1)) return bytes;
+            if (kyc >= kxc && kyc > 1) kyc = (kyc + 1) / 2;
+            else if (kxc > 1) kxc = (kxc + 1) / 2;
+            else kyc = (kyc + 1) / 2;
+        }
+    };
+    size_t smem = choose_chunk();
+    if (a.xbase && smem > ctx.max_lds()) {   // no room for the offset tables beside the region
+        a.xbase = nullptr;
+        smem = choose_chunk();
     }
     const Layout lay = layout(kyc, kxc);
-    const size_t smem = size_t(lay.total) * sizeof(T);
     if (smem > ctx.max_lds()) {
         ctx.err = "direct convolution: stride/dilation too large for the LDS tile";
         return NDC_ERR_UNSUPPORTED;

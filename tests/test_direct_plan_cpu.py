@@ -41,3 +41,11 @@ def launches(exe, dtype, *axes):
 def test_any_dilation_is_planned(exe, dtype, axes):
     """conv takes dilation 0 (every tap meets the same sample) and any dilation of one tap."""
     assert len(launches(exe, dtype, *axes)) == 1
+
+
+@pytest.mark.parametrize("dtype,axes", [(C128, [(20, 3, 1, 1), (700, 3, 1, 10)]), (F32, [(1024, 3, 1, 1), (20480, 3, 1, 20)]),
+                                        (F64, [(1026, 3, 1, 1), (20480, 3, 1, 10)]), (C128, [(700, 3, 1, 1), (700, 1, 1, 10)])])
+def test_strides_up_to_the_lds_limit(exe, dtype, axes):
+    """Regions that fill LDS but for a few hundred bytes leave no room for the offset tables."""
+    (smem, _, _), = launches(exe, dtype, *axes)
+    assert 155 * 1024 < smem <= 159 * 1024

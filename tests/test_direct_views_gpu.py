@@ -31,3 +31,12 @@ def test_any_dilation(gpu, dtype, shape, ks, dil):
     x, k = rng.integers(-9, 10, shape).astype(dtype), rng.integers(-9, 10, ks).astype(dtype)
     got = nc.conv(x, nc.with_dilation(k, dil), conv_mode("same"), padding_mode("replicate"))
     np.testing.assert_array_equal(got, O.conv(x, k, "same", "replicate", dil))   # whole numbers: exact in every type
+
+
+def test_stride_that_fills_lds(gpu):
+    """The region of 16 rows at stride 10 leaves no room for the offset tables."""
+    rng = np.random.default_rng(5)
+    x, k = (rng.integers(-9, 10, s) + 1j * rng.integers(-9, 10, s) for s in ((20, 700), (3, 3)))
+    mode = ("explicit", [[1, 1], [1, 1]], [1, 10])
+    got = nc.conv(x.astype(np.complex128), k.astype(np.complex128), conv_mode(mode), padding_mode("circular"))
+    np.testing.assert_array_equal(got, O.conv(x, k, mode, "circular"))
