@@ -69,6 +69,11 @@ struct TilePlan {
     int lp = 0;              // log2 of the points a thread holds
     bool one = false;        // one launch: every workgroup transforms the kernel itself
     bool fills = false;      // some fill writes a constant other than zero
+    // what no tile of the sums over outer taps reads (a non-finite value there
+    // still makes every output NaN): planes of x, and taps that only meet zero fill
+    bool gaps = false, idle = false;
+    int xplanes = 0;         // planes of x
+    bool nan = false;        // a fill writes a non-finite constant: every output is NaN
     TileArgs a;              // shape part; pointers unset
     size_t spec_bytes = 0;
     size_t xspec_bytes = 0;  // rank 3 and up: kept spectra of x's tiles (0: transformed once per tap)

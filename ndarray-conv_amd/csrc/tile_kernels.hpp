@@ -20,7 +20,10 @@
 //
 // Non-finite data: the whole-array transform makes every output NaN.  Within
 // a tile the FFT spreads a non-finite value to every point, so one point per
-// thread tells; it raises a flag and the fix-up launch fills y with NaN.
+// thread tells; it raises a flag and the fix-up launch fills y with NaN.  What
+// no tile transforms is looked over apart: planes of x between the taps of a
+// stride or dilation, and kept spectra of taps that only meet zero fill
+// (tile_scan_kernel).  A non-finite pad constant is known to the host.
 #pragma once
 
 #include <algorithm>
@@ -326,7 +329,13 @@ __device__ __forceinline__ OuterCell outer_cell(const TileArgs& a, int plane, in
     return c;
 }
 
-// Kernel spectra: one workgroup per outer tap.
+__device__ __forceinline__ bool nonfinite(float v) { return (__builtin_bit_cast(uint32_t, v) & 0x7f800000u) == 0x7f800000u; }
+__device__ __forceinline__ bool nonfinite(double v) {
+    return (uint32_t(__builtin_bit_cast(uint64_t, v) >> 32) & 0x7ff00000u) == 0x7ff00000u;
+}
+
+// Kernel spectra: one workgroup per outer tap.  A kept spectrum raises no flag:
+// the calls that use it do.
 template <typename R, class S, bool CPLX>
 __global__ void __launch_bounds__(S::T) tile_spec_kernel(TileArgs a) {
     using C = Cx<R>;
@@ -337,14 +346,10 @@ __global__ void __launch_bounds__(S::T) tile_spec_kernel(TileArgs a) {
     const auto tw = TileFft<R, S>::load_tw(a.tw, t);
     TileIo<R, S, CPLX, false>::load_kernel(v, a, outer_cell(a, 0, int(blockIdx.x)).ko, t);
     TileFft<R, S>::forward(v, lds, tw, t);
+    if (!a.have_spec && (nonfinite(v[0].x) || nonfinite(v[0].y))) a.flag[0] = 1;
     C* out = static_cast<C*>(a.spec) + size_t(blockIdx.x) * S::N + t;
 #pragma unroll
     for (int r = 0; r < S::PPT; ++r) out[r * S::T] = v[r];
-}
-
-__device__ __forceinline__ bool nonfinite(float v) { return (__builtin_bit_cast(uint32_t, v) & 0x7f800000u) == 0x7f800000u; }
-__device__ __forceinline__ bool nonfinite(double v) {
-    return (uint32_t(__builtin_bit_cast(uint64_t, v) >> 32) & 0x7ff00000u) == 0x7ff00000u;
 }
 
 // One kernel spectrum, read from memory.
@@ -458,6 +463,7 @@ __global__ void __launch_bounds__(S::T) tile_fwd_kernel(TileArgs a) {
         out = static_cast<C*>(a.xspec) + size_t(item) * S::N + t;
     }
     F::forward(v, lds, tw, t);
+    if (nonfinite(v[0].x) || nonfinite(v[0].y)) a.flag[0] = 1;
 #pragma unroll
     for (int r = 0; r < S::PPT; ++r) out[r * S::T] = v[r];
 }
@@ -564,12 +570,60 @@ __global__ void __launch_bounds__(S::T) tile_one_kernel(TileArgs a) {
     Io::store(v, a, buffer_of(a.y, a.y_bytes), p, t);
 }
 
-// Fills y with NaN when a tile met a non-finite value, and clears the flag.
+// Whether some output reads cell c of an outer axis inside x.
+__device__ __forceinline__ bool cell_read(const TileOuter& o, int c) {
+    for (int k = 0; k < o.a.K; ++k) {
+        const int q = c + o.a.p0 - k * o.a.d;
+        if (q < 0) break;
+        if (q % o.a.s == 0 && q / o.a.s < int(o.out.d)) return true;
+    }
+    return false;
+}
+
+// Raises the flag for non-finite values that no tile transforms: in planes of
+// x that no outer tap reads (`planes` of them to look at, `groups` parts of
+// rows each, a part per wave at a time) and in `nspec` values of kept spectra.
+template <typename R, bool CPLX>
+__global__ void __launch_bounds__(256) tile_scan_kernel(TileArgs a, int planes, int groups, int nspec) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(int(blockIdx.x * 4 + (threadIdx.x >> 6)));
+    bool bad = false;
+    for (int64_t i = wave; i < int64_t(planes) * groups; i += int64_t(gridDim.x) * 4) {
+        int plane = int(i / groups), xo = 0;
+        const int g = int(i - int64_t(plane) * groups);
+        bool read = true;
+        for (int e = a.nouter - 1; e >= 0; --e) {
+            int cell;
+            plane = div_by(a.outer[e].cells, plane, &cell);
+            read = read && cell_read(a.outer[e], cell);
+            xo += cell * a.outer[e].a.xs + a.outer[e].a.xlo;
+        }
+        if (read) continue;
+        const __amdgpu_buffer_rsrc_t px = buffer_of(static_cast<const char*>(a.x) + xo, a.x_bytes - xo);
+        for (int r = g; r < a.ax[0].n; r += groups)
+            for (int c = lane; c < a.ax[1].n; c += 64) {
+                const uint32_t off = uint32_t(r) * uint32_t(a.ax[0].xs) + uint32_t(a.ax[0].xlo) +
+                                     uint32_t(c) * uint32_t(a.ax[1].xs) + uint32_t(a.ax[1].xlo);
+                if constexpr (CPLX) {
+                    const Cx<R> v = load_cx(px, off, R(0));
+                    bad |= nonfinite(v.x) || nonfinite(v.y);
+                } else {
+                    bad |= nonfinite(load_real<R>(px, off));
+                }
+            }
+    }
+    for (int i = int(blockIdx.x) * 256 + int(threadIdx.x); i < nspec; i += int(gridDim.x) * 256)
+        bad |= nonfinite(static_cast<const R*>(a.spec)[i]);
+    if (bad) a.flag[0] = 1;
+}
+
+// Fills y with NaN when a tile met a non-finite value, and clears the flag;
+// without a flag it fills y in any case.
 template <typename R>
 __global__ void __launch_bounds__(256) tile_nan_kernel(R* y, int64_t n, uint32_t* flag) {
-    if (__builtin_amdgcn_readfirstlane(int(flag[0])) == 0) return;
+    if (flag && __builtin_amdgcn_readfirstlane(int(flag[0])) == 0) return;
     for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < n; i += int64_t(gridDim.x) * 256)
         y[i] = R(__builtin_nanf(""));
+    if (!flag) return;
     __syncthreads();
     if (threadIdx.x == 0 && atomicAdd(&flag[1], 1u) == gridDim.x - 1) {
         flag[1] = 0;   // every block has read the flag
@@ -658,8 +712,25 @@ ndc_status launch_any(const TilePlan& p, const TileArgs& a, int what, LaunchCont
     return NDC_ERR_UNSUPPORTED;
 }
 
+// Looks over what the plan's tiles leave out: planes of x (not where every
+// plane is transformed), kept spectra of taps that no tile uses.
+template <typename R, bool CPLX>
+ndc_status launch_scan(const TilePlan& p, const TileArgs& a, LaunchContext& ctx) {
+    const int planes = p.gaps && !a.xspec ? p.xplanes : 0;
+    const int nspec = p.idle && a.have_spec ? int(p.spec_bytes / sizeof(R)) : 0;
+    if (!planes && !nspec) return NDC_OK;
+    // parts of at least a row, and 64 of them for each of 256 CUs where rows allow it
+    const int groups = std::max(1, std::min(int(a.ax[0].n), 16384 / std::max(1, planes)));
+    const int64_t waves = std::max<int64_t>(int64_t(planes) * groups, (nspec + 63) / 64);
+    ctx.kbegin("tile_scan", 0, 0);
+    NDC_LAUNCH(ctx, ctx.stream(), (tile_scan_kernel<R, CPLX>), dim3(unsigned(std::min<int64_t>((waves + 3) / 4, 4096))),
+               dim3(256), 0, a, planes, groups, nspec);
+    ctx.kend();
+    return NDC_OK;
+}
+
 // what: 0 the kernel spectra, 1 the convolution, 2 the fix-up, 3 the spectra of
-// kernel and x
+// kernel and x, 4 the look over what these leave out
 template <typename R>
 ndc_status launch_tile_r(const TilePlan& p, const TileArgs& a, bool cplx, int what, LaunchContext& ctx) {
     ndc_status s = NDC_OK;
@@ -669,6 +740,8 @@ ndc_status launch_tile_r(const TilePlan& p, const TileArgs& a, bool cplx, int wh
         ctx.kbegin("tile_nan", 0, 0);
         NDC_LAUNCH(ctx, ctx.stream(), (tile_nan_kernel<R>), dim3(grid), dim3(256), 0, static_cast<R*>(a.y), n, a.flag);
         ctx.kend();
+    } else if (what == 4) {
+        s = cplx ? launch_scan<R, true>(p, a, ctx) : launch_scan<R, false>(p, a, ctx);
     } else {
         s = cplx ? launch_any<R, true>(p, a, what, ctx) : launch_any<R, false>(p, a, what, ctx);
     }

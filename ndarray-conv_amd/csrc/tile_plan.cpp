@@ -97,6 +97,43 @@ bool const_nonzero(const ndc_border& b) {
     return side1d(b.tag) == kS1Const && (b.value.re != 0 || b.value.im != 0);
 }
 
+// A constant that is not finite in the element type.
+bool const_nonfinite(const ndc_border& b, bool cplx, bool dbl) {
+    if (side1d(b.tag) != kS1Const) return false;
+    auto bad = [&](double v) { return dbl ? !std::isfinite(v) : !std::isfinite(float(v)); };
+    return bad(b.value.re) || (cplx && bad(b.value.im));
+}
+
+// Whether no output reads some cell of x along axis i: cells between the taps
+// of a stride, or of a dilation longer than the output, and past the last
+// output.  Taken for so where looking at every cell would take the host long.
+bool axis_gaps(const Plan& p, int i) {
+    const int64_t s = p.stride[i], d = p.dil[i], K = p.k_shape[i], out = p.out[i], n = p.x_shape[i];
+    if (s == 1) return K > 1 && out < d;
+    if (n > (int64_t(1) << 20) / K) return true;
+    for (int64_t c = 0; c < n; ++c) {
+        bool read = false;
+        for (int64_t k = 0; k < K && !read; ++k) {
+            const int64_t q = c + p.pad[i][0] - k * d;
+            read = q >= 0 && q % s == 0 && q / s < out;
+        }
+        if (!read) return true;
+    }
+    return false;
+}
+
+// Whether some tap of axis i meets nothing but constant fill.
+bool axis_idle(const Plan& p, int i) {
+    const int64_t s = p.stride[i], out = p.out[i], lo = p.pad[i][0], hi = lo + p.x_shape[i];
+    const bool front = side1d(p.side[i][0].tag) != kS1Const, back = side1d(p.side[i][1].tag) != kS1Const;
+    for (int64_t k = 0; k < p.k_shape[i]; ++k) {
+        const int64_t P0 = k * p.dil[i], P1 = P0 + (out - 1) * s;   // its first and last cell
+        const int64_t in = P0 >= lo ? P0 : P0 + (lo - P0 + s - 1) / s * s;
+        if (!((in <= P1 && in < hi) || (front && P0 < lo) || (back && P1 >= hi))) return true;
+    }
+    return false;
+}
+
 }  // namespace
 
 TileDiv tile_div(int64_t d) { return TileDiv{uint32_t(d), uint32_t(d == 1 ? 0 : ((int64_t(1) << 32) + d - 1) / d)}; }
@@ -175,15 +212,26 @@ bool tile_plan(const Plan& p, size_t lds, int cus, TilePlan* t) {
     if (!tile_spans_fit(p)) return false;
     int64_t taps = 1, planes = 1, xplanes = 1;
     bool fills = false;
+    t->gaps = t->idle = t->nan = false;
     for (int i = 0; i < N; ++i) {
         if (i < h) {
             taps *= p.k_shape[i];
             planes *= p.out[i];
             xplanes *= p.x_shape[i];
         }
-        for (int s = 0; s < 2; ++s) fills = fills || (p.pad[i][s] > 0 && const_nonzero(p.side[i][s]));
+        for (int s = 0; s < 2; ++s)
+            if (p.pad[i][s] > 0) {
+                fills = fills || const_nonzero(p.side[i][s]);
+                t->nan = t->nan || const_nonfinite(p.side[i][s], cplx, dbl);
+            }
     }
     if (taps > kMaxTaps) return false;
+    for (int i = 0; i < h; ++i) {
+        t->gaps = t->gaps || axis_gaps(p, i);
+        t->idle = t->idle || (!fills && axis_idle(p, i));
+    }
+    if (t->gaps && xplanes >= kSpanMax) return false;   // a broadcast view: planes are counted in 30 bits
+    t->xplanes = t->gaps ? int(xplanes) : 0;
     const bool compact = p.x_hi - p.x_lo + 1 == p.x_numel;
     const bool one = N == 1 && p.x_numel <= kScanMax;
     if (one && !compact) return false;
@@ -301,6 +349,8 @@ ndc_status launch_tile(const Plan& p, const TilePlan& t, const void* x, const vo
     a.x = x ? static_cast<const char*>(x) + p.x_lo * int64_t(dtype_size(p.dtype)) : nullptr;
     a.k = k ? static_cast<const char*>(k) + p.k_lo * int64_t(dtype_size(p.dtype)) : nullptr;
     a.y = y;
+    if (t.nan && !(ks && ks->bake))   // without a flag: y is filled in any case
+        return dbl ? launch_tile_as<double>(t, a, cplx, 2, ctx) : launch_tile_as<float>(t, a, cplx, 2, ctx);
     if (!t.tw || !t.flag) {
         const std::string key = "tile:" + std::to_string(t.lh) + ":" + std::to_string(t.lw) + ":" + std::to_string(t.lp) + (dbl ? ":d" : ":f");
         const std::vector<double> tab = tile_twiddles(t.lh, t.lw, t.lp);
@@ -336,7 +386,8 @@ ndc_status launch_tile(const Plan& p, const TilePlan& t, const void* x, const vo
         const ndc_status s = go(t.xspec_bytes ? 3 : 0);
         if (s != NDC_OK) return s;
     }
-    ndc_status s = go(1);
+    ndc_status s = t.gaps || t.idle ? go(4) : NDC_OK;
+    if (s == NDC_OK) s = go(1);
     if (s == NDC_OK && !t.one) s = go(2);
     return s;
 }

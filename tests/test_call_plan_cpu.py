@@ -40,3 +40,22 @@ def test_call_keys_tell_values_apart():
     assert len({nc._mode_key(m) for m in modes}) == len(modes)
     with pytest.raises(TypeError):   # contents unknown: never kept
         nc._pad_key(P.Const(np.array(0.5)))
+
+
+@pytest.mark.parametrize("border", ["Zeros", "Reflect", "Replicate", "Circular"])
+def test_unread_planes_are_looked_over(border):
+    """conv_fft by tiles that are transformed per tap (x past 8 MB of spectra)
+    adds the look for non-finite values, a launch of no LDS beside the fix-up's,
+    where some plane of x meets no tap."""
+    bt = getattr(B, border)
+    for n, k, d, s, p0, p1 in [(n, k, d, s, p0, p1) for n in (24, 25, 31) for k in (1, 2, 3) for d in (1, 2, 5, 13)
+                               for s in (1, 2, 3, 7) for p0 in (0, 1, 4) for p1 in (0, 3)]:
+        if n + p0 + p1 < (k - 1) * d + 1:
+            continue
+        pm = P.Custom([bt, B.Zeros, B.Zeros])
+        mode = M.Explicit([[p0, p1], [0, 0], [0, 0]], [s, 1, 1])
+        out = nc.plan((n, 300, 260), (k, 3, 3), mode, pm, dilation=[d, 1, 1], fft=True)["out_shape"][0]
+        read = {o * s + t * d - p0 for o in range(out) for t in range(k)}
+        got = nc.fft_launch_plan((n, 300, 260), (k, 3, 3), mode, pm, dilation=[d, 1, 1])
+        if not set(range(n)) <= read:
+            assert len([g for g in got if g[0] == 0]) == 2, (n, k, d, s, p0, p1, got)
