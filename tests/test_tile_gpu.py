@@ -142,7 +142,7 @@ def test_processor_after_other_kernels(gpu, dtype):
                                               ((7, 60, 45), (3, 9, 5), ("custom", [3, 4, 2], [2, 3, 1]), 1),
                                               ((3, 4, 30, 41), (2, 3, 5, 6), "same", 1), ((16, 20, 20), (16, 3, 3), "valid", 1),
                                               ((40, 200, 260), (5, 3, 3), "same", 1)])
-def test_outer_taps(gpu, dtype, shape, k, mode, dil, pm):
+def test_outer_taps_kept_spectra(gpu, dtype, shape, k, mode, dil, pm):
     rng = np.random.default_rng(sum(shape) + sum(k))
     x = rand_array(rng, tuple(2 * n for n in shape), dtype)[tuple(slice(None, None, -2) for _ in shape)]
     try:
