@@ -13,8 +13,8 @@
 // 3.3e-6 / 1.43e-5 / 3.4e-5, a run 2.1e-6 / 1.7e-5 / 4.8e-5 more for its kernel
 // and start.  Batches before (real blocks of 512 to 8192 samples from a queue
 // with spectra from a launch before) and now: 509 pairs of up to 65536 samples
-// and 255 taps 72 -> 20 us, 4096 pairs of 153 M samples in FP32 0.73 -> 0.41 ms, 300
-// pairs with 1000 to 6000 taps 197 -> 116 us, 2000 pairs under 2000 samples 58 -> 14 us.
+// and 255 taps 72 -> 20 us, 4096 pairs of 153 M samples in FP32 0.73 -> 0.35 ms, 300
+// pairs with 1000 to 6000 taps 197 -> 105 us, 2000 pairs under 2000 samples 58 -> 14 us.
 #include <hip/hip_runtime.h>
 
 #include <cstring>
@@ -72,7 +72,7 @@ __global__ void __launch_bounds__(S::T, 4) batch_tile_kernel(BatchTileArgs a, co
     C* lds = reinterpret_cast<C*>(smem_raw);
     const int t = threadIdx.x;
     if (blockIdx.x == 0 && t < kBatchHeads) a.heads[t * kBatchQueueStride] = 0;
-    const BatchTile& it = items[tilek::xcd_item(int(blockIdx.x), n)];
+    const BatchTile& it = items[batch_run_of(int(blockIdx.x), n)];
     TileAxis ax;
     ax.n = uniform(it.n);
     ax.p0 = uniform(it.p0);

@@ -1,28 +1,17 @@
 """Launches of direct convolutions planned on the host (tests/cpp/test_direct_plan.cpp):
 what the entry point accepts, it launches."""
-import os
 import subprocess
 
 import pytest
 
-from conftest import ROOT
+from host_cpp import program
 
-LIBDIR = os.path.join(ROOT, "ndarray-conv_amd", "lib")
-EXE = os.path.join(ROOT, "ndarray-conv_amd", "_build", "test_direct_plan")
 F32, F64, C128, I32 = 0, 1, 3, 6   # ndconv.h
 
 
 @pytest.fixture(scope="module")
 def exe():
-    if not os.path.exists(os.path.join(LIBDIR, "libndconv.so")):
-        pytest.skip("libndconv.so not built")
-    os.makedirs(os.path.dirname(EXE), exist_ok=True)
-    cmd = ["/opt/rocm/bin/amdclang++", "-std=c++17", "-O1", "-w", "-D__HIP_PLATFORM_AMD__", f"-I{ROOT}/include",
-           f"-I{ROOT}/ndarray-conv_amd/csrc", "-I/opt/rocm/include",
-           os.path.join(ROOT, "tests", "cpp", "test_direct_plan.cpp"), "-o", EXE, f"-L{LIBDIR}", "-lndconv",
-           "-L/opt/rocm/lib", "-lamdhip64", f"-Wl,-rpath,{LIBDIR}"]
-    subprocess.run(cmd, check=True, capture_output=True, text=True)
-    return EXE
+    return program("test_direct_plan")
 
 
 def launches(exe, dtype, *axes):
