@@ -171,27 +171,37 @@ struct BatchForm {
     int cus, blocks;       // CUs, resident workgroups of the queue's kernel
 };
 
-// Method of a pair in the queue: kMethodDirect, kMethodMfma or kMethodMfma6.
-int queue_method(const CostModel& cm, const PairShape& ps, int s, int algo, bool repeating_border) {
+// What a pair costs in FP32 (tiles or direct items).
+double fp32_cost(const CostModel& cm, const PairShape& ps, int s, int d) {
+    double v = direct_cost(cm, ps, s);
+    for (int c = 0; c < kBatchTileClasses; ++c) v = std::min(v, tile_cost(cm, ps, d, c));
+    return v;
+}
+
+// Method of a pair in the queue: kMethodDirect, kMethodMfma or kMethodMfma6.  The
+// autotuned form admits split products only to a pair for which they cost
+// less than FP32 by its own costs: what launches the rest of the batch uses must
+// not lower a pair's precision.  (With all pairs of a batch of 4096 moved to the
+// queue together, the median error against 64 bits was 3.4e-6; FP32 tiles give 2.1e-7.)
+int queue_method(const CostModel& cm, const PairShape& ps, int s, int d, int algo, bool repeating_border) {
     const bool x3 = bf16x3_admitted(ps, repeating_border);
     if (algo == NDC_BATCH_MFMA && mfma_eligible(ps, s)) return x3 ? kMethodMfma : kMethodMfma6;
     if (algo == NDC_BATCH_BF16X6 && mfma_eligible(ps, s)) return kMethodMfma6;
-    if (algo == NDC_BATCH_AUTO_BF16X3 && mfma_cost(cm, ps, s, !x3) < direct_cost(cm, ps, s))
+    if (algo == NDC_BATCH_AUTO_BF16X3 && mfma_cost(cm, ps, s, !x3) < fp32_cost(cm, ps, s, d))
         return x3 ? kMethodMfma : kMethodMfma6;
     return kMethodDirect;
 }
 
 // Methods of all pairs: a tile class or the queue's method, whichever costs
-// less among the launches that the batch uses.  The costs are those of a full
-// chip; a launch takes about one run or item longer than its work, on a chip
-// that is part empty, so all choices of launches are compared with that added:
-// a few pairs of some length do not get a launch of their own, and a small
-// batch is one launch (509 pairs, 6.3 M outputs: 20 us in one launch of 1024-point
-// tiles, 29 us with 6 pairs in a launch of 4096-point tiles beside it; 4096 pairs, 153 M
-// outputs: 359 to 374 us in one launch of the queue, 386 to 412 us where the
-// short and the long kernels went to tiles).
-std::vector<int> choose(const CostModel& cm, const std::vector<PairShape>& sh, const BatchForm& f, int algo,
-                        bool repeating_border) {
+// less among the launches that the batch uses, and what that is estimated to
+// take.  The costs are those of a full chip; a launch takes at least as long as
+// one run on it, the queue's about one item longer than its work, and all
+// choices of launches are compared with that: a few pairs of some length do not get a
+// launch of their own, and a small batch is one launch (509 pairs, 6.3 M outputs: 20 us
+// in one launch of 1024-point tiles, 29 us with 6 pairs in a launch of 4096-point
+// tiles beside it).
+std::vector<int> choose_launches(const CostModel& cm, const std::vector<PairShape>& sh, const BatchForm& f, int algo,
+                                 bool repeating_border, double* estimate) {
     constexpr int Q = kBatchTileClasses, G = Q + 1;
     constexpr double kLaunchMs = 3e-3;
     const size_t P = sh.size();
@@ -202,7 +212,7 @@ std::vector<int> choose(const CostModel& cm, const std::vector<PairShape>& sh, c
     std::vector<double> item(P);
     for (size_t i = 0; i < P; ++i) {
         const PairShape& ps = sh[i];
-        queue[i] = m[i] = queue_method(cm, ps, f.s, algo, repeating_border);
+        queue[i] = m[i] = queue_method(cm, ps, f.s, f.d, algo, repeating_border);
         bool any = false;
         for (int c = 0; c < Q; ++c) {
             // where the queue's method is a fixed one, tiles take what it does not
@@ -220,22 +230,25 @@ std::vector<int> choose(const CostModel& cm, const std::vector<PairShape>& sh, c
     }
     double best = INFINITY;
     unsigned best_mask = 0;
-    auto pick = [&](size_t i, unsigned mask) {
-        int g = -1;
+    // the cheapest group of every set of launches (-1: none takes the pair)
+    std::vector<std::array<int8_t, 1 << G>> pick(P);
+    for (size_t i = 0; i < P; ++i) {
+        pick[i][0] = -1;
         for (int c = 0; c < G; ++c)
-            if ((mask >> c & 1) && !std::isinf(cost[i][c]) && (g < 0 || cost[i][c] < cost[i][g])) g = c;
-        return g;
-    };
-    std::vector<int> group(P);
+            for (unsigned rest = 0; rest < (1u << c); ++rest) {
+                const int g = pick[i][rest];
+                const bool lower = !std::isinf(cost[i][c]) && (g < 0 || cost[i][c] < cost[i][g]);
+                pick[i][rest | 1u << c] = lower ? int8_t(c) : int8_t(g);
+            }
+    }
     for (unsigned mask = 1; mask < (1u << G); ++mask) {
         double work = 0, longest = 0;
         int64_t total[Q] = {}, runs[Q] = {}, run[Q] = {};
         unsigned used = 0;
         bool all = true;
         for (size_t i = 0; i < P && all; ++i) {
-            group[i] = sh[i].out > 0 ? pick(i, mask) : G;
-            const int g = group[i];
-            if (g == G) continue;
+            if (sh[i].out <= 0) continue;
+            const int g = pick[i][mask];
             all = g >= 0;
             if (!all) break;
             used |= 1u << g;
@@ -248,23 +261,41 @@ std::vector<int> choose(const CostModel& cm, const std::vector<PairShape>& sh, c
         }
         if (!all || used != mask) continue;
         for (int c = 0; c < Q; ++c) run[c] = run_tiles(total[c], int64_t(f.cus) * tile_slots(c));
-        for (size_t i = 0; i < P; ++i)
-            if (group[i] < Q) runs[group[i]] += (split[i][group[i]] + run[group[i]] - 1) / run[group[i]];
+        for (size_t i = 0; i < P; ++i) {
+            const int g = pick[i][mask];
+            if (sh[i].out > 0 && g < Q) runs[g] += uint32_t(split[i][g] + run[g] - 1) / uint32_t(run[g]);
+        }
         for (int c = 0; c < Q; ++c)
             if (used >> c & 1)
-                work += cm.tile_a[c] * double(runs[c]) + cm.tile_b[c] * double(total[c]) + kLaunchMs +
-                        (cm.tile_a[c] + cm.tile_b[c] * double(run[c])) * double(f.cus * tile_slots(c));
+                work += kLaunchMs + std::max(cm.tile_a[c] * double(runs[c]) + cm.tile_b[c] * double(total[c]),
+                                             (cm.tile_a[c] + cm.tile_b[c] * double(run[c])) * double(f.cus * tile_slots(c)));
         if (used >> Q & 1) work += kLaunchMs + longest * double(f.blocks);
         if (work < best) {
             best = work;
             best_mask = mask;
         }
     }
+    *estimate = best;
     for (size_t i = 0; i < P; ++i) {
-        const int g = sh[i].out > 0 ? pick(i, best_mask) : Q;
+        const int g = sh[i].out > 0 ? pick[i][best_mask] : Q;
         m[i] = g == Q ? queue[i] : kMethodTile - g;
     }
     return m;
+}
+
+// Split products, which are less exact than FP32, have to make the batch
+// faster by more than the estimates are wrong: 4096 pairs, 153 M samples, circular,
+// take 370 to 380 us in FP32 tiles, 369 to 377 with every pair in the queue, and 375 to
+// 384 with the 1650 in it that it serves at less cost, estimated as 0.98 of FP32.
+constexpr double kSplitGain = 0.95;
+
+std::vector<int> choose(const CostModel& cm, const std::vector<PairShape>& sh, const BatchForm& f, int algo,
+                        bool repeating_border) {
+    double best = 0, fp32 = 0;
+    std::vector<int> m = choose_launches(cm, sh, f, algo, repeating_border, &best);
+    if (algo != NDC_BATCH_AUTO_BF16X3) return m;
+    std::vector<int> plain = choose_launches(cm, sh, f, NDC_BATCH_AUTO, repeating_border, &fp32);
+    return best < kSplitGain * fp32 ? m : plain;
 }
 
 struct Schedule {
