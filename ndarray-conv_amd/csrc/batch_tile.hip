@@ -199,7 +199,7 @@ ndc_status launch_class(const BatchTileArgs& a, const BatchTile* items, int n, c
 bool batch_tile_tables(LaunchContext& ctx, const void* tw[kBatchTileClasses]) {
     for (int c = 0; c < kBatchTileClasses; ++c) {
         const int lw = batch_tile_log2(c), lp = c == 0 ? 2 : c == kBatchTileFar ? 4 : 3;
-        const std::vector<double> tab = tile_twiddles(0, lw, lp);
+        const std::vector<double>& tab = tile_twiddles(0, lw, lp);
         const std::vector<float> f(tab.begin(), tab.end());
         tw[c] = ctx.constant_table("tile:0:" + std::to_string(lw) + ":" + std::to_string(lp) + ":f", f.data(),
                                    f.size() * sizeof(float));

@@ -105,8 +105,8 @@ bool tile_spans_fit(const Plan& p);
 TileDiv tile_div(int64_t d);
 void tile_axis(const Plan& p, int i, int64_t ystr, TileAxis* a);
 
-// Host table of a tile's twiddles, empty for an unknown tile.
-std::vector<double> tile_twiddles(int lh, int lw, int lp);
+// Host table of a tile's twiddles (kept for the process), empty for an unknown tile.
+const std::vector<double>& tile_twiddles(int lh, int lw, int lp);
 
 // Whether the multi-pass form can transform this plan's axes at all; what it
 // refuses stays refused.

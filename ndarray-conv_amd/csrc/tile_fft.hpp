@@ -354,16 +354,21 @@ struct TileFft {
     }
     // Unnormalised inverse: v holds the last pass's points, and pass 0's on
     // return.  The last pass's points are written where they were read, so no
-    // barrier precedes the first write.
-    template <int P = S::NP - 1>
-    static __device__ __forceinline__ void inverse(C* v, C* lds, const Tw& tw, int t) {
+    // barrier precedes the first write.  before_first(v) sees pass 0's points
+    // ahead of its transforms: point 0 of each thread is the group of bin 0.
+    struct None {
+        __device__ __forceinline__ void operator()(C*) const {}
+    };
+    template <int P = S::NP - 1, class First = None>
+    static __device__ __forceinline__ void inverse(C* v, C* lds, const Tw& tw, int t, First before_first = First{}) {
+        if constexpr (P == 0) before_first(v);
         bfly_pass<P>(v, true);
         if constexpr (P > 0) {
             lds_write<P>(v, lds, thr_slot<P>(t));
             __syncthreads();
             lds_read<P - 1>(v, lds, thr_slot<P - 1>(t));
             twiddle<P - 1>(v, tw, true);
-            inverse<P - 1>(v, lds, tw, t);
+            inverse<P - 1>(v, lds, tw, t, before_first);
         }
     }
 };

@@ -19,7 +19,7 @@ namespace {
 using tilefft::Shape;
 
 template <int LH, int LW, int LP>
-std::vector<double> twiddles_of() {
+std::vector<double> make_twiddles() {
     using S = Shape<LH, LW, LP>;
     static constexpr tilefft::Map<S, 5> m5{};
     static constexpr tilefft::Map<S, 4> m4{};
@@ -30,15 +30,23 @@ std::vector<double> twiddles_of() {
         const int P = 1 << digit, M = 1 << low;
         for (int k = 1; k < P; ++k)
             for (int m = 0; m < M; ++m) {
-                const double ang = -2.0 * M_PI * double(k) * double(m) / (double(P) * double(M));
-                t[size_t(2) * (off + (k - 1) * M + m)] = std::cos(ang);
-                t[size_t(2) * (off + (k - 1) * M + m) + 1] = std::sin(ang);
+                // an angle in 64 bits would be off by several ulp of its cosine
+                const long double ang = -2.0L * 3.14159265358979323846264338327950288L * (k * m) / (P * M);
+                t[size_t(2) * (off + (k - 1) * M + m)] = double(std::cos(ang));
+                t[size_t(2) * (off + (k - 1) * M + m) + 1] = double(std::sin(ang));
             }
     };
     for (int p = 0; p < S::NP; ++p) {
         if (m5.wlow[p] > 0 && S::aw[p] > 0) fill(m5.tww[p], S::aw[p], m5.wlow[p]);
         if (m5.hlow[p] > 0 && S::ah[p] > 0) fill(m5.twh[p], S::ah[p], m5.hlow[p]);
     }
+    return t;
+}
+
+// Made once: a plan of new shapes needs the table again (0.1 to 2 ms).
+template <int LH, int LW, int LP>
+const std::vector<double>& twiddles_of() {
+    static const std::vector<double> t = make_twiddles<LH, LW, LP>();
     return t;
 }
 
@@ -188,7 +196,8 @@ bool tile_spans_fit(const Plan& p) {
     return true;
 }
 
-std::vector<double> tile_twiddles(int lh, int lw, int lp) {
+const std::vector<double>& tile_twiddles(int lh, int lw, int lp) {
+    static const std::vector<double> none;
     switch ((lh * 16 + lw) * 8 + lp) {
         case (0 * 16 + 10) * 8 + 2: return twiddles_of<0, 10, 2>();
         case (0 * 16 + 12) * 8 + 3: return twiddles_of<0, 12, 3>();
@@ -200,7 +209,7 @@ std::vector<double> tile_twiddles(int lh, int lw, int lp) {
         case (5 * 16 + 7) * 8 + 4: return twiddles_of<5, 7, 4>();
         case (6 * 16 + 7) * 8 + 4: return twiddles_of<6, 7, 4>();
         case (7 * 16 + 7) * 8 + 4: return twiddles_of<7, 7, 4>();
-        default: return {};
+        default: return none;
     }
 }
 
@@ -248,7 +257,7 @@ bool tile_plan(const Plan& p, size_t lds, int cus, TilePlan* t) {
         if (!(N > 2 ? (dbl ? c.sum64 : c.sum32) : (dbl ? c.f64 : c.f32))) continue;
         if (one && c.lw > 12) continue;
         const int64_t pts = int64_t(1) << (c.lh + c.lw);
-        if (size_t(pts * cs) > lds) continue;
+        if (size_t(pts * cs) + (N == 1 && dbl ? 32 : 0) > lds) continue;   // and two slots (mean_apart)
         int64_t vw, vh = 1;
         const int64_t nw = tiles(w, c.lw, &vw);
         const int64_t nh = N == 1 ? 1 : tiles(h, c.lh, &vh);
@@ -353,8 +362,9 @@ ndc_status launch_tile(const Plan& p, const TilePlan& t, const void* x, const vo
         return dbl ? launch_tile_as<double>(t, a, cplx, 2, ctx) : launch_tile_as<float>(t, a, cplx, 2, ctx);
     if (!t.tw || !t.flag) {
         const std::string key = "tile:" + std::to_string(t.lh) + ":" + std::to_string(t.lw) + ":" + std::to_string(t.lp) + (dbl ? ":d" : ":f");
-        const std::vector<double> tab = tile_twiddles(t.lh, t.lw, t.lp);
-        const std::vector<float> f(tab.begin(), tab.end());
+        const std::vector<double>& tab = tile_twiddles(t.lh, t.lw, t.lp);
+        std::vector<float> f;
+        if (!dbl) f.assign(tab.begin(), tab.end());
         t.tw = dbl ? ctx.constant_table(key, tab.data(), tab.size() * sizeof(double))
                    : ctx.constant_table(key, f.data(), f.size() * sizeof(float));
         const uint32_t zeros[2] = {0, 0};
