@@ -477,6 +477,38 @@ int kind_of(const Plan& p, bool exact) {
     }
 }
 
+// Whether the matrix form is the faster one, by the part of its tiles that is
+// output.  A workgroup stages and multiplies 256 columns whatever the output
+// has; the vector kernel's tiles are 64 wide, and it reads and writes a dilated
+// axis in one piece, where the phases here touch every line d times over.  So a
+// tile must be filled the more, the fewer taps (products, which the matrix cores do
+// faster) an output has.  Where every workgroup has a CU of its own, its latency
+// is all that counts.
+//
+// The lines are fitted to both forms on 2228 problems a type: images 24 to 2048
+// wide of 60 K to 16 M elements, 1x1 to 31x31 taps, strides and dilations 1 to 3.
+// Time lost against the better form: FP32 2.9%, i32 1.7%, i16 1.4%, i8 1.8% (with
+// the matrix form throughout 48, 153, 54 and 27%, in single cases 8, 28, 9 and 5
+// times).  16 M elements, us, matrix and vector: i32 62500x256, 9x1 taps, dilation 3:
+// 323, 56; FP32 the same, 1x1: 84, 37; i32 250000x64, 3x3: 246, 111; 7812x2048: 68, 117.
+bool matrix_pays(int kind, double fill, int64_t phases, double taps, int64_t blocks, int64_t cus) {
+    struct Line { double phased, plain, plain_taps; int64_t few; double few_taps; };
+    static constexpr Line f32 = {30, 0.15, 1e9, 1, 9}, i32 = {40, 0.7, 60, 1, 9}, i16 = {12, 0.25, 10, 2, 1},
+                          i8 = {4, 0.15, 5, 2, 1};
+    const Line& l = kind == kF32 ? f32 : kind == kI32 ? i32 : kind == kI16 ? i16 : i8;
+    if (blocks <= l.few * cus && taps >= l.few_taps) return true;
+    return fill >= (phases > 1 ? l.phased / taps : std::min(l.plain, l.plain_taps / taps));
+}
+
+// The same for BF16x3 against the systolic kernel of mfma_conv.hip, whose tiles are
+// narrower too: that one serves tall kernels on narrow outputs (31x31 taps, dilation
+// 2, 62500x64: 137 us against 286 here; 15x15, dilation 3, 125000x128: 171 against 315).
+// 58 of 1876 such problems were slower here; single BF16 never was.
+bool split_pays(double fill, int64_t phases, int64_t kh, int64_t kw, int64_t blocks, int64_t cus) {
+    if (std::min(kh, kw) < 12 || fill >= 0.2) return true;
+    return kh * kw >= 900 ? blocks <= 3 * cus : phases == 1 || blocks <= 6 * cus;
+}
+
 }  // namespace
 
 bool launch_matrix(const Plan& p, bool exact, const void* x, const void* k, void* y, LaunchContext& ctx,
@@ -530,6 +562,9 @@ bool launch_matrix(const Plan& p, bool exact, const void* x, const void* k, void
         if (blocks * 10 >= int64_t(ctx.cu_count()) * 9) break;
     }
     if (!rows || blocks >= (int64_t(1) << 30)) return false;
+    const double fill = double(p.out[0]) * double(p.out[1]) / (double(blocks) * rows * kTileX);
+    if (exact && !matrix_pays(kind, fill, phases[1], double(KH) * double(KW), blocks, ctx.cu_count())) return false;
+    if (kind == kBf16x3 && !split_pays(fill, phases[1], KH, KW, blocks, ctx.cu_count())) return false;
     a.ax[1].V = kTileX;
     a.ax[1].tiles = tile_div((pex + kTileX - 1) / kTileX);
     a.x = static_cast<const char*>(x) + p.x_lo * es;

@@ -1,7 +1,7 @@
 // Plans direct convolutions on the host: every launch of ndc::launch_direct is
 // recorded instead of made (LaunchContext::dry_run).  Arguments: dtype, then
 // "n k dilation stride" for each axis.  Prints the status, and the dynamic LDS
-// bytes, grid and block of each launch.
+// bytes, grid, block and form of each launch.
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -22,8 +22,8 @@ struct Dry final : LaunchContext {
     int cu_count() override { return 256; }
     size_t max_lds() override { return 160 * 1024 - kStaticLdsReserve; }
     bool dry_run() override { return true; }
-    void record_launch(const char*, size_t smem, unsigned grid, unsigned block) override {
-        std::printf("launch %zu %u %u\n", smem, grid, block);
+    void record_launch(const char* kernel, size_t smem, unsigned grid, unsigned block) override {
+        std::printf("launch %zu %u %u %s\n", smem, grid, block, std::strstr(kernel, "matrix_conv") ? "matrix" : "vector");
         ++launches;
     }
 };

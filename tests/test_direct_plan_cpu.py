@@ -15,10 +15,11 @@ def exe():
 
 
 def launches(exe, dtype, *axes):
-    """(LDS bytes, grid, block) of each launch; axes are (n, k, dilation, stride)."""
+    """(LDS bytes, grid, block, form) of each launch; axes are (n, k, dilation, stride)."""
     r = subprocess.run([exe, str(dtype)] + [str(v) for a in axes for v in a], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, (r.returncode, r.stdout, r.stderr)
-    return [tuple(int(v) for v in line.split()[1:]) for line in r.stdout.splitlines() if line.startswith("launch")]
+    rows = [line.split()[1:] for line in r.stdout.splitlines() if line.startswith("launch")]
+    return [tuple(int(v) for v in row[:3]) + (row[3],) for row in rows]
 
 
 @pytest.mark.parametrize("dtype", [F32, F64, I32])
@@ -36,5 +37,16 @@ def test_any_dilation_is_planned(exe, dtype, axes):
                                         (F64, [(1026, 3, 1, 1), (20480, 3, 1, 10)]), (C128, [(700, 3, 1, 1), (700, 1, 1, 10)])])
 def test_strides_up_to_the_lds_limit(exe, dtype, axes):
     """Regions that fill LDS but for a few hundred bytes leave no room for the offset tables."""
-    (smem, _, _), = launches(exe, dtype, *axes)
+    (smem, _, _, _), = launches(exe, dtype, *axes)
     assert 155 * 1024 < smem <= 159 * 1024
+
+
+@pytest.mark.parametrize("dtype", [F32, I32])
+@pytest.mark.parametrize("shape,taps,dil,matrix", [
+    ((62500, 256), (9, 1), 3, False), ((250000, 64), (3, 3), 3, False), ((666666, 24), (1, 7), 3, False),   # d phases, few taps
+    ((333333, 12), (3, 3), 1, False),                                                                         # a narrow tile
+    ((4000, 4000), (3, 3), 1, True), ((4000, 4000), (31, 31), 1, True), ((4000, 4000), (31, 31), 3, True),
+    ((300, 300), (5, 5), 1, True), ((60, 300), (9, 9), 2, True)])                                            # few workgroups
+def test_matrix_form_where_its_tiles_are_filled(exe, dtype, shape, taps, dil, matrix):
+    (_, _, _, form), = launches(exe, dtype, *[(n, k, dil, 1) for n, k in zip(shape, taps)])
+    assert form == ("matrix" if matrix else "vector")
