@@ -600,16 +600,32 @@ __device__ __forceinline__ bool cell_read(const TileOuter& o, int c) {
     return false;
 }
 
+// How a wave goes over a plane of x: parts of eight steps of 64 cells, cw columns (a
+// power of two) of 64 / cw rows to a step, `steps` steps side by side.
+struct ScanParts {
+    int planes;              // planes to look at
+    int cw, steps;
+    TileDiv across;          // parts along a row
+    int parts;               // of a plane
+    int nspec;               // values of kept spectra
+};
+
 // Raises the flag for non-finite values that no tile transforms: in planes of
-// x that no outer tap reads (`planes` of them to look at, `groups` parts of
-// rows each, a part per wave at a time) and in `nspec` values of kept spectra.
+// x that no outer tap reads, and in kept spectra.  Bound by memory, a read of
+// those planes: a call on 17x1612x287 f64 at outer stride 3 (42 MB of unread planes)
+// takes 25 us without and 41 with it, small ones 4 to 5 more (in whole-array passes, which
+// transform every plane, 639 and 35 to 50).
 template <typename R, bool CPLX>
-__global__ void __launch_bounds__(256) tile_scan_kernel(TileArgs a, int planes, int groups, int nspec) {
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(int(blockIdx.x * 4 + (threadIdx.x >> 6)));
+__global__ void __launch_bounds__(256) tile_scan_kernel(TileArgs a, ScanParts p) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+    // the waves of a workgroup share a plane, or take one each where it is small
+    const bool share = p.parts >= 4;
+    const int q0 = share ? int(blockIdx.x) : int(blockIdx.x) * 4 + wave, dq = int(gridDim.x) * (share ? 1 : 4);
+    const int i0 = share ? int(blockIdx.y) * 4 + wave : int(blockIdx.y), di = int(gridDim.y) * (share ? 4 : 1);
+    const int lr = lane / p.cw, lc = lane & (p.cw - 1), rs = 64 / p.cw;
     bool bad = false;
-    for (int64_t i = wave; i < int64_t(planes) * groups; i += int64_t(gridDim.x) * 4) {
-        int plane = int(i / groups), xo = 0;
-        const int g = int(i - int64_t(plane) * groups);
+    for (int q = q0; q < p.planes; q += dq) {
+        int plane = q, xo = 0;
         bool read = true;
         for (int e = a.nouter - 1; e >= 0; --e) {
             int cell;
@@ -619,19 +635,25 @@ __global__ void __launch_bounds__(256) tile_scan_kernel(TileArgs a, int planes, 
         }
         if (read) continue;
         const __amdgpu_buffer_rsrc_t px = buffer_of(static_cast<const char*>(a.x) + xo, a.x_bytes - xo);
-        for (int r = g; r < a.ax[0].n; r += groups)
-            for (int c = lane; c < a.ax[1].n; c += 64) {
+        for (int i = i0; i < p.parts; i += di) {
+            int pw;
+            const int r0 = div_by(p.across, i, &pw) * (8 / p.steps) * rs + lr, c0 = pw * p.steps * 64 + lc;
+            Cx<R> v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const int r = r0 + u / p.steps * rs, c = c0 + (u & (p.steps - 1)) * 64;
                 const uint32_t off = uint32_t(r) * uint32_t(a.ax[0].xs) + uint32_t(a.ax[0].xlo) +
                                      uint32_t(c) * uint32_t(a.ax[1].xs) + uint32_t(a.ax[1].xlo);
-                if constexpr (CPLX) {
-                    const Cx<R> v = load_cx(px, off, R(0));
-                    bad |= nonfinite(v.x) || nonfinite(v.y);
-                } else {
-                    bad |= nonfinite(load_real<R>(px, off));
-                }
+                const uint32_t at = r < a.ax[0].n && c < a.ax[1].n ? off : kNoCell;
+                if constexpr (CPLX) v[u] = load_cx(px, at, R(0));
+                else v[u] = cmake<Cx<R>>(load_real<R>(px, at), R(0));
             }
+#pragma unroll
+            for (int u = 0; u < 8; ++u) bad |= nonfinite(v[u].x) || nonfinite(v[u].y);
+        }
     }
-    for (int i = int(blockIdx.x) * 256 + int(threadIdx.x); i < nspec; i += int(gridDim.x) * 256)
+    const int block = int(blockIdx.y * gridDim.x + blockIdx.x), blocks = int(gridDim.x * gridDim.y);
+    for (int i = block * 256 + int(threadIdx.x); i < p.nspec; i += blocks * 256)
         bad |= nonfinite(static_cast<const R*>(a.spec)[i]);
     if (bad) a.flag[0] = 1;
 }
@@ -736,15 +758,25 @@ ndc_status launch_any(const TilePlan& p, const TileArgs& a, int what, LaunchCont
 // plane is transformed), kept spectra of taps that no tile uses.
 template <typename R, bool CPLX>
 ndc_status launch_scan(const TilePlan& p, const TileArgs& a, LaunchContext& ctx) {
-    const int planes = p.gaps && !a.xspec ? p.xplanes : 0;
-    const int nspec = p.idle && a.have_spec ? int(p.spec_bytes / sizeof(R)) : 0;
-    if (!planes && !nspec) return NDC_OK;
-    // parts of at least a row, and 64 of them for each of 256 CUs where rows allow it
-    const int groups = std::max(1, std::min(int(a.ax[0].n), 16384 / std::max(1, planes)));
-    const int64_t waves = std::max<int64_t>(int64_t(planes) * groups, (nspec + 63) / 64);
+    ScanParts s;
+    s.planes = p.gaps && !a.xspec ? p.xplanes : 0;
+    s.nspec = p.idle && a.have_spec ? int(p.spec_bytes / sizeof(R)) : 0;
+    if (!s.planes && !s.nspec) return NDC_OK;
+    const int h = a.ax[0].n, w = a.ax[1].n;
+    s.cw = 64;
+    while (s.cw / 2 >= w) s.cw /= 2;
+    s.steps = 1;
+    while (s.steps < 8 && s.steps * 64 < w) s.steps *= 2;
+    const int rows = 8 / s.steps * (64 / s.cw), cols = s.steps * 64, across = (w + cols - 1) / cols;
+    s.across = tile_div(across);
+    s.parts = across * ((h + rows - 1) / rows);
+    // about 32 workgroups for each of 256 CUs, of which those on planes that are read leave at once
+    const bool share = s.parts >= 4;
+    const unsigned gx = unsigned(std::max(1, std::min(share ? s.planes : (s.planes + 3) / 4, 16384)));
+    const int ny = !s.planes ? std::min(256, (s.nspec + 255) / 256)
+                   : std::min(share ? (s.parts + 3) / 4 : s.parts, std::max(1, 8192 / int(gx)));
     ctx.kbegin("tile_scan", 0, 0);
-    NDC_LAUNCH(ctx, ctx.stream(), (tile_scan_kernel<R, CPLX>), dim3(unsigned(std::min<int64_t>((waves + 3) / 4, 4096))),
-               dim3(256), 0, a, planes, groups, nspec);
+    NDC_LAUNCH(ctx, ctx.stream(), (tile_scan_kernel<R, CPLX>), dim3(gx, unsigned(ny)), dim3(256), 0, a, s);
     ctx.kend();
     return NDC_OK;
 }
