@@ -424,7 +424,7 @@ def run_batch(args):
                for nm, v in prof.items()}
     report = bp.report()
 
-    # the FP32-only autotuned form (direct and FFT items only) on the same batch
+    # the FP32-only autotuned form (direct items and tile runs) on the same batch
     ys, names = [y_head], [args.batch_algo]
     fp32 = None
     if args.batch_algo != "auto":

@@ -15,8 +15,8 @@
 // dilation 2) takes 457 us on 64x128 tiles, 1.1 ns per complex point and CU
 // where the transforms' own arithmetic takes 0.6; its 1.07 GB would take 200 us.
 // The multi-pass transforms of the same call took 9.1 ms (seven passes over
-// 1.2-2.7 GB of spectra), of a 200x5000 one 38 us against 18 here, of a
-// 10x100x200 complex one 65 against 29.
+// 1.2-2.7 GB of spectra), of a 200x5000 one 38 us against 17 here, of a
+// 10x100x200 complex one 65 against 26.
 //
 // Non-finite data: the whole-array transform makes every output NaN.  Within
 // a tile the FFT spreads a non-finite value to every point, so one point per

@@ -73,7 +73,7 @@ constexpr Cand kCands[] = {
 // marker of a cell that is not read (tile_kernels.hpp kNoCell) lies past it.
 constexpr int64_t kSpanMax = int64_t(1) << 30;
 // Inputs up to this size are looked over by every workgroup of a one-launch
-// plan (64 loads per thread at most).
+// plan (64 loads per thread at most, 128 of complex elements).
 constexpr int64_t kScanMax = 16384;
 constexpr int64_t kMaxTaps = 16;
 // Kept spectra of x's tiles, as long as they stay in cache: at 6.5 MB
