@@ -274,9 +274,7 @@ bool tile_plan(const Plan& p, size_t lds, int cus, TilePlan* t) {
         const double per = c.point * (dbl ? 1.8 : 1.0) * double(pts) / cus;
         const double xspec = double(xplanes) * double(pi) * double(pts * cs);
         const bool keep = N > 2 && !fills && xspec <= double(kKeptMax) && double(xplanes) < double(planes) * double(taps);
-        // summing planes of constant fill takes 1.8 times as long (a case analysis
-        // per point and tap): 30x49x15 f64, 16x20x1 taps: 66 us against 38 in passes
-        const double trips = N > 2 ? 0.425 * (1.0 + double(taps)) * (fills ? 1.8 : 1.0) : 1.0;
+        const double trips = N > 2 ? 0.425 * (1.0 + double(taps)) : 1.0;
         const double cost = keep ? 1.1 * c.lat + 0.5 * per * double(pi) * double(xplanes + planes) +
                                        double(items) * double(taps) * double(pts * cs) / 2000.0 + 3000.0
                                  : (c.lat + per * double(items)) * trips +
