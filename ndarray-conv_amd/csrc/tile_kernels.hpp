@@ -334,9 +334,9 @@ __device__ __forceinline__ bool nonfinite(double v) {
     return (uint32_t(__builtin_bit_cast(uint64_t, v) >> 32) & 0x7ff00000u) == 0x7ff00000u;
 }
 
-// Kernel spectra: one workgroup per outer tap.  A kept spectrum raises no flag:
-// the calls that use it do.
-template <typename R, class S, bool CPLX>
+// Kernel spectra: one workgroup per outer tap.  CHECK raises the flag for taps that
+// no tile may use (outer axes); a kept spectrum raises none, the calls that use it do.
+template <typename R, class S, bool CPLX, bool CHECK>
 __global__ void __launch_bounds__(S::T) tile_spec_kernel(TileArgs a) {
     using C = Cx<R>;
     extern __shared__ unsigned char smem_raw[];
@@ -346,10 +346,11 @@ __global__ void __launch_bounds__(S::T) tile_spec_kernel(TileArgs a) {
     const auto tw = TileFft<R, S>::load_tw(a.tw, t);
     TileIo<R, S, CPLX, false>::load_kernel(v, a, outer_cell(a, 0, int(blockIdx.x)).ko, t);
     TileFft<R, S>::forward(v, lds, tw, t);
-    if (!a.have_spec && (nonfinite(v[0].x) || nonfinite(v[0].y))) a.flag[0] = 1;
     C* out = static_cast<C*>(a.spec) + size_t(blockIdx.x) * S::N + t;
 #pragma unroll
     for (int r = 0; r < S::PPT; ++r) out[r * S::T] = v[r];
+    if constexpr (CHECK)
+        if (nonfinite(v[0].x) || nonfinite(v[0].y)) a.flag[0] = 1;
 }
 
 // Tiles whose zero-frequency product passes the inverse transform by, in two
@@ -463,6 +464,8 @@ __global__ void __launch_bounds__(S::T) tile_fwd_kernel(TileArgs a) {
     extern __shared__ unsigned char smem_raw[];
     C* lds = reinterpret_cast<C*>(smem_raw);
     const int t = threadIdx.x, nk = a.have_spec ? 0 : a.ntaps;
+    uint32_t* flag = a.flag;   // loaded ahead of its use
+    asm volatile("" : "+s"(flag));
     const auto tw = F::load_tw(a.tw, t);
     C v[S::PPT];
     C* out;
@@ -483,9 +486,9 @@ __global__ void __launch_bounds__(S::T) tile_fwd_kernel(TileArgs a) {
         out = static_cast<C*>(a.xspec) + size_t(item) * S::N + t;
     }
     F::forward(v, lds, tw, t);
-    if (nonfinite(v[0].x) || nonfinite(v[0].y)) a.flag[0] = 1;
 #pragma unroll
     for (int r = 0; r < S::PPT; ++r) out[r * S::T] = v[r];
+    if (nonfinite(v[0].x) || nonfinite(v[0].y)) flag[0] = 1;
 }
 
 // tile_sum_kernel from kept spectra of x: a tile of x is transformed once and
@@ -725,10 +728,15 @@ ndc_status launch_shape(const TilePlan& p, const TileArgs& a, int what, LaunchCo
         return NDC_ERR_UNSUPPORTED;
     }
     ctx.kbegin("tile_spec", double(a.k_bytes) + double(p.spec_bytes), 5.0 * S::N * S::LN * a.ntaps);
-    if (!lds_fits(ctx, reinterpret_cast<const void*>(&tile_spec_kernel<R, S, CPLX>), smem)) return NDC_ERR_UNSUPPORTED;
-    NDC_LAUNCH(ctx, ctx.stream(), (tile_spec_kernel<R, S, CPLX>), dim3(unsigned(a.ntaps)), dim3(S::T), smem, a);
-    ctx.kend();
-    return NDC_OK;
+    auto go = [&](auto kernel) -> ndc_status {
+        if (!lds_fits(ctx, reinterpret_cast<const void*>(kernel), smem)) return NDC_ERR_UNSUPPORTED;
+        NDC_LAUNCH(ctx, ctx.stream(), kernel, dim3(unsigned(a.ntaps)), dim3(S::T), smem, a);
+        ctx.kend();
+        return NDC_OK;
+    };
+    if constexpr (S::LH != 0 && S::LP < 4)
+        if (a.nouter && !a.have_spec) return go(&tile_spec_kernel<R, S, CPLX, true>);
+    return go(&tile_spec_kernel<R, S, CPLX, false>);
 }
 
 template <typename R, bool CPLX>
